@@ -223,16 +223,19 @@ typedef struct tm_match_config {
 	uint32_t schedule;       /* TM_SCHED_*                                  */
 	uint32_t batch_size;     /* PLAIN: queries per (partition, batch) launch,
 	                            0 = 256 (reference parameters.hh:22);
-	                            PERSISTENT: queries per work item (64, 128
-	                            or 256), 0 = 64                              */
+	                            PERSISTENT: 64, 128 or 256, 0 = 64; queries
+	                            per work item of the steps that log or order
+	                            work items or stop at full key sets without
+	                            a rich-filter pass (the matrix kernel of the
+	                            others sizes its own)                        */
 	uint32_t chunk_blocks;   /* PLAIN: least blocks per segment of a unit
 	                            (0 = 64); PERSISTENT: blocks per segment of
-	                            the table (0 = automatic: at most 1024, and
-	                            smaller for submissions too small to fill
-	                            the GPU)                                     */
+	                            the table (0 = automatic, by the step's
+	                            size)                                        */
 	uint32_t waves_per_group;/* waves per workgroup (4, 8 or 16); 0 = by
 	                            step size for PERSISTENT (16 up to 16 query
-	                            tiles, 8 up to 256, else 4), 8 for PLAIN     */
+	                            tiles, 8 up to 256, else 4; 8 in the matrix
+	                            kernel), 8 for PLAIN                         */
 	uint32_t groups_per_cu;  /* PERSISTENT: resident workgroups per CU; 0 = auto */
 	uint64_t hit_capacity;   /* HITS / KEYS_ALL: hit slots; 0 = default      */
 	uint32_t use_graph;      /* PERSISTENT: replay steady-state steps from a
@@ -240,24 +243,15 @@ typedef struct tm_match_config {
 	uint32_t log_units;      /* record per-work-item hit counts and cycles   */
 	uint32_t order_by_cost;  /* PERSISTENT: visit partitions in the order set
 	                            by tm_ring_set_order                          */
-	uint32_t variant;        /* PERSISTENT inner loop, 1..7, 10 or 18, as
-	                            bits; bit 0: candidate query words from
-	                            scalar loads (else LDS broadcasts); bit 1:
-	                            KEYS_UNIQUE hits go through a per-wave key
-	                            log drained 64 lanes at a time; bit 2: early
-	                            exit after words 0-1; bit 3: the next
-	                            block's data is loaded while one is tested;
-	                            bit 4: blocks in rounds of 4, whose loads
-	                            overlap; 0 or other values: default (2)      */
+	uint32_t variant;        /* accepted and ignored (there is one inner loop)  */
 	uint32_t full_exit;      /* PERSISTENT KEYS_UNIQUE: stop testing a query
 	                            once its key set holds every key of the
 	                            table (results unchanged); 0 = default (on),
 	                            1 = on, 2 = off                              */
-	uint32_t compact_tiles;  /* PERSISTENT KEYS_UNIQUE / KEY_BITMAP: steps of
-	                            more query tiles than this match only the
-	                            queries the rich-filter pass leaves
-	                            incomplete, packed into tiles of their own;
-	                            0 = default (128)                            */
+	uint32_t compact_tiles;  /* accepted and ignored: every KEYS_UNIQUE /
+	                            KEY_BITMAP step with a rich-filter pass
+	                            matches only the queries that pass leaves
+	                            incomplete                                   */
 	uint32_t reserved[4];
 } tm_match_config;
 

@@ -19,6 +19,7 @@
 #include <cstring>
 #include <numeric>
 #include <thread>
+#include <unordered_map>
 
 using namespace tmx;
 
@@ -31,8 +32,6 @@ void tm_fib::release() {
 	dfree(key_dict);
 	dfree(part_info);
 	dfree(part_stat);
-	dfree(sup_info);
-	sup_groups = 0;
 	dfree(slot_epoch);
 	dfree(d_rich_words);
 	dfree(d_rich_bm);
@@ -122,7 +121,8 @@ int build_blocks(const uint32_t * words, const uint32_t * part_offsets, const ui
 				 const uint32_t * key_offsets, const uint32_t * keys, const uint32_t * filter_ids, uint64_t fid_base,
 				 const std::vector<int> & order, const std::vector<uint32_t> & dict, bool inline_ok,
 				 std::vector<uint32_t> & ovf, uint32_t p_base, uint32_t b_base, uint32_t reserve_pct,
-				 block_build & bb, uint32_t last_cap = 0) {
+				 block_build & bb, uint32_t last_cap = 0,
+				 const std::unordered_map<uint32_t, uint32_t> * rich_of = nullptr) {
 	const uint32_t n = part_offsets[n_parts];
 	std::vector<uint32_t> pblock(n_parts + 1, 0);
 	for (uint32_t p = 0; p < n_parts; ++p) {
@@ -205,8 +205,12 @@ int build_blocks(const uint32_t * words, const uint32_t * part_offsets, const ui
 			info[6] = lane + 1;
 			ps[6] += 1;
 			bb.fid[(size_t)blk * 64 + lane] = filter_ids ? filter_ids[i] : (uint32_t)(fid_base + i);
-			TM_CHECK(key_slot(keys, key_offsets[i], key_offsets[i + 1], dict, inline_ok, ovf,
-							  bb.keys[(size_t)blk * 64 + lane]));
+			uint64_t & slot = bb.keys[(size_t)blk * 64 + lane];
+			TM_CHECK(key_slot(keys, key_offsets[i], key_offsets[i + 1], dict, inline_ok, ovf, slot));
+			if (rich_of && key_offsets[i + 1] - key_offsets[i] >= RICH_MIN_KEYS) {
+				const auto it = rich_of->find(i);
+				if (it != rich_of->end()) slot |= (uint64_t)it->second << 48;
+			}
 		}
 	}
 	return TM_OK;
@@ -258,7 +262,7 @@ struct ins_rec {
 // AND mask and valid-lane count.
 __global__ void __launch_bounds__(256)
 k_insert_lanes(const ins_rec * __restrict__ recs, uint32_t n, uint32_t n_blocks, uint32_t * __restrict__ blk_words,
-			   uint32_t * __restrict__ blk_info, uint32_t * __restrict__ sup_info, uint64_t * __restrict__ slot_keys,
+			   uint32_t * __restrict__ blk_info, uint64_t * __restrict__ slot_keys,
 			   uint32_t * __restrict__ slot_fid, uint32_t * __restrict__ slot_epoch, uint32_t epoch) {
 	const uint32_t i = blockIdx.x * 256 + threadIdx.x;
 	if (i >= n) return;
@@ -272,26 +276,10 @@ k_insert_lanes(const ins_rec * __restrict__ recs, uint32_t n, uint32_t n_blocks,
 	for (int j = 0; j < 6; ++j) {
 		blk_words[(size_t)r.block * BLOCK_WORDS + j * 64 + r.lane] = r.w[j];
 		atomicAnd(&blk_info[(size_t)r.block * 8 + j], r.w[j]);
-		if (sup_info) atomicAnd(&sup_info[(size_t)(r.block / SUP_BLOCKS) * 8 + j], r.w[j]);
 	}
 	atomicMax(&blk_info[(size_t)r.block * 8 + 6], r.lane + 1);
 	slot_keys[(size_t)r.block * 64 + r.lane] = r.kv;
 	slot_fid[(size_t)r.block * 64 + r.lane] = r.fid;
-}
-
-// Group masks: AND of the masks of blocks [8g, 8g + 8) (words 0-5; empty
-// blocks hold all ones), one thread per group.
-__global__ void __launch_bounds__(256)
-k_sup_masks(const uint32_t * __restrict__ blk_info, uint32_t nb, uint32_t * __restrict__ sup_info) {
-	const uint32_t gi = blockIdx.x * 256 + threadIdx.x;
-	if ((uint64_t)gi * SUP_BLOCKS >= nb) return;
-	uint32_t m[6] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
-	const uint32_t b1 = min(gi * SUP_BLOCKS + SUP_BLOCKS, nb);
-	for (uint32_t b = gi * SUP_BLOCKS; b < b1; ++b)
-		for (int j = 0; j < 6; ++j) m[j] &= blk_info[(size_t)b * 8 + j];
-	for (int j = 0; j < 6; ++j) sup_info[(size_t)gi * 8 + j] = m[j];
-	sup_info[(size_t)gi * 8 + 6] = 0;
-	sup_info[(size_t)gi * 8 + 7] = 0;
 }
 
 // Lane epochs of blocks [b0, nb): lanes already valid get `visible`, the
@@ -319,26 +307,6 @@ k_remap_keys(uint64_t * __restrict__ slot_keys, uint64_t n, const uint32_t * __r
 		o |= (id == KEY_NONE ? (uint64_t)KEY_NONE : (uint64_t)map[id]) << (16 * x);
 	}
 	slot_keys[i] = o;
-}
-
-// Group masks of every block, into a fresh array when the block count
-// outgrew the current one.  `fresh` says whether sup_info moved (rings must
-// then re-read the FIB, as for any other array that moved).
-int refresh_sup(tm_fib * fib, bool & fresh) {
-	const uint64_t ng = ((uint64_t)fib->n_blocks + SUP_BLOCKS - 1) / SUP_BLOCKS;
-	fresh = false;
-	if (!fib->sup_info || ng > fib->sup_groups) {
-		dfree(fib->sup_info);
-		fib->sup_groups = 0;
-		TM_CHECK(dalloc(&fib->sup_info, std::max<uint64_t>(ng, 1) * 8));
-		fib->sup_groups = std::max<uint64_t>(ng, 1);
-		fresh = true;
-	}
-	if (ng) hipLaunchKernelGGL(k_sup_masks, dim3((uint32_t)((ng + 255) / 256)), dim3(256), 0, 0, fib->blk_info,
-							   fib->n_blocks, fib->sup_info);
-	TM_HIP(hipGetLastError());
-	TM_HIP(hipDeviceSynchronize());
-	return TM_OK;
 }
 
 } // namespace
@@ -447,40 +415,11 @@ int tm_fib_upload(tm_fib * fib, const uint32_t * words, uint32_t n,
 	std::iota(order.begin(), order.end(), 0);
 	std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return freq[a] < freq[b]; });
 
-	std::vector<uint32_t> h_ovf(1, 0);   // overflow key lists (count, ids...)
-	block_build bb;
-	// With a reserve, one more partition: empty, mask 0 (every query selects
-	// it), room for about 1% of the table.  Inserted filters that contain no
-	// partition's mask go there instead of needing a new partition, so that
-	// they can be inserted live.
-	const bool catch_all = fib->reserve_pct > 0;
-	std::vector<uint32_t> off2, masks2;
-	const uint32_t * po = part_offsets;
-	const uint32_t * pm = part_masks;
-	uint32_t np = n_parts, last_cap = 0;
-	if (catch_all) {
-		off2.assign(part_offsets, part_offsets + n_parts + 1);
-		off2.push_back(n);
-		masks2.assign(part_masks, part_masks + (size_t)n_parts * 6);
-		masks2.resize(masks2.size() + 6, 0u);
-		po = off2.data();
-		pm = masks2.data();
-		np = n_parts + 1;
-		last_cap = std::max<uint32_t>(16, (n / 64) / 100);
-	}
-	TM_CHECK(build_blocks(words, po, pm, np, key_offsets, keys, filter_ids, 0, order, dict, inline_ok, h_ovf, 0, 0,
-						  fib->reserve_pct, bb, last_cap));
-	uint64_t maxp = 0;
-	std::vector<uint32_t> h_psize(np, 0);
-	for (uint32_t p = 0; p < np; ++p) {
-		h_psize[p] = po[p + 1] - po[p];
-		maxp = std::max<uint64_t>(maxp, h_psize[p]);
-	}
-
 	// rich filters: the MAX_RICH with the most keys (at least RICH_MIN_KEYS),
 	// their words and their key sets as dense bitmaps
 	std::vector<uint32_t> rich_words, rich_bm;
 	uint32_t n_rich_full = 0;
+	std::unordered_map<uint32_t, uint32_t> rich_of;   // filter -> 1 + index
 	{
 		std::vector<std::pair<uint32_t, uint32_t>> cand;   // (keys, filter)
 		for (uint32_t i = 0; i < n; ++i) {
@@ -514,7 +453,38 @@ int tm_fib_upload(tm_fib * fib, const uint32_t * words, uint32_t n,
 				rich_words.insert(rich_words.end(), bw.begin() + r * 8, bw.begin() + r * 8 + 8);
 				rich_bm.insert(rich_bm.end(), bm.begin() + r * kwr, bm.begin() + (r + 1) * kwr);
 				n_rich_full += pass == 0;
+				rich_of[cand[r].second] = (uint32_t)rich_of.size() + 1;
 			}
+	}
+
+	std::vector<uint32_t> h_ovf(1, 0);   // overflow key lists (count, ids...)
+	block_build bb;
+	// With a reserve, one more partition: empty, mask 0 (every query selects
+	// it), room for about 1% of the table.  Inserted filters that contain no
+	// partition's mask go there instead of needing a new partition, so that
+	// they can be inserted live.
+	const bool catch_all = fib->reserve_pct > 0;
+	std::vector<uint32_t> off2, masks2;
+	const uint32_t * po = part_offsets;
+	const uint32_t * pm = part_masks;
+	uint32_t np = n_parts, last_cap = 0;
+	if (catch_all) {
+		off2.assign(part_offsets, part_offsets + n_parts + 1);
+		off2.push_back(n);
+		masks2.assign(part_masks, part_masks + (size_t)n_parts * 6);
+		masks2.resize(masks2.size() + 6, 0u);
+		po = off2.data();
+		pm = masks2.data();
+		np = n_parts + 1;
+		last_cap = std::max<uint32_t>(16, (n / 64) / 100);
+	}
+	TM_CHECK(build_blocks(words, po, pm, np, key_offsets, keys, filter_ids, 0, order, dict, inline_ok, h_ovf, 0, 0,
+						  fib->reserve_pct, bb, last_cap, &rich_of));
+	uint64_t maxp = 0;
+	std::vector<uint32_t> h_psize(np, 0);
+	for (uint32_t p = 0; p < np; ++p) {
+		h_psize[p] = po[p + 1] - po[p];
+		maxp = std::max<uint64_t>(maxp, h_psize[p]);
 	}
 
 	fib->release();
@@ -538,11 +508,6 @@ int tm_fib_upload(tm_fib * fib, const uint32_t * words, uint32_t n,
 	fib->n_rich_full = n_rich_full;
 	fib->n_parts = np;
 	fib->n_blocks = bb.nb;
-	{
-		bool fresh;
-		TM_CHECK(refresh_sup(fib, fresh));
-		bytes += fib->sup_groups * 32;
-	}
 	fib->n_keys = K;
 	fib->n_filters = n;
 	fib->n_key_instances = nkeys;
@@ -700,7 +665,7 @@ int live_commit_locked(tm_fib * fib, live_plan * pl) {
 	if (n) {
 		TM_HIP(hipMemcpyAsync(fib->d_recs, pl->recs.data(), sizeof(ins_rec) * n, hipMemcpyHostToDevice, s));
 		hipLaunchKernelGGL(k_insert_lanes, dim3((n + 255) / 256), dim3(256), 0, s, (const ins_rec *)fib->d_recs, n,
-						   fib->n_blocks, fib->blk_words, fib->blk_info, fib->sup_info, fib->slot_keys, fib->slot_fid, fib->slot_epoch, pl->epoch);
+						   fib->n_blocks, fib->blk_words, fib->blk_info, fib->slot_keys, fib->slot_fid, fib->slot_epoch, pl->epoch);
 		TM_HIP(hipGetLastError());
 	}
 	TM_HIP(hipMemcpyAsync(fib->part_info, pl->part_info.data(), pl->part_info.size() * 4, hipMemcpyHostToDevice, s));
@@ -954,7 +919,7 @@ int tm_fib_insert(tm_fib * fib, const uint32_t * words, uint32_t n, const uint32
 		int rc = put(d_recs, recs);
 		if (rc == TM_OK) {
 			hipLaunchKernelGGL(k_insert_lanes, dim3((uint32_t)((recs.size() + 255) / 256)), dim3(256), 0, 0, d_recs,
-							   (uint32_t)recs.size(), fib->n_blocks, fib->blk_words, fib->blk_info, fib->sup_info, fib->slot_keys, fib->slot_fid,
+							   (uint32_t)recs.size(), fib->n_blocks, fib->blk_words, fib->blk_info, fib->slot_keys, fib->slot_fid,
 							   fib->slot_epoch, e);
 			hipError_t e = hipGetLastError();
 			if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -964,12 +929,6 @@ int tm_fib_insert(tm_fib * fib, const uint32_t * words, uint32_t n, const uint32
 		TM_CHECK(rc);
 		TM_CHECK(put(fib->part_info, fib->h_part_info, (size_t)P * 8));
 		TM_CHECK(put(fib->part_stat, fib->h_part_stat, (size_t)P * 8));
-	}
-	// group masks of the new blocks (and of the blocks the lanes above joined)
-	{
-		bool fresh;
-		TM_CHECK(refresh_sup(fib, fresh));
-		if (fresh) bump = true;
 	}
 	fib->n_filters += n;
 	fib->n_key_instances += nkeys;
@@ -1087,6 +1046,21 @@ int check_image(uint64_t nb, uint64_t P, uint64_t K, const std::vector<uint32_t>
 	return TM_OK;
 }
 
+// A slot's mark of a rich filter (bits 48..63 of an overflow slot) says that
+// the rich-filter pass ORs this slot's keys: marks that do not name a rich
+// filter of the same words are dropped.
+void keep_rich_marks(uint64_t nb, const std::vector<uint32_t> & words, const std::vector<uint32_t> & rich_words,
+					 uint64_t n_rich, std::vector<uint64_t> & skeys) {
+	for (uint64_t i = 0; i < nb * 64; ++i) {
+		const uint64_t kv = skeys[i], r = kv >> 48;
+		if ((kv & 0xFFFF) != KEY_NONE || r == 0 || kv == ~0ULL) continue;
+		bool same = r <= n_rich;
+		for (int j = 0; same && j < 6; ++j)
+			same = rich_words[(r - 1) * 8 + j] == words[(i / 64) * BLOCK_WORDS + (uint64_t)j * 64 + i % 64];
+		if (!same) skeys[i] = kv & 0xFFFFFFFFFFFFULL;
+	}
+}
+
 } // namespace
 
 extern "C" {
@@ -1182,6 +1156,7 @@ int tm_fib_load(tm_fib * fib, const char * path) {
 	TM_CHECK(read_array(f, pcap, P, "partition capacities"));
 	TM_CHECK(read_array(f, order, 192, "bit order"));
 	TM_CHECK(check_image(nb, P, h.n_keys, info, skeys, ovf, dict, pinfo, psize, pcap, order));
+	keep_rich_marks(nb, words, rich_w, h.n_rich, skeys);
 
 	fib->release();
 	uint64_t bytes = 0;
@@ -1204,11 +1179,6 @@ int tm_fib_load(tm_fib * fib, const char * path) {
 	fib->n_rich_full = (uint32_t)h.n_rich_full;
 	fib->n_parts = (uint32_t)P;
 	fib->n_blocks = (uint32_t)nb;
-	{
-		bool fresh;
-		TM_CHECK(refresh_sup(fib, fresh));
-		bytes += fib->sup_groups * 32;
-	}
 	fib->n_keys = (uint32_t)h.n_keys;
 	fib->n_filters = h.n_filters;
 	fib->n_key_instances = h.n_key_instances;

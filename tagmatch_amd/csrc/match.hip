@@ -5,27 +5,33 @@
 // One submission of nq queries runs as a fixed sequence of kernels on the
 // ring's stream, with no host synchronisation in the persistent schedule:
 //
-//   k_lookup_count / scan / k_lookup_fill
-//        query -> partitions with mask & ~q == 0, grouped per partition
-//        (reference front_end.cc:465-477 do_match, on the device);
-//   k_build_items
-//        cut each partition's query list into batches of 64*TILES queries
-//        and its blocks into chunks: one work item per (batch, chunk)
-//        (reference front_end.cc:350-376 batching of 256 queries);
-//   k_match
-//        per work item: for each 64-filter block, a candidate pass with one
-//        query per lane tests the block's AND mask against 64 queries at
-//        once; for each surviving query, one filter per lane tests
-//        f & ~q == 0 (reference gpu.cu:60-607 phases 2 and 3).  Hits are
-//        expanded to dense key ids and OR-ed into per-query key bitmaps
-//        (staged in LDS), or appended as (query, filter) pairs;
+//   k_step_init
+//        zeroes what the step counts in;
+//   k_rich_rows   (KEYS_UNIQUE, KEY_BITMAP)
+//        rows start with the keys of the rich filters each query contains;
+//        the queries whose rows are not complete are listed;
+//   k_lookup_hist
+//        queries per partition (reference front_end.cc:465-477 do_match, on
+//        the device);
+//   k_match_x   (match_matrix.hip)
+//        the listed queries against every block of 64 filters: candidates
+//        from the blocks' AND masks, then the subset tests (reference
+//        gpu.cu:60-607 phases 2 and 3), both on the matrix cores.  Hits OR
+//        their filters' dense key ids into per-query key bitmaps, or their
+//        values are counted and then written behind one another;
 //   k_bm_count / scan / k_bm_write   (KEYS_UNIQUE)
 //        bitmap -> sorted distinct keys (reference tagmatch_query.hh:99-119
 //        sort + unique, and back_end.cc:288-301 key expansion);
-//   k_hits_count / scan / k_hits_write  (HITS, KEYS_ALL)
-//        group hits per query and expand them to ids or keys.
+//   k_gather_stats.
+//
+// The plain schedule (k_lookup_count / scan / k_lookup_fill, k_build_items,
+// then one launch of k_match_q per (partition, batch), and k_hits_count /
+// k_hits_write for hit lists) follows the reference's dispatch shape
+// (front_end.cc:350-376, back_end.cc:243-286).
 #include "cost_model.h"
 #include "fib.h"
+#include "match_dev.h"
+#include "match_matrix.h"
 
 #include <algorithm>
 #include <chrono>
@@ -44,19 +50,13 @@ constexpr int QPAD = 32;         // queue cursors 256 B apart: atomics on one li
 constexpr uint32_t SEG_MAX_BLOCKS = 1024;   // persistent: largest block segment (measured at 10M)
 constexpr uint32_t SEG_MAX_BLOCKS_EXIT = 4096;   // the same with the full-key-set exit: most items
                                                  // skip their blocks, and fewer items cost less
-constexpr uint32_t SEG_MAX_BLOCKS_COMPACT = 1024;   // compacted steps: the tiles of an XCD share a
-                                                   // segment small enough for its L2 (2.8 ms at
-                                                   // 10M filters, 1M queries, against 3.45 with 4096)
 constexpr uint32_t WSEG_BASE = 64;          // block weight: fixed part, in units of one expected hit
 constexpr uint32_t WSEG_MAX_TILES = 256;    // persistent: tiles up to which segments are cut by weight
-constexpr uint64_t COMPACT_MIN_TILES = 128;   // persistent: tiles above which steps are compacted
 constexpr uint32_t PRICE_SAMPLE_TILES = 1024;  // cost model: tiles priced when only totals are needed
 constexpr uint32_t NO_QUERY = 0xFFFFFFFFu;
+constexpr uint64_t ROWS_LDS_MAX_WORK = 80000000;   // queries x blocks of steps whose rows are built in local memory
+constexpr uint64_t HCNT_MAX = 1ull << 26;     // hit-list steps: counts of (segment, query), at most
 constexpr size_t MAX_GRAPHS = 16;             // captured step sizes kept per ring
-
-__device__ inline uint32_t mbcnt64(uint64_t m) {
-	return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
 
 // ------------------------------------------------------------- lookup
 
@@ -163,24 +163,6 @@ k_build_items(const uint32_t * __restrict__ pcount, const uint64_t * __restrict_
 
 // ------------------------------------------------------------- match
 
-// The overflow list a slot points to, bounded by the table's overflow words:
-// whatever a slot holds, nothing outside the table is read (n = 0 then).
-__device__ inline uint32_t ovf_list(uint64_t kv, const uint32_t * __restrict__ ovf, uint32_t ovf_n, uint32_t & off) {
-	off = (uint32_t)(kv >> 16);
-	if (off >= ovf_n) return 0;
-	const uint32_t n = ovf[off];
-	return n < ovf_n - off ? n : 0;
-}
-
-// Number of keys in a slot (inline ids or an overflow list).
-__device__ inline uint32_t key_count(uint64_t kv, const uint32_t * __restrict__ ovf, uint32_t ovf_n) {
-	uint32_t off;
-	if ((kv & 0xFFFFu) == KEY_NONE) return ovf_list(kv, ovf, ovf_n, off);
-	uint32_t n = 0;
-	for (int x = 0; x < 4; ++x) n += ((kv >> (16 * x)) & 0xFFFFu) != KEY_NONE;
-	return n;
-}
-
 // ------------------------------------------------------------- query-major match
 
 // Persistent schedule.  A work item is a group of NQ = 64*TILES consecutive
@@ -204,16 +186,10 @@ __device__ inline uint32_t key_count(uint64_t kv, const uint32_t * __restrict__ 
 struct mq_args {
 	dev_fib_view f;
 	const uint32_t * __restrict__ q;          // nq x 8 words
-	const uint32_t * __restrict__ qinv;       // nq x 8 inverted words (VAR 1)
 	uint32_t nq;
 	const uint32_t * __restrict__ porder;     // partition schedule order (NULL: 0..P-1)
 	const uint32_t * __restrict__ iorder;     // query tile of each work item (NULL: identity; nseg 1 only)
 	const uint32_t * __restrict__ qmap;       // query of each local index (NULL: identity)
-	const uint32_t * __restrict__ units;      // explicit units, 8 words each: partition,
-	                                          // first query, queries, tiles, segments,
-	                                          // blocks per segment, first block, end block
-	const uint32_t * __restrict__ uprefix;    // n_units + 1: first work item of each unit
-	uint32_t n_units;
 	uint32_t blk_lo, blk_hi;                  // blocks the launch covers
 	int32_t log_unit;                         // >= 0: add hits, keys, ticks into this log row
 	uint32_t ntiles;                          // query tiles
@@ -233,16 +209,10 @@ struct mq_args {
 	uint32_t epoch;                           // lanes with a later epoch are not seen
 	uint32_t full_exit;                       // KEYS_UNIQUE + LDS bitmaps: skip queries whose
 	                                          // bitmap holds every key
-	uint32_t groups;                          // walk blocks in groups, skipping a group whose
-	                                          // AND mask no query holds (compacted steps)
 	uint32_t last_mask;                       // valid bits of a bitmap row's last word
 	uint32_t * qfull;                         // nseg > 1 with full_exit: per query, set once its
 	                                          // merged gbm row holds every key
 	const uint32_t * __restrict__ segb;       // nseg + 1 segment bounds (NULL: seg_blocks each)
-	const uint32_t * __restrict__ nq_dev;     // device query count (NULL: nq), with
-	const uint32_t * __restrict__ ntiles_dev; // device tile count, segments, blocks per segment
-	                                          // (NULL: ntiles, nseg, seg_blocks)
-	uint32_t map_rows;                        // KEYS_UNIQUE: local query i is row and flag qmap[i]
 	const uint32_t * __restrict__ step_vals;  // replayed steps: [0] epoch, [1] valid overflow words,
 	                                          // written before each replay (NULL: epoch, f.ovf_n)
 };
@@ -275,21 +245,6 @@ __device__ inline void or_keys(uint32_t * row, uint64_t kv, const uint32_t * __r
 		}
 	}
 }
-
-// Uniform loads through the constant address space compile to scalar
-// loads (s_load) into SGPRs; used for data that no thread writes during the
-// kernel (FIB block info, partition info, inverted query words).
-typedef const __attribute__((address_space(4))) uint32_t cu32_t;
-
-__device__ inline uint4 sld4(const uint32_t * p) {
-	cu32_t * c = (cu32_t *)(p);
-	return make_uint4(c[0], c[1], c[2], c[3]);
-}
-__device__ inline uint2 sld2(const uint32_t * p) {
-	cu32_t * c = (cu32_t *)(p);
-	return make_uint2(c[0], c[1]);
-}
-__device__ inline uint32_t sld1(const uint32_t * p) { return *(cu32_t *)(p); }
 
 // (f0 & q0) | ... | (f5 & q5): one v_and_b32 and five v_and_or_b32 in one
 // asm block.  Left to itself the compiler balances the OR tree into
@@ -426,22 +381,18 @@ struct hit_sink {
 };
 
 // MODE 0: key bitmaps (LDS_BM: in LDS, else in gbm with workgroup-scope
-// atomics); MODE 1: hit pairs.  VAR 0: candidate query words from LDS, two
-// tests per iteration; VAR 1: from pre-inverted query words in HBM through
-// scalar loads, four independent tests per iteration.
-// The default one-tile, 4-wave instance (large and compacted steps) is held
-// to 8 waves per SIMD (64 VGPRs, a few spilled outside the test loop): at
-// 10M filters its compacted launch took 2.25 instead of 2.32 ms and the
-// every-match step 642 instead of 675 ms.  The 8- and 16-wave instances of
-// small steps are left free: held the same way, 1024-query serving steps
-// took 0.19 instead of 0.16 ms.
-template <int MODE, bool LDS_BM, int TILES, int NW, int VAR>
+// atomics); MODE 1: hit pairs.  The plain schedule runs on this kernel, and
+// the persistent steps that the matrix kernel does not take: those that
+// stop testing a query as soon as its row holds every key without a
+// rich-filter pass before (rows are checked before every partition here),
+// and those that log or order work items.
+template <int MODE, bool LDS_BM, int TILES, int NW>
 __global__ void __launch_bounds__(NW * 64)
-__attribute__((amdgpu_waves_per_eu(TILES == 1 && VAR == 2 && NW == 4 ? 8 : 1)))
+__attribute__((amdgpu_waves_per_eu(TILES == 1 && NW == 4 ? 8 : 1)))
 k_match_q(mq_args a) {
 	constexpr int NQ = TILES * 64;
 	constexpr int NT = NW * 64;
-	constexpr bool KLOG = MODE == 0 && (VAR & 2);
+	constexpr bool KLOG = MODE == 0;
 	__shared__ __align__(16) uint32_t s_q[NQ * 8];
 	__shared__ uint32_t s_item[2];
 	__shared__ uint32_t s_hits, s_keys;
@@ -458,16 +409,9 @@ k_match_q(mq_args a) {
 	// item serializes small launches)
 	uint64_t w_hits = 0, w_visit = 0, w_test = 0, w_hev = 0;
 	bool bm_dirty = true;   // LDS bitmap rows hold bits of an earlier item (uniform)
-	// counts written by earlier kernels of the step (compacted submissions)
-	const uint32_t nq_all = a.nq_dev ? sld1(a.nq_dev) : a.nq;
-	const uint32_t ntiles_all = a.ntiles_dev ? sld1(a.ntiles_dev) : a.ntiles;
-	const uint32_t nseg_all = a.ntiles_dev ? sld1(a.ntiles_dev + 1) : a.nseg;
 	// the inserts the step sees: from memory when a captured graph replays it
 	const uint32_t epoch = a.step_vals ? sld1(a.step_vals) : a.epoch;
 	const uint32_t ovf_n = a.step_vals ? sld1(a.step_vals + 1) : a.f.ovf_n;
-	const uint32_t seg_blocks_all = a.ntiles_dev ? sld1(a.ntiles_dev + 2) : a.seg_blocks;
-	// bitmap row (and flag) of local query i
-	auto row_of = [&](uint32_t i) -> uint32_t { return a.map_rows ? a.qmap[i] : i; };
 
 	for (;;) {
 		uint64_t t_start = 0;
@@ -492,35 +436,16 @@ k_match_q(mq_args a) {
 		// one contiguous range of blocks (small submissions spread over the
 		// whole GPU); segment-major, so concurrent items share filter blocks.
 		uint32_t item, seg_b0 = 0, seg_b1 = 0xFFFFFFFFu, r_begin = 0, r_end = P;
-		uint32_t q0, q_end = nq_all;
-		if (a.units) {
-			// explicit (partition, query range) units: the item's unit by
-			// binary search over the item prefix; segment-major in the unit
-			uint32_t lo = 0, hi = a.n_units;
-			while (hi - lo > 1) {
-				const uint32_t mid = (lo + hi) >> 1;
-				if (sld1(a.uprefix + mid) <= item0) lo = mid; else hi = mid;
-			}
-			const uint4 u0 = sld4(a.units + (size_t)lo * 8);       // part, first query, queries, tiles
-			const uint4 u1 = sld4(a.units + (size_t)lo * 8 + 4);   // segments, seg blocks, first, end block
-			const uint32_t local = item0 - sld1(a.uprefix + lo);
-			const uint32_t seg = local / u0.w;
-			item = local - seg * u0.w;
-			q0 = u0.y + item * NQ;
-			q_end = u0.y + u0.z;
-			seg_b0 = u1.z + seg * u1.y;
-			seg_b1 = min(seg_b0 + u1.y, u1.w);
-			r_begin = u0.x;
-			r_end = seg_b1 > seg_b0 ? u0.x + 1 : u0.x;
-		} else if (nseg_all > 1 || a.blk_lo != 0 || a.blk_hi < a.f.n_blocks) {
-			const uint32_t seg = item0 / ntiles_all;
-			item = item0 - seg * ntiles_all;
+		const uint32_t q_end = a.nq;
+		if (a.nseg > 1 || a.blk_lo != 0 || a.blk_hi < a.f.n_blocks) {
+			const uint32_t seg = item0 / a.ntiles;
+			item = item0 - seg * a.ntiles;
 			if (a.segb) {   // segments of equal estimated work
 				seg_b0 = sld1(a.segb + seg);
 				seg_b1 = sld1(a.segb + seg + 1);
 			} else {
-				seg_b0 = a.blk_lo + seg * seg_blocks_all;
-				seg_b1 = min(seg_b0 + seg_blocks_all, a.blk_hi);
+				seg_b0 = a.blk_lo + seg * a.seg_blocks;
+				seg_b1 = min(seg_b0 + a.seg_blocks, a.blk_hi);
 			}
 			if (seg_b1 > seg_b0) {
 				r_begin = sld1(a.f.blk_info + (size_t)seg_b0 * 8 + 7);
@@ -531,7 +456,7 @@ k_match_q(mq_args a) {
 		} else {
 			item = a.iorder ? sld1(a.iorder + item0) : item0;
 		}
-		if (!a.units) q0 = item * NQ;
+		const uint32_t q0 = item * NQ;
 
 		for (uint32_t t = tid; t < (uint32_t)NQ; t += NT) {
 			uint32_t * d = &s_q[t * 8];
@@ -590,7 +515,7 @@ k_match_q(mq_args a) {
 		const bool use_flags = MODE == 0 && LDS_BM && a.full_exit && a.qfull;
 		auto load_flags = [&](int t) -> uint64_t {
 			const uint32_t qrow = q0 + t * 64 + lane;
-			return __ballot(qrow < q_end && __hip_atomic_load(&a.qfull[row_of(qrow)], __ATOMIC_RELAXED,
+			return __ballot(qrow < q_end && __hip_atomic_load(&a.qfull[qrow], __ATOMIC_RELAXED,
 															  __HIP_MEMORY_SCOPE_AGENT) != 0u);
 		};
 #pragma unroll
@@ -615,7 +540,7 @@ k_match_q(mq_args a) {
 			sink.add(h, jl, gq, b, kv, lane);
 		};
 		for (uint32_t r = r_begin; r < r_end; ++r) {
-			const uint32_t p = a.porder && nseg_all <= 1 ? sld1(a.porder + r) : r;
+			const uint32_t p = a.porder && a.nseg <= 1 ? sld1(a.porder + r) : r;
 			const uint32_t * pi = a.f.part_info + (size_t)p * 8;
 			const uint4 pa = sld4(pi);
 			const uint4 pb = sld4(pi + 4);
@@ -653,7 +578,7 @@ k_match_q(mq_args a) {
 					// (k_rich_rows) already filled.
 					if (use_flags && (qsel[t] & ~qfullm[t])) qfullm[t] |= load_flags(t);
 					qsel[t] &= ~qfullm[t];
-					if (nseg_all <= 1 && qsel[t])
+					if (a.nseg <= 1 && qsel[t])
 						qsel[t] &= ~__ballot(row_full(&s_bm[(t * 64 + lane) * kw], kw, lane, a.last_mask));
 					anyq |= qsel[t];
 				}
@@ -670,96 +595,31 @@ k_match_q(mq_args a) {
 				for (int t = 0; t < TILES; ++t) {
 					uint64_t c = cand[t];
 					n_test += (uint32_t)__popcll(c);
-					if ((VAR & 5) == 0) {
-						// candidate query words broadcast from LDS, two per iteration:
-						// the lowest and the highest candidate left (one and the same
-						// for the last of an odd count).  Scalar work per pair kept
-						// small (the scalar unit is as busy as the vector one here):
-						// bits cleared by index, and one branch over both results for
-						// the common pair without hits.
-						while (c) {
-							const uint32_t j0 = (uint32_t)__builtin_ctzll(c);
-							const uint32_t j1 = 63u - (uint32_t)__builtin_clzll(c);
-							c &= ~((1ULL << j0) | (1ULL << j1));
-							const bool has1 = j1 != j0;
-							const uint32_t * qq0 = &s_q[(t * 64 + j0) * 8];
-							const uint32_t * qq1 = &s_q[(t * 64 + j1) * 8];
-							const uint4 a0 = *reinterpret_cast<const uint4 *>(qq0);
-							const uint2 c0 = *reinterpret_cast<const uint2 *>(qq0 + 4);
-							const uint4 a1 = *reinterpret_cast<const uint4 *>(qq1);
-							const uint2 c1 = *reinterpret_cast<const uint2 *>(qq1 + 4);
-							const uint32_t acc0 = test6(f0, f1, f2, f3, f4, f5, a0.x, a0.y, a0.z, a0.w, c0.x, c0.y);
-							const uint32_t acc1 = test6(f0, f1, f2, f3, f4, f5, a1.x, a1.y, a1.z, a1.w, c1.x, c1.y);
-							const uint64_t r0 = __ballot(acc0 == 0), r1 = __ballot(acc1 == 0);
-							if (((r0 | r1) & lmask) == 0) continue;   // (r1 = r0 when j1 = j0)
-							const uint64_t h0 = r0 & lmask;
-							const uint64_t h1 = has1 ? r1 & lmask : 0ULL;
-							if (h0) on_hit(h0, t * 64 + j0, b, kv);
-							if (h1) on_hit(h1, t * 64 + j1, b, kv);
-						}
-					} else if ((VAR & 1) == 0) {
-						// early exit variant: words 0-1 first, two per iteration
-						while (c) {
-							const uint32_t j0 = (uint32_t)__builtin_ctzll(c);
-							c &= c - 1;
-							const uint64_t keep1 = c ? ~0ULL : 0ULL;
-							const uint32_t j1 = c ? (uint32_t)__builtin_ctzll(c) : j0;
-							c &= c - 1;
-							const uint32_t * qq0 = &s_q[(t * 64 + j0) * 8];
-							const uint32_t * qq1 = &s_q[(t * 64 + j1) * 8];
-							uint32_t acc0, acc1;
-							if (VAR & 4) {
-								const uint2 a0 = *reinterpret_cast<const uint2 *>(qq0);
-								const uint2 a1 = *reinterpret_cast<const uint2 *>(qq1);
-								acc0 = (f0 & a0.x) | (f1 & a0.y);
-								acc1 = (f0 & a1.x) | (f1 & a1.y);
-								// early exit: words 0-1 already reject every filter
-								// for both candidates (the common case)
-								const uint64_t alive = (__ballot(acc0 == 0) | (__ballot(acc1 == 0) & keep1)) & lmask;
-								if (alive == 0) continue;
-								const uint2 b0 = *reinterpret_cast<const uint2 *>(qq0 + 2);
-								const uint2 c0 = *reinterpret_cast<const uint2 *>(qq0 + 4);
-								const uint2 b1 = *reinterpret_cast<const uint2 *>(qq1 + 2);
-								const uint2 c1 = *reinterpret_cast<const uint2 *>(qq1 + 4);
-								acc0 |= (f2 & b0.x) | (f3 & b0.y) | (f4 & c0.x) | (f5 & c0.y);
-								acc1 |= (f2 & b1.x) | (f3 & b1.y) | (f4 & c1.x) | (f5 & c1.y);
-							} else {
-								const uint4 a0 = *reinterpret_cast<const uint4 *>(qq0);
-								const uint2 c0 = *reinterpret_cast<const uint2 *>(qq0 + 4);
-								const uint4 a1 = *reinterpret_cast<const uint4 *>(qq1);
-								const uint2 c1 = *reinterpret_cast<const uint2 *>(qq1 + 4);
-								acc0 = (f0 & a0.x) | (f1 & a0.y) | (f2 & a0.z) | (f3 & a0.w) | (f4 & c0.x) | (f5 & c0.y);
-								acc1 = (f0 & a1.x) | (f1 & a1.y) | (f2 & a1.z) | (f3 & a1.w) | (f4 & c1.x) | (f5 & c1.y);
-							}
-							const uint64_t h0 = __ballot(acc0 == 0) & lmask;
-							const uint64_t h1 = __ballot(acc1 == 0) & lmask & keep1;
-							if (h0) on_hit(h0, t * 64 + j0, b, kv);
-							if (h1) on_hit(h1, t * 64 + j1, b, kv);
-						}
-					} else {
-						// candidate query words through scalar loads, two per iteration
-						const uint32_t * qbase = a.qinv + (size_t)(q0 + t * 64) * 8;
-						while (c) {
-							const uint32_t j0 = (uint32_t)__builtin_ctzll(c);
-							c &= c - 1;
-							const uint64_t keep1 = c ? ~0ULL : 0ULL;
-							const uint32_t j1 = c ? (uint32_t)__builtin_ctzll(c) : j0;
-							c &= c - 1;
-							const uint2 a0 = sld2(qbase + j0 * 8), a1 = sld2(qbase + j1 * 8);
-							uint32_t acc0 = (f0 & a0.x) | (f1 & a0.y);
-							uint32_t acc1 = (f0 & a1.x) | (f1 & a1.y);
-							if (VAR & 4) {
-								const uint64_t alive = (__ballot(acc0 == 0) | (__ballot(acc1 == 0) & keep1)) & lmask;
-								if (alive == 0) continue;
-							}
-							const uint4 b0 = sld4(qbase + j0 * 8 + 2), b1 = sld4(qbase + j1 * 8 + 2);
-							acc0 |= (f2 & b0.x) | (f3 & b0.y) | (f4 & b0.z) | (f5 & b0.w);
-							acc1 |= (f2 & b1.x) | (f3 & b1.y) | (f4 & b1.z) | (f5 & b1.w);
-							const uint64_t h0 = __ballot(acc0 == 0) & lmask;
-							const uint64_t h1 = __ballot(acc1 == 0) & lmask & keep1;
-							if (h0) on_hit(h0, t * 64 + j0, b, kv);
-							if (h1) on_hit(h1, t * 64 + j1, b, kv);
-						}
+					// candidate query words broadcast from LDS, two per iteration:
+					// the lowest and the highest candidate left (one and the same
+					// for the last of an odd count).  Scalar work per pair kept
+					// small (the scalar unit is as busy as the vector one here):
+					// bits cleared by index, and one branch over both results for
+					// the common pair without hits.
+					while (c) {
+						const uint32_t j0 = (uint32_t)__builtin_ctzll(c);
+						const uint32_t j1 = 63u - (uint32_t)__builtin_clzll(c);
+						c &= ~((1ULL << j0) | (1ULL << j1));
+						const bool has1 = j1 != j0;
+						const uint32_t * qq0 = &s_q[(t * 64 + j0) * 8];
+						const uint32_t * qq1 = &s_q[(t * 64 + j1) * 8];
+						const uint4 a0 = *reinterpret_cast<const uint4 *>(qq0);
+						const uint2 c0 = *reinterpret_cast<const uint2 *>(qq0 + 4);
+						const uint4 a1 = *reinterpret_cast<const uint4 *>(qq1);
+						const uint2 c1 = *reinterpret_cast<const uint2 *>(qq1 + 4);
+						const uint32_t acc0 = test6(f0, f1, f2, f3, f4, f5, a0.x, a0.y, a0.z, a0.w, c0.x, c0.y);
+						const uint32_t acc1 = test6(f0, f1, f2, f3, f4, f5, a1.x, a1.y, a1.z, a1.w, c1.x, c1.y);
+						const uint64_t r0 = __ballot(acc0 == 0), r1 = __ballot(acc1 == 0);
+						if (((r0 | r1) & lmask) == 0) continue;   // (r1 = r0 when j1 = j0)
+						const uint64_t h0 = r0 & lmask;
+						const uint64_t h1 = has1 ? r1 & lmask : 0ULL;
+						if (h0) on_hit(h0, t * 64 + j0, b, kv);
+						if (h1) on_hit(h1, t * 64 + j1, b, kv);
 					}
 				}
 			};
@@ -776,124 +636,21 @@ k_match_q(mq_args a) {
 				return any;
 			};
 			const uint32_t be = fb + nb;
-			if (VAR & 16) {
-				// GB blocks per round: their info with one scalar-load wait, then
-				// the words of every block that has candidates with one vector
-				// wait, then the tests; the loads of a round overlap.
-				constexpr int GB = 4;
-				for (uint32_t b0 = fb + wave; b0 < be; b0 += NW * GB) {
-					uint64_t cand[GB][TILES];
-					uint64_t any[GB];
-					uint32_t nv[GB];
+			// one block: its candidates from its mask, then its tests
+			auto visit = [&](uint32_t b) {
+				const uint32_t * bi = a.f.blk_info + (size_t)b * 8;
+				const uint4 ma = sld4(bi), mb = sld4(bi + 4);
+				uint64_t cand[TILES];
+				if (block_cands(ma, mb, cand) == 0) return;
+				++n_visit;
+				uint32_t c_f[6];
+				const uint32_t * bw = a.f.blk_words + (size_t)b * BLOCK_WORDS + lane;
 #pragma unroll
-					for (int g = 0; g < GB; ++g) {
-						// past the end: read the last block, use nothing
-						const uint32_t b = min(b0 + g * NW, be - 1);
-						const uint4 ma = sld4(a.f.blk_info + (size_t)b * 8);
-						const uint4 mb = sld4(a.f.blk_info + (size_t)b * 8 + 4);
-						nv[g] = mb.z;
-						any[g] = block_cands(ma, mb, cand[g]);
-						if (b0 + g * NW >= be) any[g] = 0;
-					}
-					uint64_t anyall = 0;
-#pragma unroll
-					for (int g = 0; g < GB; ++g) anyall |= any[g];
-					if (anyall == 0) continue;
-					uint32_t cf[GB][6];
-					uint64_t kv[GB];
-#pragma unroll
-					for (int g = 0; g < GB; ++g) {
-						kv[g] = 0;
-#pragma unroll
-						for (int j = 0; j < 6; ++j) cf[g][j] = 0;
-						if (any[g]) {
-							const uint32_t b = b0 + g * NW;
-							const uint32_t * bw = a.f.blk_words + (size_t)b * BLOCK_WORDS + lane;
-#pragma unroll
-							for (int j = 0; j < 6; ++j) cf[g][j] = bw[j * 64];
-							if (MODE == 0) kv[g] = a.f.slot_keys[(size_t)b * 64 + lane];
-						}
-					}
-#pragma unroll
-					for (int g = 0; g < GB; ++g) {
-						if (!any[g]) continue;
-						++n_visit;
-						test_block(b0 + g * NW, cf[g], kv[g], cand[g], nv[g]);
-					}
-				}
-			} else if (VAR & 8) {
-				// software pipeline: the next block's mask, words and key slots
-				// are loaded while this block is tested
-				uint4 p_ma = make_uint4(0, 0, 0, 0), p_mb = make_uint4(0, 0, 0, 0);
-				uint32_t p_f[6] = {0, 0, 0, 0, 0, 0};
-				uint64_t p_kv = 0;
-				if (fb + wave < be) {
-					const uint32_t b = fb + wave;
-					p_ma = sld4(a.f.blk_info + (size_t)b * 8);
-					p_mb = sld4(a.f.blk_info + (size_t)b * 8 + 4);
-					const uint32_t * bw = a.f.blk_words + (size_t)b * BLOCK_WORDS + lane;
-#pragma unroll
-					for (int j = 0; j < 6; ++j) p_f[j] = bw[j * 64];
-					if (MODE == 0) p_kv = a.f.slot_keys[(size_t)b * 64 + lane];
-				}
-				for (uint32_t b = fb + wave; b < be; b += NW) {
-					const uint4 ma = p_ma, mb = p_mb;
-					uint32_t c_f[6];
-#pragma unroll
-					for (int j = 0; j < 6; ++j) c_f[j] = p_f[j];
-					const uint64_t c_kv = p_kv;
-					const uint32_t bn = b + NW;
-					if (bn < be) {
-						p_ma = sld4(a.f.blk_info + (size_t)bn * 8);
-						p_mb = sld4(a.f.blk_info + (size_t)bn * 8 + 4);
-						const uint32_t * bw = a.f.blk_words + (size_t)bn * BLOCK_WORDS + lane;
-#pragma unroll
-						for (int j = 0; j < 6; ++j) p_f[j] = bw[j * 64];
-						if (MODE == 0) p_kv = a.f.slot_keys[(size_t)bn * 64 + lane];
-					}
-					uint64_t cand[TILES];
-					if (block_cands(ma, mb, cand) == 0) continue;
-					++n_visit;
-					test_block(b, c_f, c_kv, cand, mb.z);
-				}
-			} else {
-				// one block: its candidates from its mask, then its tests
-				auto visit = [&](uint32_t b) {
-					const uint32_t * bi = a.f.blk_info + (size_t)b * 8;
-					const uint4 ma = sld4(bi), mb = sld4(bi + 4);
-					uint64_t cand[TILES];
-					if (block_cands(ma, mb, cand) == 0) return;
-					++n_visit;
-					uint32_t c_f[6];
-					const uint32_t * bw = a.f.blk_words + (size_t)b * BLOCK_WORDS + lane;
-#pragma unroll
-					for (int j = 0; j < 6; ++j) c_f[j] = bw[j * 64];
-					const uint64_t c_kv = MODE == 0 ? a.f.slot_keys[(size_t)b * 64 + lane] : 0;
-					test_block(b, c_f, c_kv, cand, mb.z);
-				};
-				if (a.groups && a.f.sup_info) {
-					// Compacted steps: groups of SUP_BLOCKS blocks (aligned in
-					// the table), one group per wave at a time; a group whose
-					// AND of block masks no selected query contains is skipped
-					// whole (at 10M filters, 21M block scans per compacted
-					// launch become 14M group and block scans in a CPU model of
-					// the same layout, and the kernel 2.65 -> 2.42 ms).  Other
-					// steps keep one block per wave in turn: their items are
-					// short, and a group per wave leaves waves idle (a
-					// 1024-query step took 0.27 ms instead of 0.20).
-					const uint32_t g0 = fb / SUP_BLOCKS, g1 = (be + SUP_BLOCKS - 1) / SUP_BLOCKS;
-					for (uint32_t gi = g0 + wave; gi < g1; gi += NW) {
-						const uint32_t * si = a.f.sup_info + (size_t)gi * 8;
-						const uint4 sa = sld4(si), sb = sld4(si + 4);
-						uint64_t scand[TILES];
-						if (block_cands(sa, sb, scand) == 0) continue;
-						const uint32_t b1 = min(gi * SUP_BLOCKS + SUP_BLOCKS, be);
-						for (uint32_t b = max(gi * SUP_BLOCKS, fb); b < b1; ++b) visit(b);
-					}
-				} else {
-					for (uint32_t b = fb + wave; b < be; b += NW) visit(b);
-				}
-			}
+				for (int j = 0; j < 6; ++j) c_f[j] = bw[j * 64];
+				const uint64_t c_kv = MODE == 0 ? a.f.slot_keys[(size_t)b * 64 + lane] : 0;
+				test_block(b, c_f, c_kv, cand, mb.z);
+			};
+			for (uint32_t b = fb + wave; b < be; b += NW) visit(b);
 		}
 		if (MODE == 1 && sink.hcnt) sink.flush(lane);
 		if (KLOG && sink.hcnt) sink.drain(lane);
@@ -911,19 +668,18 @@ k_match_q(mq_args a) {
 		// (several segments, or rows filled before the launch) need no flush.
 		const bool item_hits = s_hits != 0;
 		if (LDS_BM) bm_dirty = item_hits;
-		if (MODE == 0 && LDS_BM && (item_hits || (nseg_all <= 1 && !a.qfull))) {
+		if (MODE == 0 && LDS_BM && (item_hits || (a.nseg <= 1 && !a.qfull))) {
 			const uint32_t nrows = min(q_end, q0 + NQ) - q0;
 			const uint32_t nw = nrows * kw;
 			uint32_t * dst = a.gbm + (size_t)q0 * kw;
-			if (nseg_all > 1) {
+			if (a.nseg > 1) {
 				// Other segments of the tile write the same rows: an atomic
 				// only for bits a row does not hold yet (rows fill up, and most
 				// words are then complete).  One wave per row; a row that is
 				// now full flags its query for the full-key-set exit.
 				for (uint32_t j = wave; j < nrows; j += NW) {
 					const uint32_t * src = s_bm + (size_t)j * kw;
-					const uint32_t grow = row_of(q0 + j);
-					uint32_t * drow = a.gbm + (size_t)grow * kw;
+					uint32_t * drow = a.gbm + (size_t)(q0 + j) * kw;
 					uint32_t any = 0;
 					for (uint32_t w = lane; w < kw; w += 64) any |= src[w];
 					if (__ballot(any != 0) == 0) continue;   // nothing from this segment
@@ -936,17 +692,11 @@ k_match_q(mq_args a) {
 						all &= u;
 					}
 					if (a.qfull && __ballot(all != 0xFFFFFFFFu) == 0 && lane == 0)
-						atomicMax(&a.qfull[grow], 1u);
+						atomicMax(&a.qfull[q0 + j], 1u);
 				}
 			} else {
-				// with flags (rich-filter pass, explicit units) the rows hold
-				// keys already: merge
-				if (a.map_rows) {
-					for (uint32_t w = tid; w < nw; w += NT) {
-						const uint32_t j = w / kw;
-						a.gbm[(size_t)row_of(q0 + j) * kw + (w - j * kw)] |= s_bm[w];
-					}
-				} else if (a.qfull) {
+				// with flags (rich-filter pass) the rows hold keys already: merge
+				if (a.qfull) {
 					for (uint32_t w = tid; w < nw; w += NT) dst[w] |= s_bm[w];
 				} else {
 					for (uint32_t w = tid; w < nw; w += NT) dst[w] = s_bm[w];
@@ -972,14 +722,6 @@ k_match_q(mq_args a) {
 		atomicAdd(&a.counters[3], (unsigned long long)w_test);
 		atomicAdd(&a.counters[4], (unsigned long long)w_hev);
 	}
-}
-
-// Inverted query words (6 + 2 pad per query) for the scalar-load variant.
-__global__ void __launch_bounds__(256)
-k_invert_queries(const uint32_t * __restrict__ q, uint32_t nq, uint32_t * __restrict__ qinv) {
-	const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-	if (i >= nq * 8) return;
-	qinv[i] = (i & 7) < 6 ? ~q[i] : 0u;
 }
 
 // Queue bounds for `items` work items, NQUEUE contiguous ranges.
@@ -1158,19 +900,38 @@ k_hits_write(const uint2 * __restrict__ hits, const unsigned long long * __restr
 }
 
 // Collect the submission's counters in one array for a single D2H copy.
-__global__ void k_gather_stats(const uint64_t * __restrict__ pbase, uint32_t P,
+__global__ void __launch_bounds__(64)
+k_gather_stats(const uint32_t * __restrict__ pcount, uint32_t P,
 							   const unsigned long long * __restrict__ counters,
+							   const uint64_t * __restrict__ wg_stats, uint32_t n_wg,
 							   const uint64_t * __restrict__ off, uint32_t nq,
 							   const uint64_t * __restrict__ item_prefix, uint64_t * __restrict__ out) {
-	if (threadIdx.x == 0 && blockIdx.x == 0) {
-		out[0] = pbase[P];        // (query, partition) pairs
-		out[1] = counters[0];     // hit slots taken
-		out[2] = counters[1];     // hits
+	uint64_t pairs = 0;
+	for (uint32_t p = threadIdx.x; p < P; p += 64) pairs += pcount[p];
+	uint64_t hits = threadIdx.x == 0 ? counters[1] : 0, visits = threadIdx.x == 0 ? counters[2] : 0;
+	uint64_t tests = threadIdx.x == 0 ? counters[3] : 0, events = threadIdx.x == 0 ? counters[4] : 0;
+	for (uint32_t w = threadIdx.x; w < n_wg; w += 64) {
+		hits += wg_stats[(size_t)w * 4];
+		visits += wg_stats[(size_t)w * 4 + 1];
+		tests += wg_stats[(size_t)w * 4 + 2];
+		events += wg_stats[(size_t)w * 4 + 3];
+	}
+	for (int d = 32; d > 0; d >>= 1) {
+		pairs += __shfl_xor(pairs, d, 64);
+		hits += __shfl_xor(hits, d, 64);
+		visits += __shfl_xor(visits, d, 64);
+		tests += __shfl_xor(tests, d, 64);
+		events += __shfl_xor(events, d, 64);
+	}
+	if (threadIdx.x == 0) {
+		out[0] = pairs;           // (query, partition) pairs
+		out[1] = n_wg ? hits : counters[0];   // hit slots taken
+		out[2] = hits;            // hits
 		out[3] = off ? off[nq] : 0;   // result values (none: KEY_BITMAP rows)
 		out[4] = item_prefix[P];  // work items
-		out[5] = counters[2];     // block visits
-		out[6] = counters[3];     // subset tests
-		out[7] = counters[4];     // tests with hits
+		out[5] = visits;          // block visits
+		out[6] = tests;           // subset tests
+		out[7] = events;          // tests with hits
 	}
 }
 
@@ -1257,7 +1018,8 @@ k_seg_bounds(const uint64_t * __restrict__ prefix, uint32_t nb, uint32_t nseg, u
 __global__ void __launch_bounds__(256)
 k_rich_rows(const uint32_t * __restrict__ q, uint32_t nq, uint32_t qpw, const uint32_t * __restrict__ rw,
 			const uint32_t * __restrict__ rbm, uint32_t nr, uint32_t nfull, uint32_t kw, uint32_t last_mask,
-			uint32_t * __restrict__ gbm, uint32_t * __restrict__ qfull) {
+			uint32_t * __restrict__ gbm, uint32_t * __restrict__ qfull, uint32_t * __restrict__ active,
+			uint32_t * __restrict__ qact, uint32_t * __restrict__ n_active) {
 	const uint32_t lane = threadIdx.x & 63;
 	const uint32_t base = (blockIdx.x * 4 + (threadIdx.x >> 6)) * qpw;
 	if (base >= nq) return;
@@ -1349,86 +1111,19 @@ k_rich_rows(const uint32_t * __restrict__ q, uint32_t nq, uint32_t qpw, const ui
 		if (lane == j) done_full = f;
 	}
 	if (valid) qfull[qi] = done_full ? 2u : 0u;
-}
-
-// Queries whose rows are not yet full after the rich-filter pass, listed
-// for a match over them alone, in order of a key made of their ACT_KEY_BITS
-// rarest bits (the table's significance order), those holding the rarest
-// bits first.  A tile then holds queries that share their rare bits, and a
-// block, whose AND mask holds the rare bits of its filters, has a candidate
-// in fewer tiles: at 10M filters and about 10k active queries, 8.8M
-// (tile, block) visits instead of 12.5M in arbitrary order (measured on the
-// CPU over the same layout).  Order within a key is arbitrary; results do
-// not depend on the order.
-constexpr uint32_t ACT_KEY_BITS = 12;
-constexpr uint32_t ACT_BUCKETS = 1u << ACT_KEY_BITS;
-
-struct act_key_bits {
-	uint8_t pos[ACT_KEY_BITS];   // bit positions, rarest first
-};
-
-__device__ inline uint32_t act_bucket(const uint32_t * __restrict__ qw, const act_key_bits & kb) {
-	uint32_t k = 0;
-#pragma unroll
-	for (uint32_t i = 0; i < ACT_KEY_BITS; ++i) {
-		const uint32_t b = kb.pos[i];
-		k = (k << 1) | ((qw[b >> 5] >> (b & 31)) & 1u);
-	}
-	return (ACT_BUCKETS - 1u) - k;
-}
-
-// Active queries per key bucket (LDS counters, one global atomic per
-// non-empty bucket and workgroup).
-__global__ void __launch_bounds__(256)
-k_act_hist(const uint32_t * __restrict__ q, uint32_t nq, const uint32_t * __restrict__ qfull, act_key_bits kb,
-		   uint32_t * __restrict__ hist) {
-	__shared__ uint32_t h[ACT_BUCKETS];
-	for (uint32_t i = threadIdx.x; i < ACT_BUCKETS; i += 256) h[i] = 0;
-	__syncthreads();
-	for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < nq; i += gridDim.x * 256)
-		if (qfull[i] == 0u) atomicAdd(&h[act_bucket(q + (size_t)i * 8, kb)], 1u);
-	__syncthreads();
-	for (uint32_t i = threadIdx.x; i < ACT_BUCKETS; i += 256)
-		if (h[i]) atomicAdd(&hist[i], h[i]);
-}
-
-// Each active query to its bucket's next slot; the active count to
-// n_active[0] (base[ACT_BUCKETS] is the total).
-__global__ void __launch_bounds__(256)
-k_act_scatter(const uint32_t * __restrict__ q, uint32_t nq, const uint32_t * __restrict__ qfull, act_key_bits kb,
-			  const uint64_t * __restrict__ base, uint32_t * __restrict__ cursor, uint32_t * __restrict__ list,
-			  uint32_t * __restrict__ n_active) {
-	const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-	if (i == 0) n_active[0] = (uint32_t)base[ACT_BUCKETS];
-	if (i >= nq || qfull[i] != 0u) return;
-	const uint32_t b = act_bucket(q + (size_t)i * 8, kb);
-	list[base[b] + atomicAdd(&cursor[b], 1u)] = i;
-}
-
-// Shape of a compacted step from its active query count: ceil(n / nqg)
-// tiles, cut into segments as the host cuts other steps (about two items
-// per resident workgroup, at most seg_max blocks each).  act[1..3] = tiles,
-// segments, blocks per segment; queue bounds and the item count follow.
-__global__ void k_init_queues_active(uint32_t * __restrict__ act, uint32_t nqg, uint32_t nblk, uint32_t resident,
-									 uint32_t seg_max, uint64_t * __restrict__ qbeg,
-									 unsigned long long * __restrict__ qnext, uint64_t * __restrict__ n_items) {
-	const uint32_t t = threadIdx.x;
-	const uint64_t tiles = ((uint64_t)act[0] + nqg - 1) / nqg;
-	uint32_t nseg = 1;
-	if (tiles > 0) {
-		nseg = (uint32_t)min((2ull * resident + tiles - 1) / tiles, (uint64_t)max(nblk / 16, 1u));
-		nseg = max(nseg, (nblk + seg_max - 1) / seg_max);
-	}
-	const uint32_t sb = nseg > 1 ? (nblk + nseg - 1) / nseg : max(nblk, 1u);
-	if (nseg > 1) nseg = (nblk + sb - 1) / sb;
-	const uint64_t items = tiles * nseg;
-	if (t <= NQUEUE) qbeg[t] = items * t / NQUEUE;
-	if (t < NQUEUE) qnext[t * QPAD] = items * t / NQUEUE;
-	if (t == 0) {
-		act[1] = (uint32_t)tiles;
-		act[2] = nseg;
-		act[3] = sb;
-		*n_items = items;
+	if (active) {
+		const uint64_t am = __ballot(valid && !done_full);
+		if (am) {
+			uint32_t at = 0;
+			if (lane == 0) at = atomicAdd(n_active, (uint32_t)__popcll(am));
+			at = __shfl(at, 0, 64) + mbcnt64(am);
+			if (valid && !done_full) {
+				active[at] = qi;
+				uint4 * d = reinterpret_cast<uint4 *>(qact + (size_t)at * 8);
+				d[0] = x;
+				d[1] = make_uint4(y.x, y.y, 0u, 0u);
+			}
+		}
 	}
 }
 
@@ -1473,43 +1168,27 @@ k_lookup_hist(const uint32_t * __restrict__ q, uint32_t nq, const uint32_t * __r
 
 using mq_fn = void (*)(mq_args);
 
-template <int MODE, bool LDS_BM, int TILES, int VAR>
+template <int MODE, bool LDS_BM, int TILES>
 mq_fn pick_q_waves(int nw) {
 	switch (nw) {
-	case 4: return k_match_q<MODE, LDS_BM, TILES, 4, VAR>;
-	case 16: return k_match_q<MODE, LDS_BM, TILES, 16, VAR>;
-	default: return k_match_q<MODE, LDS_BM, TILES, 8, VAR>;
+	case 4: return k_match_q<MODE, LDS_BM, TILES, 4>;
+	case 16: return k_match_q<MODE, LDS_BM, TILES, 16>;
+	default: return k_match_q<MODE, LDS_BM, TILES, 8>;
 	}
 }
 
-template <int MODE, bool LDS_BM, int VAR>
+template <int MODE, bool LDS_BM>
 mq_fn pick_q_tiles(int tiles, int nw) {
 	switch (tiles) {
-	case 1: return pick_q_waves<MODE, LDS_BM, 1, VAR>(nw);
-	case 2: return pick_q_waves<MODE, LDS_BM, 2, VAR>(nw);
-	default: return pick_q_waves<MODE, LDS_BM, 4, VAR>(nw);
+	case 1: return pick_q_waves<MODE, LDS_BM, 1>(nw);
+	case 2: return pick_q_waves<MODE, LDS_BM, 2>(nw);
+	default: return pick_q_waves<MODE, LDS_BM, 4>(nw);
 	}
 }
 
-template <int VAR>
-mq_fn pick_q_mode(int mode, bool lds_bm, int tiles, int nw) {
-	if (mode == 0) return lds_bm ? pick_q_tiles<0, true, VAR>(tiles, nw) : pick_q_tiles<0, false, VAR>(tiles, nw);
-	return pick_q_tiles<1, false, VAR>(tiles, nw);
-}
-
-mq_fn pick_match_q(int mode, bool lds_bm, int tiles, int nw, int var) {
-	switch (var) {
-	case 1: return pick_q_mode<1>(mode, lds_bm, tiles, nw);
-	case 2: return pick_q_mode<2>(mode, lds_bm, tiles, nw);
-	case 3: return pick_q_mode<3>(mode, lds_bm, tiles, nw);
-	case 4: return pick_q_mode<4>(mode, lds_bm, tiles, nw);
-	case 5: return pick_q_mode<5>(mode, lds_bm, tiles, nw);
-	case 6: return pick_q_mode<6>(mode, lds_bm, tiles, nw);
-	case 7: return pick_q_mode<7>(mode, lds_bm, tiles, nw);
-	case 10: return pick_q_mode<10>(mode, lds_bm, tiles, nw);
-	case 18: return pick_q_mode<18>(mode, lds_bm, tiles, nw);
-	default: return pick_q_mode<2>(mode, lds_bm, tiles, nw);
-	}
+mq_fn pick_match_q(int mode, bool lds_bm, int tiles, int nw) {
+	if (mode == 0) return lds_bm ? pick_q_tiles<0, true>(tiles, nw) : pick_q_tiles<0, false>(tiles, nw);
+	return pick_q_tiles<1, false>(tiles, nw);
 }
 
 } // namespace
@@ -1526,7 +1205,10 @@ struct tm_ring {
 
 	uint32_t * h_q = nullptr;      // pinned staging, max_q x 8
 	uint32_t * d_q = nullptr;      // max_q x 8
-	uint32_t * d_qinv = nullptr;   // max_q x 8, inverted (variant 1)
+	uint32_t * d_qact = nullptr;   // max_q x 8: words of the active queries
+	int mx_groups[MX_MODES] = {};
+	uint64_t * d_wgstat = nullptr;  // MX_MAX_GROUPS x 4: the matrix kernel's statistics
+	uint32_t n_wgstat = 0;          // records of the last step (0: counted in d_cnt)
 	uint32_t * d_pcount = nullptr; // P
 	uint64_t * d_pbase = nullptr;  // P + 1
 	unsigned long long * d_pcur = nullptr;
@@ -1541,9 +1223,7 @@ struct tm_ring {
 	uint32_t * d_gbm = nullptr;
 	uint32_t * d_qfull = nullptr;   // max_q: full-key-set flags of merged rows
 	uint32_t * d_active = nullptr;  // max_q: queries left after the rich-filter pass
-	uint32_t * d_nact = nullptr;    // active queries, their tiles, segments, blocks per segment
-	uint32_t * d_ahist = nullptr;   // 2 x ACT_BUCKETS: active queries per key bucket, then cursors
-	uint64_t * d_abase = nullptr;   // ACT_BUCKETS + 1: first slot of each key bucket
+	uint32_t * d_nact = nullptr;    // their count
 	uint32_t * d_bw = nullptr;      // per block: work estimate (weighted segments)
 	uint64_t * d_bprefix = nullptr; // n_blocks + 1: exclusive prefix of d_bw
 	uint64_t * d_bscan = nullptr;   // scan scratch for d_bprefix
@@ -1564,6 +1244,9 @@ struct tm_ring {
 	size_t scan_words = 0;
 	uint64_t * d_stat = nullptr;
 	uint64_t * h_stat = nullptr;   // pinned, 8
+	uint32_t * d_hcnt = nullptr;   // hit-list steps: values per segment and query
+	uint64_t hcnt_cap = 0;
+	bool hits_grown = false;       // the last step had more hits than the ring's hit capacity
 	uint32_t * d_log = nullptr;
 	uint64_t log_cap = 0;
 	uint32_t * d_stage = nullptr;     // plain: key bitmap rows of one unit's batch
@@ -1592,7 +1275,7 @@ struct tm_ring {
 	bool use_iorder = false;
 
 	// effective launch parameters
-	int tiles = 4, wgs_per_cu = 2, waves = 8, variant = 1;
+	int tiles = 4, wgs_per_cu = 2, waves = 8;
 	int wgs_for[3] = {1, 1, 1};     // resident workgroups per CU with 4, 8, 16 waves
 	uint32_t chunk = 256;
 	uint32_t plain_bq = 256;   // PLAIN: queries per (partition, batch) unit
@@ -1667,9 +1350,11 @@ void tm_ring::release() {
 	h_stat = nullptr;
 	h_step = nullptr;
 	dfree(d_step);
-	dfree(d_q); dfree(d_qinv); dfree(d_pcount); dfree(d_pbase); dfree(d_pcur); dfree(d_list);
+	dfree(d_q); dfree(d_qact); dfree(d_wgstat); dfree(d_hcnt);
+	hcnt_cap = 0;
+	 dfree(d_pcount); dfree(d_pbase); dfree(d_pcur); dfree(d_list);
 	dfree(d_sched); dfree(d_iprefix); dfree(d_qbeg); dfree(d_qnext); dfree(d_porder);
-	dfree(d_gbm); dfree(d_qfull); dfree(d_active); dfree(d_nact); dfree(d_ahist); dfree(d_abase); dfree(d_bw); dfree(d_bprefix); dfree(d_bscan); dfree(d_segb); dfree(d_hits); dfree(d_qcount); dfree(d_off); dfree(d_qcur);
+	dfree(d_gbm); dfree(d_qfull); dfree(d_active); dfree(d_nact); dfree(d_bw); dfree(d_bprefix); dfree(d_bscan); dfree(d_segb); dfree(d_hits); dfree(d_qcount); dfree(d_off); dfree(d_qcur);
 	dfree(d_vals); dfree(d_cnt); dfree(d_scan); dfree(d_stat); dfree(d_log);
 	dfree(d_units); dfree(d_ufeat); dfree(d_stage); dfree(d_uitems); dfree(d_ubeg); dfree(d_unext);
 	dfree(d_xunits); dfree(d_xprefix); dfree(d_iota);
@@ -1721,13 +1406,12 @@ int resolve_params(tm_ring * r) {
 	r->chunk = 1u << 30;   // work items of the lookup: one per (partition, batch)
 	const size_t max_lds = (size_t)dev().max_lds;
 	const size_t nq_grp = (size_t)r->tiles * 64;
-	r->variant = ((c.variant >= 1 && c.variant <= 7) || c.variant == 10 || c.variant == 18) ? (int)c.variant : 2;
 	int nw = c.waves_per_group ? (int)c.waves_per_group : (c.schedule == TM_SCHED_PLAIN ? 8 : 4);
 	if (nw != 4 && nw != 8 && nw != 16)
 		return set_error(TM_ERR_INVALID, "waves_per_group must be 4, 8 or 16 (got %d)", nw);
 	r->waves = nw;
 	size_t static_lds = nq_grp * 32 + 64 + (mode_of(c) == 1 ? (size_t)nw * HBUF * 8 : 8) +
-						((mode_of(c) == 0 && (r->variant & 2)) ? (size_t)nw * 64 * 16 : 16);
+						(mode_of(c) == 0 ? (size_t)nw * 64 * 16 : 16);
 	size_t bm = nq_grp * r->kw * 4;
 	r->lds_bm = (mode_of(c) == 0) && bm + static_lds <= max_lds;
 	r->stage_lds = r->lds_bm ? bm : 0;
@@ -1735,12 +1419,12 @@ int resolve_params(tm_ring * r) {
 	for (int i = 0; i < 3; ++i) {
 		// resident workgroups per CU from the kernel's registers and LDS
 		const int w = 4 << i;
-		const mq_fn fn = pick_match_q(mode_of(c), r->lds_bm, r->tiles, w, r->variant);
+		const mq_fn fn = pick_match_q(mode_of(c), r->lds_bm, r->tiles, w);
 		int n = 0;
 		if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(fn), w * 64,
 														  r->stage_lds) != hipSuccess || n < 1) {
 			const size_t st = nq_grp * 32 + 64 + (mode_of(c) == 1 ? (size_t)w * HBUF * 8 : 8) +
-							  ((mode_of(c) == 0 && (r->variant & 2)) ? (size_t)w * 64 * 16 : 16);
+							  (mode_of(c) == 0 ? (size_t)w * 64 * 16 : 16);
 			n = std::max(1, std::min((int)(std::min<size_t>(160 * 1024, max_lds) / (r->stage_lds + st)), 28 / w));
 		}
 		r->wgs_for[i] = std::max(1, std::min(want, n));
@@ -1752,11 +1436,8 @@ int resolve_params(tm_ring * r) {
 // Waves per workgroup of a persistent step of `tiles` query tiles: the
 // configured value, or by default more waves for fewer tiles (a small step
 // has few items in flight per tile, and more waves share each item's blocks).
-int step_waves(const tm_ring * r, uint64_t tiles, bool compacted) {
+int step_waves(const tm_ring * r, uint64_t tiles) {
 	if (r->cfg.waves_per_group) return r->waves;
-	// a compacted step has few tiles but many segments: 4 waves (measured at
-	// 10M filters, 1M queries: 2.8 ms against 3.0 ms with 8)
-	if (compacted) return 4;
 	return tiles <= 16 ? 16 : tiles <= 256 ? 8 : 4;
 }
 int wgs_for_waves(const tm_ring * r, int nw) { return r->wgs_for[nw == 4 ? 0 : nw == 8 ? 1 : 2]; }
@@ -1803,6 +1484,8 @@ void enqueue_front(tm_ring * r, uint32_t nq) {
 					   r->plain_bq, r->chunk, r->d_sched, r->d_iprefix, r->d_qbeg, r->d_qnext);
 }
 
+void enqueue_stats(tm_ring * r, uint32_t nq);
+
 void enqueue_finalize(tm_ring * r, uint32_t nq) {
 	hipStream_t s = r->s;
 	const int mode = r->cfg.mode;
@@ -1833,8 +1516,148 @@ void enqueue_finalize(tm_ring * r, uint32_t nq) {
 			hipLaunchKernelGGL(k_hits_write<false>, dim3(gh), dim3(256), 0, s, r->d_hits, r->d_cnt, r->hit_cap, v,
 							   r->d_qcur, r->d_vals, r->val_cap);
 	}
-	hipLaunchKernelGGL(k_gather_stats, dim3(1), dim3(64), 0, s, r->d_pbase, r->P, r->d_cnt,
+	enqueue_stats(r, nq);
+}
+
+void enqueue_stats(tm_ring * r, uint32_t nq) {
+	hipStream_t s = r->s;
+	const int mode = r->cfg.mode;
+	hipLaunchKernelGGL(k_gather_stats, dim3(1), dim3(64), 0, s, r->d_pcount, r->P, r->d_cnt,
+					   r->d_wgstat, r->n_wgstat,
 					   mode == TM_MODE_KEY_BITMAP ? (const uint64_t *)nullptr : r->d_off, nq, r->d_iprefix, r->d_stat);
+}
+
+// Zeroes what a step's kernels count in.
+__global__ void __launch_bounds__(256)
+k_step_init(uint32_t * __restrict__ pcount, uint32_t P, unsigned long long * __restrict__ cnt,
+			unsigned long long * __restrict__ qnext, uint32_t n_queues, uint32_t * __restrict__ nact) {
+	const uint32_t t = threadIdx.x;
+	for (uint32_t p = t; p < P; p += 256) pcount[p] = 0;
+	if (t < 8) cnt[t] = 0;
+	if (t < n_queues) qnext[t * QPAD] = 0;
+	if (t == 8 && nact) nact[0] = 0;
+}
+
+mx_args matrix_args(tm_ring * r, int mode) {
+	mx_args a;
+	std::memset(&a, 0, sizeof(a));
+	a.f = r->fib->view();
+	a.q = r->d_q;
+	a.nblk = r->fib->n_blocks;
+	a.seg_fixed = r->cfg.chunk_blocks;
+	if (!r->mx_groups[mode]) r->mx_groups[mode] = (int)mx_resident(mode);
+	a.resident = (uint32_t)r->mx_groups[mode];
+	a.wg_stats = r->d_wgstat;
+	a.qnext = r->d_qnext;
+	a.gbm = r->d_gbm;
+	a.n_items = r->d_iprefix + r->P;
+	a.rich_bm = r->fib->d_rich_bm;
+	a.n_rich = r->fib->n_rich;
+	a.slot_epoch = r->fib->slot_epoch;
+	a.epoch = r->epoch;
+	return a;
+}
+
+// Segments of a hit-list step: as many as its per-segment counts may take.
+mx_shape hits_shape(const tm_ring * r, uint32_t nq, uint32_t resident) {
+	const uint64_t rows = std::max<uint64_t>(1, HCNT_MAX / std::max<uint32_t>(nq, 1));
+	const uint32_t seg_min = (uint32_t)((r->fib->n_blocks + rows - 1) / rows);
+	return mx_shape_of(MX_COUNT, nq, r->fib->n_blocks, resident, r->cfg.chunk_blocks ? std::max(r->cfg.chunk_blocks, seg_min) : 0, seg_min);
+}
+
+// HITS and KEYS_ALL: one pass counts each query's values by segment, their
+// prefix sums place them, and a second pass writes them.  The match runs
+// twice, but without a hit list in between, whose entries (8 bytes written
+// and read twice, two contended global atomics each) cost more: 1024
+// queries at 10M filters, 7.4M hits, took 1.1 ms to match and 3.4 ms to
+// group from a list.
+int enqueue_values(tm_ring * r, mx_args a, uint32_t rows, uint32_t grid, bool events) {
+	hipStream_t s = r->s;
+	const bool ids = r->cfg.mode == TM_MODE_HITS;
+	a.hcnt = r->d_hcnt;
+	r->n_wgstat = grid;
+	if (events) TM_HIP(hipEventRecord(r->em0, s));
+	mx_launch(a, ids ? MX_COUNT : MX_COUNT_KEYS, grid, s);
+	mx_prefix(r->d_hcnt, rows, a.nq, r->d_qcount, s);
+	scan_u32_to_u64(r->d_qcount, r->d_off, a.nq, r->d_scan, s);
+	a.qnext = r->d_qnext + NQUEUE * QPAD;
+	a.off = r->d_off;
+	a.vals = r->d_vals;
+	a.vcap = r->val_cap;
+	mx_launch(a, ids ? MX_WRITE : MX_WRITE_KEYS, grid, s);
+	TM_HIP(hipGetLastError());
+	if (events) TM_HIP(hipEventRecord(r->em1, s));
+	r->step_weighted = false;
+	enqueue_stats(r, a.nq);
+	return TM_OK;
+}
+
+// The persistent step on the matrix cores.
+int enqueue_matrix(tm_ring * r, uint32_t nq, bool events) {
+	hipStream_t s = r->s;
+	const uint32_t P = r->P;
+	const bool keys = mode_of(r->cfg) == 0;
+	const bool exit_on = keys && r->lds_bm && r->kw > 0 && r->cfg.full_exit != 2;
+	const bool rich_pass = keys && r->kw > 0 && r->fib->n_rich > 0 && nq > 0;
+	const bool compact = rich_pass && exit_on;
+	const uint32_t last_mask = (r->fib->n_keys & 31) ? (1u << (r->fib->n_keys & 31)) - 1u : 0xFFFFFFFFu;
+	hipLaunchKernelGGL(k_step_init, dim3(1), dim3(256), 0, s, r->d_pcount, P, r->d_cnt, r->d_qnext,
+					   keys ? NQUEUE : 2 * NQUEUE, r->d_nact);
+	if (rich_pass) {
+		uint32_t qpw = 64;
+		while (qpw > 1 && (uint64_t)nq < (uint64_t)qpw * 4096) qpw >>= 1;
+		const uint32_t waves = (nq + qpw - 1) / qpw;
+		hipLaunchKernelGGL(k_rich_rows, dim3((waves + 3) / 4), dim3(256), 0, s, r->d_q, nq, qpw, r->fib->d_rich_words,
+						   r->fib->d_rich_bm, r->fib->n_rich, r->fib->n_rich_full, r->kw, last_mask, r->d_gbm,
+						   r->d_qfull, compact ? r->d_active : nullptr, r->d_qact, r->d_nact);
+	} else if (keys) {
+		fill_u32(r->d_gbm, 0, (uint64_t)nq * r->kw, s);
+	}
+	if (nq) {
+		if (P <= 16384) {
+			const uint32_t gh = (uint32_t)std::min<uint64_t>((nq + 255) / 256, 2048);
+			hipLaunchKernelGGL(k_lookup_hist, dim3(gh), dim3(256), (size_t)P * 4, s, r->d_q, nq, r->fib->part_info, P,
+							   r->d_pcount);
+		} else {
+			hipLaunchKernelGGL(k_lookup_count, dim3((nq + 255) / 256), dim3(256), 0, s, r->d_q, nq, r->fib->part_info,
+							   P, r->d_pcount);
+		}
+	}
+	if (!keys) {
+		mx_args a = matrix_args(r, MX_COUNT);
+		a.nq = nq;
+		const mx_shape h = hits_shape(r, nq, a.resident);
+		a.seg_fixed = h.seg;
+		return enqueue_values(r, a, h.nseg, a.resident, events);
+	}
+	// Rows in local memory where the match sets most of their bits: without
+	// a rich-filter pass, or in small steps where no rich filter holds every
+	// key.  In larger ones more queries per item win.  Both sides measured
+	// (filters, queries: local, HBM): 104k, 4.9k: 0.40, 0.49 ms; 101k, 44k:
+	// 1.08, 1.32; 402k, 13k: 0.51, 0.48; 158k, 612k: 14.9, 13.3; 1M, 100k:
+	// 1.73, 1.25.
+	const bool sparse = !rich_pass || (compact && r->fib->n_rich_full == 0 &&
+									   (uint64_t)nq * r->fib->n_blocks <= ROWS_LDS_MAX_WORK);
+	const int mode = sparse && r->kw <= MX_LDS_KW && r->kw > 0 ? MX_KEYS_LDS : MX_KEYS;
+	mx_args a = matrix_args(r, mode);
+	a.nq = nq;
+	if (compact) {
+		a.q = r->d_qact;
+		a.qmap = r->d_active;
+		a.nq_dev = r->d_nact;
+	}
+	a.rich_done = rich_pass;
+	a.qfull = rich_pass && !compact ? r->d_qfull : nullptr;
+	r->qfull_valid = rich_pass;
+	a.step_vals = (r->cfg.use_graph && r->d_step) ? r->d_step : nullptr;
+	if (events) TM_HIP(hipEventRecord(r->em0, s));
+	mx_launch(a, mode, a.resident, s);
+	r->n_wgstat = a.resident;
+	TM_HIP(hipGetLastError());
+	if (events) TM_HIP(hipEventRecord(r->em1, s));
+	r->step_weighted = false;
+	enqueue_finalize(r, nq);
+	return TM_OK;
 }
 
 // The persistent step: everything between the query upload and the stats.
@@ -1847,13 +1670,9 @@ int enqueue_persistent(tm_ring * r, uint32_t nq, bool events) {
 	const uint64_t tiles = (nq + nqg - 1) / nqg;
 	const bool exit_on = keyrows(r->cfg) && r->lds_bm && r->kw > 0 && r->cfg.full_exit != 2;
 	const bool rich_pass = exit_on && r->fib->n_rich > 0 && nq > 0;
-	// Compacted step: only the queries whose rows the pass leaves incomplete
-	// are matched (large steps only: the extra kernels cost about 0.1 ms,
-	// more than a step of up to ~8k queries gains)
-	const uint64_t compact_min = r->cfg.compact_tiles ? r->cfg.compact_tiles : COMPACT_MIN_TILES;
-	const bool compact = rich_pass && tiles > compact_min && !r->use_iorder && !r->cfg.log_units &&
-						 (r->variant & 1) == 0;
-	const int nw = step_waves(r, tiles, compact);
+	if (!r->use_iorder && !r->cfg.log_units && (!exit_on || rich_pass)) return enqueue_matrix(r, nq, events);
+	r->n_wgstat = 0;
+	const int nw = step_waves(r, tiles);
 	// Small submissions: cut each tile's work into block segments so that
 	// the items fill the GPU (about two per resident workgroup).  Needs the
 	// key bitmaps in LDS (flushed with atomicOr) or the hit-list modes.
@@ -1901,51 +1720,20 @@ int enqueue_persistent(tm_ring * r, uint32_t nq, bool events) {
 		const uint32_t waves = (nq + qpw - 1) / qpw;
 		hipLaunchKernelGGL(k_rich_rows, dim3((waves + 3) / 4), dim3(256), 0, s, r->d_q, nq, qpw, r->fib->d_rich_words,
 						   r->fib->d_rich_bm, r->fib->n_rich, r->fib->n_rich_full, r->kw, last_mask, r->d_gbm,
-						   r->d_qfull);
+						   r->d_qfull, (uint32_t *)nullptr, (uint32_t *)nullptr, (uint32_t *)nullptr);
 	} else if (nseg > 1 && keyrows(r->cfg)) {
 		fill_u32(r->d_gbm, 0, (uint64_t)nq * r->kw, s);
 		fill_u32(r->d_qfull, 0, nq, s);
 	}
-	// Compacted step: the active queries in tiles of their own (rows and
-	// flags through the list); their count stays on the device.  The lookup
-	// counts of every query come from k_lookup_hist, as the match sees only
-	// the active ones.
-	if (compact) {
-		fill_u32(r->d_nact, 0, 4, s);
-		if (P <= 16384) {
-			const uint32_t gh = (uint32_t)std::min<uint64_t>((nq + 255) / 256, 2048);
-			hipLaunchKernelGGL(k_lookup_hist, dim3(gh), dim3(256), (size_t)P * 4, s, r->d_q, nq, r->fib->part_info, P,
-							   r->d_pcount);
-		} else {
-			hipLaunchKernelGGL(k_lookup_count, dim3((nq + 255) / 256), dim3(256), 0, s, r->d_q, nq, r->fib->part_info,
-							   P, r->d_pcount);
-		}
-		act_key_bits kb;
-		for (uint32_t i = 0; i < ACT_KEY_BITS; ++i) kb.pos[i] = (uint8_t)r->fib->h_order[i];
-		fill_u32(r->d_ahist, 0, 2 * ACT_BUCKETS, s);   // counts, then cursors
-		hipLaunchKernelGGL(k_act_hist, dim3((uint32_t)std::min<uint64_t>((nq + 255) / 256, 1024)), dim3(256), 0, s,
-						   r->d_q, nq, r->d_qfull, kb, r->d_ahist);
-		scan_u32_to_u64(r->d_ahist, r->d_abase, ACT_BUCKETS, r->d_scan, s);
-		hipLaunchKernelGGL(k_act_scatter, dim3((nq + 255) / 256), dim3(256), 0, s, r->d_q, nq, r->d_qfull, kb,
-						   r->d_abase, r->d_ahist + ACT_BUCKETS, r->d_active, r->d_nact);
-		const uint32_t seg_max = r->cfg.chunk_blocks ? r->cfg.chunk_blocks : SEG_MAX_BLOCKS_COMPACT;
-		hipLaunchKernelGGL(k_init_queues_active, dim3(1), dim3(64), 0, s, r->d_nact, (uint32_t)nqg, nblk,
-						   (uint32_t)resident, seg_max, r->d_qbeg, r->d_qnext, r->d_iprefix + P);
-	} else {
-		hipLaunchKernelGGL(k_init_queues, dim3(1), dim3(64), 0, s, items, r->d_qbeg, r->d_qnext);
-	}
+	hipLaunchKernelGGL(k_init_queues, dim3(1), dim3(64), 0, s, items, r->d_qbeg, r->d_qnext);
 	mq_args a;
 	std::memset(&a, 0, sizeof(a));
 	a.f = r->fib->view();
 	a.q = r->d_q;
 	a.nq = nq;
-	a.nq_dev = compact ? r->d_nact : nullptr;
-	a.ntiles_dev = compact ? r->d_nact + 1 : nullptr;
-	a.map_rows = compact;
 	a.porder = r->have_order ? r->d_porder : nullptr;
 	a.iorder = r->use_iorder ? r->d_iorder : nullptr;
 	a.full_exit = exit_on;
-	a.groups = compact;
 	a.last_mask = last_mask;
 	a.slot_epoch = r->fib->slot_epoch;
 	a.epoch = r->epoch;
@@ -1953,14 +1741,13 @@ int enqueue_persistent(tm_ring * r, uint32_t nq, bool events) {
 	a.ntiles = (uint32_t)tiles;
 	a.nseg = nseg;
 	a.seg_blocks = seg_blocks;
-	a.segb = weighted && !compact ? r->d_segb : nullptr;
+	a.segb = weighted ? r->d_segb : nullptr;
 	a.blk_lo = 0;
 	a.blk_hi = nblk;
 	a.log_unit = -1;
-	a.qmap = compact ? r->d_active : nullptr;
 	a.qnext = r->d_qnext;
 	a.qbeg = r->d_qbeg;
-	a.pcount = compact ? nullptr : r->d_pcount;
+	a.pcount = r->d_pcount;
 	a.gbm = r->d_gbm;
 	// flags hold this submission's state: cleared or set by the pass above
 	a.qfull = (nseg > 1 || rich_pass) ? r->d_qfull : nullptr;
@@ -1970,20 +1757,13 @@ int enqueue_persistent(tm_ring * r, uint32_t nq, bool events) {
 	a.counters = r->d_cnt;
 	a.log = r->cfg.log_units ? r->d_log : nullptr;
 	a.log_cap = r->log_cap;
-	if (r->variant & 1) {
-		a.qinv = r->d_qinv;
-		const uint64_t nw = (uint64_t)nq * 8;
-		hipLaunchKernelGGL(k_invert_queries, dim3((uint32_t)std::max<uint64_t>(1, (nw + 255) / 256)), dim3(256), 0, s,
-						   r->d_q, nq, r->d_qinv);
-	}
-	mq_fn fn = pick_match_q(mode_of(r->cfg), r->lds_bm, r->tiles, nw, r->variant);
+	mq_fn fn = pick_match_q(mode_of(r->cfg), r->lds_bm, r->tiles, nw);
 	uint32_t grid = (uint32_t)std::min<uint64_t>(resident, std::max<uint64_t>(items, 1));
 	if (events) TM_HIP(hipEventRecord(r->em0, s));
 	hipLaunchKernelGGL(fn, dim3(grid), dim3(nw * 64), r->stage_lds, s, a);
 	TM_HIP(hipGetLastError());
 	if (events) TM_HIP(hipEventRecord(r->em1, s));
-	scan_u32_to_u64(r->d_pcount, r->d_pbase, P, r->d_scan, s);
-	if (!compact) fill_u64(r->d_iprefix + P, items, 1, s);
+	fill_u64(r->d_iprefix + P, items, 1, s);
 	enqueue_finalize(r, nq);
 	return TM_OK;
 }
@@ -2055,6 +1835,7 @@ int enqueue_plain(tm_ring * r, uint32_t nq) {
 }
 
 int run_plain(tm_ring * r, uint32_t nq, const uint32_t * list, std::vector<punit> & units) {
+	r->n_wgstat = 0;
 	hipStream_t s = r->s;
 	const uint32_t bq = r->plain_bq;
 	const uint64_t resident = (uint64_t)dev().num_cu * r->wgs_per_cu;
@@ -2117,7 +1898,7 @@ int run_plain(tm_ring * r, uint32_t nq, const uint32_t * list, std::vector<punit
 	a.slot_epoch = f->slot_epoch;
 	a.epoch = r->epoch;
 	a.last_mask = 0xFFFFFFFFu;
-	mq_fn fn = pick_match_q(mode_of(r->cfg), r->lds_bm, r->tiles, r->waves, r->variant);
+	mq_fn fn = pick_match_q(mode_of(r->cfg), r->lds_bm, r->tiles, r->waves);
 	TM_HIP(hipEventRecord(r->em0, s));
 	for (uint32_t i = 0; i < nu; ++i) {
 		const punit & u = units[i];
@@ -2176,7 +1957,7 @@ int ensure_capacity(tm_ring * r) {
 		TM_CHECK(dalloc(&r->d_sched, P + 1));
 		TM_CHECK(dalloc(&r->d_iprefix, P + 1));
 		TM_CHECK(dalloc(&r->d_qbeg, NQUEUE + 1));
-		TM_CHECK(dalloc(&r->d_qnext, NQUEUE * QPAD));
+		TM_CHECK(dalloc(&r->d_qnext, 2 * NQUEUE * QPAD));
 		TM_CHECK(dalloc(&r->d_porder, P + 1));
 		TM_CHECK(dalloc(&r->d_cnt, 8));
 		TM_CHECK(dalloc(&r->d_stat, 8));
@@ -2196,13 +1977,6 @@ int ensure_capacity(tm_ring * r) {
 		TM_CHECK(dalloc(&r->d_qfull, std::max<uint32_t>(r->max_q, 1)));
 		TM_CHECK(dalloc(&r->d_active, std::max<uint32_t>(r->max_q, 1)));
 		TM_CHECK(dalloc(&r->d_nact, 4));
-		TM_CHECK(dalloc(&r->d_ahist, 2 * ACT_BUCKETS));
-		TM_CHECK(dalloc(&r->d_abase, ACT_BUCKETS + 1));
-	}
-	if (r->scan_words < scan_tmp_words(ACT_BUCKETS)) {   // the key buckets' scan
-		dfree(r->d_scan);
-		r->scan_words = scan_tmp_words(ACT_BUCKETS);
-		TM_CHECK(dalloc(&r->d_scan, r->scan_words));
 	}
 	if (!keyrows(r->cfg) && !r->d_hits) {
 		uint64_t cap = r->cfg.hit_capacity ? r->cfg.hit_capacity : std::max<uint64_t>(1 << 20, (uint64_t)r->max_q * 64);
@@ -2246,9 +2020,8 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 		fill_u32(r->d_gbm, 0, (uint64_t)nq * r->kw, s);
 		fill_u32(r->d_qfull, 0, nq, s);
 	}
-	fill_u32(r->d_pcount, 0, r->P, s);
-	fill_u64(reinterpret_cast<uint64_t *>(r->d_cnt), 0, 8, s);
-	scan_u32_to_u64(r->d_pcount, r->d_pbase, r->P, r->d_scan, s);
+	hipLaunchKernelGGL(k_step_init, dim3(1), dim3(256), 0, s, r->d_pcount, r->P, r->d_cnt, r->d_qnext,
+					   2 * NQUEUE, (uint32_t *)nullptr);
 	if (r->cfg.schedule == TM_SCHED_PLAIN) {
 		if (!r->d_iota) {
 			TM_CHECK(dalloc(&r->d_iota, std::max<uint32_t>(r->max_q, 1)));
@@ -2275,26 +2048,28 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 		return run_plain(r, nq, r->d_iota, units);
 	}
 	// persistent: segment size from the whole submission's work
-	const uint32_t nqg = 64 * r->tiles;
-	const uint64_t resident = (uint64_t)dev().num_cu * r->wgs_per_cu;
+	const bool keys = keyrows(r->cfg);
+	const int mode = !keys ? MX_COUNT : r->kw > MX_LDS_KW || r->kw == 0 ? MX_KEYS : MX_KEYS_LDS;
+	mx_args a = matrix_args(r, mode);
+	const uint32_t nqg = mx_super(mode);
+	const uint64_t resident = a.resident;
 	uint64_t work = 0;   // tile x blocks
 	for (uint32_t i = 0; i < n; ++i) {
 		const uint32_t p = r->u_part[i], qn = r->u_off[i + 1] - r->u_off[i];
 		work += (uint64_t)((qn + nqg - 1) / nqg) * f->h_part_info[(size_t)p * 8 + 7];
 	}
 	uint32_t seg = r->cfg.chunk_blocks ? r->cfg.chunk_blocks
-									   : (uint32_t)std::max<uint64_t>(4, (work + 4 * resident - 1) / (4 * resident));
-	if (keyrows(r->cfg) && !r->lds_bm) seg = 0xFFFFFFFFu;   // rows in HBM: one workgroup per tile
+									   : (uint32_t)std::max<uint64_t>(64, (work + 4 * resident - 1) / (4 * resident));
 	std::vector<uint32_t> tab((size_t)std::max<uint32_t>(n, 1) * 8, 0), pre(n + 1, 0);
 	uint32_t max_nseg = 1;
 	uint64_t items = 0;
-	const bool tuned = !(keyrows(r->cfg) && !r->lds_bm) && !r->cfg.chunk_blocks;
+	const bool tuned = !r->cfg.chunk_blocks;
 	for (uint32_t i = 0; i < n; ++i) {
 		const uint32_t p = r->u_part[i], q0 = r->u_off[i], qn = r->u_off[i + 1] - q0;
 		const uint32_t blo = f->h_part_info[(size_t)p * 8 + 6], nb = f->h_part_info[(size_t)p * 8 + 7];
 		const uint32_t ntiles = (qn + nqg - 1) / nqg;
 		const uint32_t useg = tuned && r->seg_bucket[size_bucket(nb)] ? r->seg_bucket[size_bucket(nb)] : seg;
-		const uint32_t sb = std::max<uint32_t>(1, std::min<uint32_t>(useg, std::max<uint32_t>(nb, 1)));
+		const uint32_t sb = std::max<uint32_t>(1, std::min<uint32_t>(std::min(useg, MX_MAX_SEG), std::max<uint32_t>(nb, 1)));
 		const uint32_t nseg = nb ? (nb + sb - 1) / sb : 1;
 		uint32_t * t = &tab[(size_t)i * 8];
 		t[0] = p; t[1] = q0; t[2] = qn; t[3] = std::max<uint32_t>(ntiles, 1);
@@ -2310,40 +2085,24 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 	TM_CHECK(grow_u32(&r->d_xprefix, r->xprefix_cap, pre.size()));
 	TM_HIP(hipMemcpyAsync(r->d_xunits, tab.data(), tab.size() * 4, hipMemcpyHostToDevice, s));
 	TM_HIP(hipMemcpyAsync(r->d_xprefix, pre.data(), pre.size() * 4, hipMemcpyHostToDevice, s));
-	hipLaunchKernelGGL(k_init_queues, dim3(1), dim3(64), 0, s, items, r->d_qbeg, r->d_qnext);
-	mq_args a;
-	std::memset(&a, 0, sizeof(a));
-	a.f = f->view();
-	a.q = r->d_q;
 	a.nq = nq;
 	a.units = r->d_xunits;
 	a.uprefix = r->d_xprefix;
-	a.slot_epoch = f->slot_epoch;
-	a.epoch = r->epoch;
 	a.n_units = n;
-	a.ntiles = 1;
-	a.nseg = max_nseg;
-	a.seg_blocks = 1;
-	a.blk_lo = 0;
-	a.blk_hi = f->n_blocks;
-	a.log_unit = -1;
-	a.qnext = r->d_qnext;
-	a.qbeg = r->d_qbeg;
-	a.gbm = r->d_gbm;
-	a.qfull = r->d_qfull;
-	a.hits = r->d_hits;
-	a.hit_cap = r->hit_cap;
-	a.counters = r->d_cnt;
-	a.full_exit = keyrows(r->cfg) && r->lds_bm && r->kw > 0 && r->cfg.full_exit != 2;
-	a.last_mask = (f->n_keys & 31) ? (1u << (f->n_keys & 31)) - 1u : 0xFFFFFFFFu;
-	mq_fn fn = pick_match_q(mode_of(r->cfg), r->lds_bm, r->tiles, r->waves, r->variant);
 	const uint32_t grid = (uint32_t)std::min<uint64_t>(resident, std::max<uint64_t>(items, 1));
+	if (!keys) {
+		TM_CHECK(grow_u32(&r->d_hcnt, r->hcnt_cap, (uint64_t)max_nseg * nq));
+		fill_u32(r->d_hcnt, 0, (uint64_t)max_nseg * nq, s);   // units have different numbers of segments
+		TM_CHECK(enqueue_values(r, a, max_nseg, grid, true));
+		TM_HIP(hipStreamSynchronize(s));   // tab and pre are pageable host memory
+		return TM_OK;
+	}
 	TM_HIP(hipEventRecord(r->em0, s));
-	hipLaunchKernelGGL(fn, dim3(grid), dim3(r->waves * 64), r->stage_lds, s, a);
+	r->n_wgstat = grid;
+	mx_launch(a, mode, grid, s);
 	TM_HIP(hipGetLastError());
 	TM_HIP(hipEventRecord(r->em1, s));
 	TM_HIP(hipStreamSynchronize(s));   // tab and pre are pageable host memory
-	fill_u64(r->d_iprefix + r->P, items, 1, s);
 	enqueue_finalize(r, nq);
 	return TM_OK;
 }
@@ -2643,6 +2402,7 @@ int submit_common(tm_ring * r, uint32_t nq) {
 	r->st = tm_status();
 	r->last_nq = nq;
 	r->retries = 0;
+	r->hits_grown = false;
 	r->epoch = r->fib->epoch;   // the inserts this submission sees
 	TM_CHECK(sync_fib(r));
 	TM_CHECK(ensure_capacity(r));
@@ -2657,6 +2417,15 @@ int submit_common(tm_ring * r, uint32_t nq) {
 		TM_CHECK(ensure_pack(r, std::max<uint64_t>(nq, 1)));
 	}
 	if (!r->units_mode) TM_CHECK(price_submission(r, r->run_nq));
+	if (!r->units_mode && !keyrows(r->cfg) && r->cfg.schedule == TM_SCHED_PERSISTENT && !r->cfg.log_units) {
+		const mx_args a = matrix_args(r, MX_COUNT);
+		const mx_shape h = hits_shape(r, r->run_nq, a.resident);
+		const uint64_t need = (uint64_t)h.nseg * r->run_nq;
+		if (need > r->hcnt_cap) {
+			drop_graph(r);
+			TM_CHECK(grow_u32(&r->d_hcnt, r->hcnt_cap, need));
+		}
+	}
 	int rc = enqueue_step(r, true);
 	if (rc != TM_OK) return rc;
 	r->pending = true;
@@ -2703,7 +2472,8 @@ int tm_ring_create(tm_fib * fib, uint32_t max_queries, const tm_match_config * c
 	}
 	rc = dalloc(&r->d_q, (size_t)max_queries * 8);
 	if (rc == TM_OK) rc = dalloc(&r->d_step, 2);
-	if (rc == TM_OK) rc = dalloc(&r->d_qinv, (size_t)max_queries * 8);
+	if (rc == TM_OK) rc = dalloc(&r->d_qact, (size_t)max_queries * 8);
+	if (rc == TM_OK) rc = dalloc(&r->d_wgstat, (size_t)MX_MAX_GROUPS * 4);
 	if (rc == TM_OK) rc = ensure_capacity(r);
 	if (rc != TM_OK) { r->release(); delete r; return rc; }
 	*out = r;
@@ -2847,7 +2617,9 @@ int tm_wait(tm_ring * r, tm_status * st) {
 				uint64_t cap = slots + slots / 4 + 1024;
 				TM_CHECK(dalloc(&r->d_hits, cap));
 				r->hit_cap = cap;
-				again = true;
+				// a matrix step keeps no hit list: its values are whole
+				if (r->n_wgstat) r->hits_grown = true;
+				else again = true;
 			}
 			if (results > r->val_cap) {
 				TM_CHECK(grow_u32(&r->d_vals, r->val_cap, results + results / 4 + 1024));
@@ -2887,7 +2659,7 @@ int tm_wait(tm_ring * r, tm_status * st) {
 		r->st.n_results = r->h_stat[3];
 		if (r->cfg.schedule == TM_SCHED_PERSISTENT) r->st.n_items = (uint32_t)r->h_stat[4];
 		r->st.hit_capacity = r->hit_cap;
-		r->st.overflow = r->retries > 0;
+		r->st.overflow = r->retries > 0 || r->hits_grown;
 		r->st.error = TM_OK;
 		r->st.device_ms = dms;
 		r->st.match_ms = mms;
@@ -3182,11 +2954,11 @@ constexpr size_t SC_STAT = SC_CNT + sc_round(8 * 8);                    // u64 [
 constexpr size_t SC_NACT = SC_STAT + sc_round(8 * 8);                   // u32 [4]
 constexpr size_t SC_SCAN = SC_NACT + sc_round(4 * 4);                   // u64 [scan words of P]
 constexpr size_t SC_SCAN_WORDS = (SC_P + 255) / 256 + 2;                // >= scan_tmp_words(P)
-constexpr size_t SC_AHIST = SC_SCAN + sc_round(SC_SCAN_WORDS * 8);      // u32 [2 x ACT_BUCKETS]
-constexpr size_t SC_ABASE = SC_AHIST + sc_round(2 * ACT_BUCKETS * 4);    // u64 [ACT_BUCKETS + 1]
-constexpr size_t SC_QFULL = SC_ABASE + sc_round((ACT_BUCKETS + 1) * 8);  // u32 [Q]
+constexpr size_t SC_QFULL = SC_SCAN + sc_round(SC_SCAN_WORDS * 8);      // u32 [Q]
 constexpr size_t SC_ACTIVE = SC_QFULL + sc_round(SC_Q * 4);             // u32 [Q]
-constexpr size_t SC_BYTES = SC_ACTIVE + sc_round(SC_Q * 4);
+constexpr size_t SC_QACT = SC_ACTIVE + sc_round(SC_Q * 4);               // u32 [Q x 8]
+constexpr size_t SC_WGSTAT = SC_QACT + sc_round(SC_Q * 32);              // u64 [MX_MAX_GROUPS x 4]
+constexpr size_t SC_BYTES = SC_WGSTAT + sc_round((size_t)MX_MAX_GROUPS * 32);
 
 static __device__ __align__(256) unsigned char scratch[SC_BYTES];
 
@@ -3236,7 +3008,7 @@ int tm_match_rows_static(tm_fib * fib, const uint32_t * dev_queries, uint32_t nq
 	r.P = fib->n_parts;
 	r.kw = (fib->n_keys + 31) / 32;
 	TM_CHECK(resolve_params(&r));
-	if (scan_tmp_words(r.P) > SC_SCAN_WORDS || scan_tmp_words(ACT_BUCKETS) > SC_SCAN_WORDS)
+	if (scan_tmp_words(r.P) > SC_SCAN_WORDS)
 		return set_error(TM_ERR_STATE, "scan scratch too small");
 	r.no_weights = true;
 	r.s = static_cast<hipStream_t>(stream);
@@ -3251,10 +3023,10 @@ int tm_match_rows_static(tm_fib * fib, const uint32_t * dev_queries, uint32_t nq
 	r.d_stat = reinterpret_cast<uint64_t *>(sc + SC_STAT);
 	r.d_nact = reinterpret_cast<uint32_t *>(sc + SC_NACT);
 	r.d_scan = reinterpret_cast<uint64_t *>(sc + SC_SCAN);
-	r.d_ahist = reinterpret_cast<uint32_t *>(sc + SC_AHIST);
-	r.d_abase = reinterpret_cast<uint64_t *>(sc + SC_ABASE);
 	r.d_qfull = reinterpret_cast<uint32_t *>(sc + SC_QFULL);
 	r.d_active = reinterpret_cast<uint32_t *>(sc + SC_ACTIVE);
+	r.d_qact = reinterpret_cast<uint32_t *>(sc + SC_QACT);
+	r.d_wgstat = reinterpret_cast<uint64_t *>(sc + SC_WGSTAT);
 	r.epoch = fib->epoch;   // the inserts this call sees
 	fib->in_flight.fetch_add(1);
 	int rc = enqueue_persistent(&r, nq, false);

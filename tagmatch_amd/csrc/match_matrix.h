@@ -1,0 +1,123 @@
+// The matrix-core match kernel's launch interface.  Internal to
+// libtagmatch_amd.so.
+#pragma once
+
+#include "fib.h"
+
+namespace tmx {
+
+// What a launch does with its hits:
+//   MX_KEYS      their keys into rows in HBM (which hold most keys already);
+//   MX_KEYS_LDS  the same through rows in local memory (rows that start empty);
+//   MX_COUNT, MX_COUNT_KEYS   values per query and segment (filter ids; keys);
+//   MX_WRITE, MX_WRITE_KEYS   the values, behind those of earlier segments.
+enum mx_mode { MX_KEYS, MX_KEYS_LDS, MX_COUNT, MX_COUNT_KEYS, MX_WRITE, MX_WRITE_KEYS, MX_MODES };
+
+constexpr uint32_t MX_LDS_KW = 64;      // MX_KEYS_LDS: words of a row, at most
+constexpr uint32_t MX_QUEUES = 8;       // work queues, one per XCD
+constexpr uint32_t MX_QPAD = 32;        // queue cursors 256 B apart
+constexpr uint32_t MX_MAX_SEG = 16384;  // blocks per work item, at most
+constexpr uint32_t MX_MAX_GROUPS = 2048;   // workgroups of a launch, at most
+constexpr uint32_t MX_VISITS = 1024;    // blocks of a pass, at most
+
+constexpr int MX_WAVES = 8;             // waves per workgroup
+
+// Queries per work item, at most, and the words of the candidate masks (an
+// odd number of words per block, two for 64 queries and one).  Two
+// workgroups of 8 waves share a CU's 160 KB of local memory; within that,
+// more queries per item mean more candidates for each block whose filters
+// are loaded and spread.  Rows in local memory (48 KB for 192 queries at
+// 2048 keys) leave room for fewer: match times of the uneven units (541k
+// queries) 4.1 ms with 192, 4.7 with 128, 4.2 with 448 and one workgroup of
+// 16 waves per CU.
+__host__ __device__ constexpr uint32_t mx_super(int mode) {
+	return mode == MX_KEYS ? 2048u : mode == MX_KEYS_LDS ? 192u : 1536u;
+}
+__host__ __device__ constexpr uint32_t mx_mask_words(int mode) {
+	return mode == MX_KEYS ? 64u * 65u : mode == MX_KEYS_LDS ? 128u * 7u : 64u * 49u;
+}
+__host__ __device__ constexpr uint32_t mx_visits(int mode) { return mode == MX_KEYS_LDS ? 128u : MX_VISITS; }
+
+// Work items of a launch over nq queries and nblk blocks: item = segment *
+// nsuper + super, segments of seg blocks, supers of sq queries.  Few queries:
+// one item per workgroup.  Otherwise four per workgroup or more, so that
+// uneven items even out, as long as a segment has 64 blocks.  seg_min: least
+// blocks per segment (a bound on the segments), 0: none.
+struct mx_shape {
+	uint32_t sq, nsuper, seg, nseg;
+};
+__host__ __device__ inline mx_shape mx_shape_of(int mode, uint32_t nq, uint32_t nblk, uint32_t resident,
+												uint32_t seg_fixed, uint32_t seg_min) {
+	uint32_t sq = mx_super(mode);
+	if (nq < sq) sq = nq > 64 ? (nq + 63) & ~63u : 64u;
+	// few blocks: fewer queries per item (20k queries, 8.8k blocks: 0.70
+	// instead of 1.30 ms)
+	while (sq > 256 && (uint64_t)((nq + sq - 1) / sq) * ((nblk + 63) / 64) < 4ull * resident) sq = (sq / 2 + 63) & ~63u;
+	const uint32_t nsuper = (nq + sq - 1) / sq;
+	const uint32_t fit = mx_mask_words(mode) / (2 * (sq / 64) + 1);
+	const uint32_t most = (fit < mx_visits(mode) ? fit : mx_visits(mode)) & ~31u;   // 64 or more
+	uint32_t seg = most;
+	if ((uint64_t)nsuper * ((nblk + 63) / 64) <= 4ull * resident) {
+		const uint64_t per = ((uint64_t)nblk * nsuper + resident - 1) / resident;
+		const uint64_t up = (per + 31) & ~31ull;
+		seg = up < 32 ? 32u : up < MX_VISITS ? (uint32_t)up : MX_VISITS;
+	} else {
+		while (seg > 64 && (uint64_t)nsuper * ((nblk + seg - 1) / seg) < 4ull * resident) {
+			seg = (seg / 2) & ~31u;
+			if (seg < 64) seg = 64;
+		}
+	}
+	if (seg < seg_min) seg = seg_min;
+	if (seg_fixed) seg = seg_fixed;
+	if (seg > MX_MAX_SEG) seg = MX_MAX_SEG;
+	mx_shape h;
+	h.sq = sq;
+	h.nsuper = nsuper;
+	h.seg = seg;
+	h.nseg = (nblk + seg - 1) / seg;
+	return h;
+}
+
+struct mx_args {
+	dev_fib_view f;
+	const uint32_t * __restrict__ q;       // words of each local query, 8 apart
+	const uint32_t * __restrict__ qmap;    // query (result row) of each local query (NULL: identity)
+	uint32_t nq;                           // local queries
+	const uint32_t * __restrict__ nq_dev;  // device count of local queries (NULL: nq)
+	uint32_t nblk;                         // blocks of the table
+	uint32_t seg_fixed;                    // configured blocks per item (0: by the launch's size)
+	uint32_t seg_min;                      // least blocks per item (0: any)
+	uint32_t resident;                     // workgroups of the launch
+	const uint32_t * __restrict__ units;   // explicit units, 8 words each: partition, first query,
+	                                       // queries, supers, segments, blocks per segment, first
+	                                       // block, end block
+	const uint32_t * __restrict__ uprefix; // n_units + 1: first work item of each unit
+	uint32_t n_units;
+	unsigned long long * qnext;            // MX_QUEUES cursors, MX_QPAD apart, zero at the start
+	uint32_t * gbm;                        // key rows
+	const uint32_t * __restrict__ qfull;   // flags of rows that hold every key (NULL: none known)
+	const uint32_t * __restrict__ rich_bm; // key bitmaps of the rich filters
+	uint32_t n_rich;
+	uint32_t rich_done;                    // the rows already hold the rich filters' keys
+	uint32_t * hcnt;                       // MX_COUNT..: values of each query, one row of nq per segment;
+	                                       // MX_WRITE..: values of earlier segments
+	const uint64_t * __restrict__ off;     // MX_WRITE..: first value of each query
+	uint32_t * vals;
+	uint64_t vcap;
+	uint64_t * wg_stats;                   // per workgroup: hits, block visits, subset tests, tests
+	                                       // with hits
+	uint64_t * n_items;                    // receives the launch's work items
+	const uint32_t * __restrict__ slot_epoch;
+	uint32_t epoch;
+	const uint32_t * __restrict__ step_vals;   // replayed steps: [0] epoch, [1] valid overflow words
+};
+
+// hcnt's rows (segments) to each query's values of earlier segments, and the
+// queries' totals.
+void mx_prefix(uint32_t * hcnt, uint32_t rows, uint32_t nq, uint32_t * total, hipStream_t s);
+
+// Workgroups that fit the GPU at once.
+uint32_t mx_resident(int mode);
+void mx_launch(const mx_args & a, int mode, uint32_t grid, hipStream_t s);
+
+} // namespace tmx
