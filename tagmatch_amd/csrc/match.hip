@@ -1584,7 +1584,12 @@ int enqueue_values(tm_ring * r, mx_args a, uint32_t rows, uint32_t grid, bool ev
 	a.off = r->d_off;
 	a.vals = r->d_vals;
 	a.vcap = r->val_cap;
+	// (the hit list of the other schedules is free here)
+	a.lists = reinterpret_cast<uint4 *>(r->d_hits);
+	a.lists_cap = r->hit_cap / 2;
+	a.n_lists = r->d_cnt + 5;
 	mx_launch(a, ids ? MX_WRITE : MX_WRITE_KEYS, grid, s);
+	if (!ids) mx_write_lists(a, s);
 	TM_HIP(hipGetLastError());
 	if (events) TM_HIP(hipEventRecord(r->em1, s));
 	r->step_weighted = false;
@@ -2618,8 +2623,12 @@ int tm_wait(tm_ring * r, tm_status * st) {
 				TM_CHECK(dalloc(&r->d_hits, cap));
 				r->hit_cap = cap;
 				// a matrix step keeps no hit list: its values are whole
-				if (r->n_wgstat) r->hits_grown = true;
-				else again = true;
+				if (r->n_wgstat) {
+					r->hits_grown = true;
+					drop_graph(r);   // holds the old buffer
+				} else {
+					again = true;
+				}
 			}
 			if (results > r->val_cap) {
 				TM_CHECK(grow_u32(&r->d_vals, r->val_cap, results + results / 4 + 1024));

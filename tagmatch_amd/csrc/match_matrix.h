@@ -18,6 +18,7 @@ constexpr uint32_t MX_QUEUES = 8;       // work queues, one per XCD
 constexpr uint32_t MX_QPAD = 32;        // queue cursors 256 B apart
 constexpr uint32_t MX_MAX_SEG = 16384;  // blocks per work item, at most
 constexpr uint32_t MX_MAX_GROUPS = 2048;   // workgroups of a launch, at most
+constexpr uint32_t MX_LONG_LIST = 64;  // MX_WRITE_KEYS: keys of a list that is written apart, at least
 constexpr uint32_t MX_VISITS = 1024;    // blocks of a pass, at most
 
 constexpr int MX_WAVES = 8;             // waves per workgroup
@@ -104,6 +105,10 @@ struct mx_args {
 	const uint64_t * __restrict__ off;     // MX_WRITE..: first value of each query
 	uint32_t * vals;
 	uint64_t vcap;
+	uint4 * lists;                         // MX_WRITE_KEYS: long key lists to write (first value, 64
+	                                       // bits; list; keys), lists_cap of them at most
+	uint64_t lists_cap;
+	unsigned long long * n_lists;          // their number, zero at the start
 	uint64_t * wg_stats;                   // per workgroup: hits, block visits, subset tests, tests
 	                                       // with hits
 	uint64_t * n_items;                    // receives the launch's work items
@@ -115,6 +120,9 @@ struct mx_args {
 // hcnt's rows (segments) to each query's values of earlier segments, and the
 // queries' totals.
 void mx_prefix(uint32_t * hcnt, uint32_t rows, uint32_t nq, uint32_t * total, hipStream_t s);
+
+// MX_WRITE_KEYS: the lists it recorded.
+void mx_write_lists(const mx_args & a, hipStream_t s);
 
 // Workgroups that fit the GPU at once.
 uint32_t mx_resident(int mode);

@@ -235,6 +235,18 @@ k_match_x(mx_args a) {
 							const uint32_t id = (uint32_t)(kv >> (16 * x)) & 0xFFFFu;
 							if (at0 + x < a.vcap) a.vals[at0 + x] = a.f.key_dict[id < a.f.n_keys ? id : 0u];
 						}
+					// long lists are left to k_write_lists: one wave would be
+					// busy with its own for long after the others
+					const uint64_t lb = __ballot(cnt >= MX_LONG_LIST);
+					if (lb) {
+						uint64_t r = 0;
+						if (lane == 0) r = atomicAdd(a.n_lists, (unsigned long long)__popcll(lb));
+						r = (uint64_t)__shfl((unsigned long long)r, 0) + mbcnt64(lb);
+						if (cnt >= MX_LONG_LIST && r < a.lists_cap) {
+							a.lists[r] = make_uint4((uint32_t)at0, (uint32_t)(at0 >> 32), off, cnt);
+							cnt = 0;
+						}
+					}
 				}
 				uint32_t * row = MODE == MX_KEYS_LDS ? s_rows + qi * kw : a.gbm + (size_t)gq * kw;
 				bool lst = false;
@@ -598,6 +610,33 @@ k_prefix(uint32_t * __restrict__ hcnt, uint32_t rows, uint32_t nq, uint32_t * __
 	}
 }
 
+// The recorded lists, a wave for each in turn, eight ids per lane in flight.
+__global__ void __launch_bounds__(256)
+k_write_lists(const uint4 * __restrict__ lists, const unsigned long long * __restrict__ n_lists, uint64_t cap,
+			  dev_fib_view f, uint32_t * __restrict__ vals, uint64_t vcap) {
+	const uint32_t lane = threadIdx.x & 63;
+	const uint64_t n = min((uint64_t)*n_lists, cap);
+	for (uint64_t r = ((uint64_t)blockIdx.x * 256 + threadIdx.x) >> 6; r < n; r += (uint64_t)gridDim.x * 4) {
+		const uint4 l = lists[r];
+		const uint64_t at = (uint64_t)l.x | ((uint64_t)l.y << 32);
+		for (uint32_t i0 = 0; i0 < l.w; i0 += 512) {
+			uint32_t id[8];
+#pragma unroll
+			for (uint32_t k = 0; k < 8; ++k) {
+				const uint32_t i = i0 + k * 64 + lane;
+				id[k] = i < l.w ? f.ovf[l.z + 1 + i] : 0u;
+			}
+#pragma unroll
+			for (uint32_t k = 0; k < 8; ++k) id[k] = f.key_dict[id[k] < f.n_keys ? id[k] : 0u];
+#pragma unroll
+			for (uint32_t k = 0; k < 8; ++k) {
+				const uint32_t i = i0 + k * 64 + lane;
+				if (i < l.w && at + i < vcap) vals[at + i] = id[k];
+			}
+		}
+	}
+}
+
 using mx_fn = void (*)(mx_args);
 mx_fn kernel_of(int mode) {
 	switch (mode) {
@@ -614,6 +653,10 @@ mx_fn kernel_of(int mode) {
 
 void mx_prefix(uint32_t * hcnt, uint32_t rows, uint32_t nq, uint32_t * total, hipStream_t s) {
 	if (nq) hipLaunchKernelGGL(k_prefix, dim3((nq + 63) / 64), dim3(1024), 0, s, hcnt, rows, nq, total);
+}
+
+void mx_write_lists(const mx_args & a, hipStream_t s) {
+	hipLaunchKernelGGL(k_write_lists, dim3(2048), dim3(256), 0, s, a.lists, a.n_lists, a.lists_cap, a.f, a.vals, a.vcap);
 }
 
 uint32_t mx_resident(int mode) {

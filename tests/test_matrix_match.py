@@ -15,15 +15,16 @@ pytestmark = pytest.mark.gpu
 
 def table(n, n_keys, long_lists, seed):
     """n canonical filters, every other one with 1-4 keys, `long_lists` of
-    them with 33-60; the empty and the full filter among them."""
+    them with 33-130; the empty and the full filter among them."""
     rng = np.random.default_rng(seed)
     g = tm.Generator(seed=0x5EED + seed)
     w, _, _ = g.filters(n)
     w[0], w[1] = 0, 0xFFFFFFFF
     w = np.unique(w, axis=0)
     cnt = rng.integers(1, 5, len(w))
-    cnt[rng.choice(len(w), min(long_lists, len(w)), replace=False)] = rng.integers(33, 61, min(long_lists, len(w)))
+    cnt[rng.choice(len(w), min(long_lists, len(w)), replace=False)] = rng.integers(33, 131, min(long_lists, len(w)))
     ko = np.zeros(len(w) + 1, np.uint64)
+    cnt = np.minimum(cnt, n_keys)
     np.cumsum(cnt, out=ko[1:])
     k = np.concatenate([rng.choice(n_keys, c, replace=False) for c in cnt]).astype(np.uint32) * 5 + 1
     return tm.canonicalize(w, ko, k)
