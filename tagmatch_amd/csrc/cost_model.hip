@@ -30,6 +30,8 @@ struct tm_mlp {
 	uint32_t cap = 0;
 	float * d_x = nullptr, * d_t = nullptr, * d_h1 = nullptr, * d_h2 = nullptr, * d_y = nullptr;
 	float * d_dy = nullptr, * d_dh1 = nullptr, * d_dh2 = nullptr, * d_loss = nullptr;
+	float * d_part = nullptr;   // gradient vectors of the row chunks
+	uint64_t part_cap = 0;
 	hipStream_t s = nullptr;
 
 	size_t o_w1() const { return 0; }
@@ -46,7 +48,8 @@ struct tm_mlp {
 	}
 	void release() {
 		free_batch();
-		dfree(d_p); dfree(d_g); dfree(d_m); dfree(d_v); dfree(d_loss);
+		dfree(d_p); dfree(d_g); dfree(d_m); dfree(d_v); dfree(d_loss); dfree(d_part);
+		part_cap = 0;
 		if (s) (void)hipStreamDestroy(s);
 		s = nullptr;
 	}
@@ -54,17 +57,81 @@ struct tm_mlp {
 
 namespace {
 
-// Y[n][b] = act(X[n][a] W[a][b] + bias[b]); one thread per output element.
+// Y[n][m] = X[n][K] B[K][m], a 64 x 64 tile per workgroup and 4 x 4 per
+// thread, operands in local memory 16 of K at a time; each output adds its
+// products in ascending order of K.
+//   BACK false: B = W[K][m]; sums start at bias[c]; ReLU if relu
+//   BACK true:  B = W[m][K] transposed; outputs whose H is not positive are 0
+// Bound by its operands' bytes at the cost model's sizes: the 65536 x 64 x 64
+// backward product takes 21 us, one thread per output with W's rows read a
+// line per lane 283 us.
+template <bool BACK>
 __global__ void __launch_bounds__(256)
-k_dense(const float * __restrict__ X, const float * __restrict__ W, const float * __restrict__ bias,
-		float * __restrict__ Y, uint32_t n, uint32_t a, uint32_t b, int relu) {
-	const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-	if (i >= (uint64_t)n * b) return;
-	const uint32_t r = (uint32_t)(i / b), c = (uint32_t)(i % b);
-	float acc = bias[c];
-	const float * x = X + (size_t)r * a;
-	for (uint32_t k = 0; k < a; ++k) acc = fmaf(x[k], W[(size_t)k * b + c], acc);
-	Y[i] = (relu && acc < 0.f) ? 0.f : acc;
+k_layer(const float * __restrict__ X, const float * __restrict__ W, const float * __restrict__ bias,
+		const float * __restrict__ H, float * __restrict__ Y, uint32_t n, uint32_t K, uint32_t m, int relu) {
+	__shared__ float s_x[16][68], s_w[16][68];
+	const uint32_t tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+	const uint32_t r0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
+	float acc[4][4];
+#pragma unroll
+	for (int j = 0; j < 4; ++j) {
+		const uint32_t c = c0 + tx * 4 + j;
+		const float b = !BACK && c < m ? bias[c] : 0.f;
+#pragma unroll
+		for (int i = 0; i < 4; ++i) acc[i][j] = b;
+	}
+	float lx[4], lw[4];   // the next 16 of K, loaded while these are multiplied
+	auto load = [&](uint32_t k0) {
+#pragma unroll
+		for (int e = 0; e < 4; ++e) {
+			const uint32_t x = tid + e * 256, k = x & 15, r = x >> 4;   // 16 of K per row
+			lx[e] = r0 + r < n && k0 + k < K ? X[(size_t)(r0 + r) * K + k0 + k] : 0.f;
+			if (BACK) {
+				lw[e] = c0 + r < m && k0 + k < K ? W[(size_t)(c0 + r) * K + k0 + k] : 0.f;
+			} else {
+				const uint32_t c = x & 63, kk = x >> 6;
+				lw[e] = c0 + c < m && k0 + kk < K ? W[(size_t)(k0 + kk) * m + c0 + c] : 0.f;
+			}
+		}
+	};
+	load(0);
+	for (uint32_t k0 = 0; k0 < K; k0 += 16) {
+#pragma unroll
+		for (int e = 0; e < 4; ++e) {
+			const uint32_t x = tid + e * 256;
+			s_x[x & 15][x >> 4] = lx[e];
+			if (BACK) s_w[x & 15][x >> 4] = lw[e];
+			else s_w[x >> 6][x & 63] = lw[e];
+		}
+		__syncthreads();
+		if (k0 + 16 < K) load(k0 + 16);
+#pragma unroll
+		for (uint32_t k = 0; k < 16; ++k) {
+			const float4 x = *reinterpret_cast<const float4 *>(&s_x[k][ty * 4]);
+			const float4 w = *reinterpret_cast<const float4 *>(&s_w[k][tx * 4]);
+			const float xs[4] = {x.x, x.y, x.z, x.w}, ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+			for (int i = 0; i < 4; ++i)
+#pragma unroll
+				for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(xs[i], ws[j], acc[i][j]);
+		}
+		__syncthreads();
+	}
+#pragma unroll
+	for (int i = 0; i < 4; ++i) {
+		const uint32_t r = r0 + ty * 4 + i;
+		if (r >= n) break;
+#pragma unroll
+		for (int j = 0; j < 4; ++j) {
+			const uint32_t c = c0 + tx * 4 + j;
+			if (c >= m) break;
+			const size_t at = (size_t)r * m + c;
+			float v = acc[i][j];
+			if (BACK) v = H[at] <= 0.f ? 0.f : v;
+			else if (relu && v < 0.f) v = 0.f;
+			Y[at] = v;
+		}
+	}
 }
 
 // dY = 2 (Y - T) / (n m); loss += sum (Y - T)^2 / (n m)
@@ -88,39 +155,83 @@ k_mse(const float * __restrict__ Y, const float * __restrict__ T, float * __rest
 	if (threadIdx.x == 0) atomicAdd(loss, s[0]);
 }
 
-// dH[n][a] = (dY[n][b] W[a][b]^T) * (H > 0)
+// dW[a][b] = A^T dY, db[b] = sum_rows dY over the rows of one chunk (rows
+// blockIdx.z * per ...), into that chunk's gradient vector `part` + chunk *
+// stride: a 64 x 64 tile of dW per workgroup, 4 x 4 per thread, 16 rows of
+// the operands in local memory at a time; the first tile of k sums db.
+// k_sum_chunks adds the chunks: one thread's walk over all 65536 rows left
+// most of the chip idle (16 ms for the 64 x 64 layer, 20 us in 512 chunks of
+// these tiles, most of it load latency), and a sum of chunk sums rounds less than one running sum.
 __global__ void __launch_bounds__(256)
-k_back(const float * __restrict__ dY, const float * __restrict__ W, const float * __restrict__ H,
-	   float * __restrict__ dH, uint32_t n, uint32_t a, uint32_t b) {
-	const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-	if (i >= (uint64_t)n * a) return;
-	const uint32_t r = (uint32_t)(i / a), k = (uint32_t)(i % a);
-	if (H[i] <= 0.f) {
-		dH[i] = 0.f;
-		return;
+k_wgrad(const float * __restrict__ A, const float * __restrict__ dY, float * __restrict__ part, uint64_t stride,
+		size_t o_w, size_t o_b, uint32_t n, uint32_t a, uint32_t b, uint32_t per) {
+	__shared__ float s_a[16][68], s_d[16][68];
+	const uint32_t tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+	const uint32_t k0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
+	const uint32_t r0 = blockIdx.z * per, r1 = min(n, r0 + per);
+	float * out = part + (size_t)blockIdx.z * stride;
+	float acc[4][4] = {}, db[4] = {};
+	float la[4], ld[4];   // the next 16 rows, loaded while these are multiplied
+	auto load = [&](uint32_t rb) {
+#pragma unroll
+		for (int e = 0; e < 4; ++e) {
+			const uint32_t r = rb + ((tid + e * 256) >> 6), c = tid & 63;
+			la[e] = r < r1 && k0 + c < a ? A[(size_t)r * a + k0 + c] : 0.f;
+			ld[e] = r < r1 && c0 + c < b ? dY[(size_t)r * b + c0 + c] : 0.f;
+		}
+	};
+	load(r0);
+	for (uint32_t rb = r0; rb < r1; rb += 16) {
+#pragma unroll
+		for (int e = 0; e < 4; ++e) {
+			const uint32_t r = (tid + e * 256) >> 6, c = tid & 63;
+			s_a[r][c] = la[e];
+			s_d[r][c] = ld[e];
+		}
+		__syncthreads();
+		if (rb + 16 < r1) load(rb + 16);
+#pragma unroll
+		for (uint32_t r = 0; r < 16; ++r) {
+			const float4 x = *reinterpret_cast<const float4 *>(&s_a[r][ty * 4]);
+			const float4 d = *reinterpret_cast<const float4 *>(&s_d[r][tx * 4]);
+			const float xs[4] = {x.x, x.y, x.z, x.w}, ds[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+			for (int j = 0; j < 4; ++j) {
+				db[j] += ds[j];
+#pragma unroll
+				for (int i = 0; i < 4; ++i) acc[i][j] = fmaf(xs[i], ds[j], acc[i][j]);
+			}
+		}
+		__syncthreads();
 	}
-	float acc = 0.f;
-	const float * dy = dY + (size_t)r * b;
-	for (uint32_t c = 0; c < b; ++c) acc = fmaf(dy[c], W[(size_t)k * b + c], acc);
-	dH[i] = acc;
+#pragma unroll
+	for (int j = 0; j < 4; ++j) {
+		const uint32_t c = c0 + tx * 4 + j;
+		if (c >= b) break;
+		if (k0 == 0 && ty == 0) out[o_b + c] = db[j];
+#pragma unroll
+		for (int i = 0; i < 4; ++i) {
+			const uint32_t k = k0 + ty * 4 + i;
+			if (k < a) out[o_w + (size_t)k * b + c] = acc[i][j];
+		}
+	}
 }
 
-// dW[a][b] = A^T dY, db[b] = sum_rows dY; one thread per (k, c), k == a is
-// the bias row.
+// g = sum of the chunks' gradient vectors; a workgroup takes 64 parameters,
+// its four waves a quarter of the chunks each.
 __global__ void __launch_bounds__(256)
-k_wgrad(const float * __restrict__ A, const float * __restrict__ dY, float * __restrict__ dW,
-		float * __restrict__ db, uint32_t n, uint32_t a, uint32_t b) {
-	const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-	if (i >= (a + 1) * b) return;
-	const uint32_t k = i / b, c = i % b;
+k_sum_chunks(const float * __restrict__ part, uint64_t np, uint32_t chunks, float * __restrict__ g) {
+	__shared__ float s[4][64];
+	const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	const uint64_t i = (uint64_t)blockIdx.x * 64 + lane;
 	float acc = 0.f;
-	if (k < a) {
-		for (uint32_t r = 0; r < n; ++r) acc = fmaf(A[(size_t)r * a + k], dY[(size_t)r * b + c], acc);
-		dW[(size_t)k * b + c] = acc;
-	} else {
-		for (uint32_t r = 0; r < n; ++r) acc += dY[(size_t)r * b + c];
-		db[c] = acc;
+	if (i < np) {
+#pragma unroll 8
+		for (uint32_t c = chunks * w / 4; c < chunks * (w + 1) / 4; ++c) acc += part[(size_t)c * np + i];
 	}
+	s[w][lane] = acc;
+	__syncthreads();
+	if (w == 0 && i < np) g[i] = (s[0][lane] + s[1][lane]) + (s[2][lane] + s[3][lane]);
 }
 
 __global__ void __launch_bounds__(256)
@@ -162,34 +273,61 @@ int ensure_batch(tm_mlp * m, uint32_t n) {
 	return TM_OK;
 }
 
+dim3 layer_grid(uint32_t n, uint32_t m) { return dim3((n + 63) / 64, (m + 63) / 64); }
+
 // forward on the n rows already in d_x
 void forward(tm_mlp * m, uint32_t n) {
 	const float * P = m->d_p;
-	hipLaunchKernelGGL(k_dense, dim3(grid((uint64_t)n * m->h)), dim3(256), 0, m->s, m->d_x, P + m->o_w1(),
-					   P + m->o_b1(), m->d_h1, n, m->n_in, m->h, 1);
-	hipLaunchKernelGGL(k_dense, dim3(grid((uint64_t)n * m->h)), dim3(256), 0, m->s, m->d_h1, P + m->o_w2(),
-					   P + m->o_b2(), m->d_h2, n, m->h, m->h, 1);
-	hipLaunchKernelGGL(k_dense, dim3(grid((uint64_t)n * m->n_out)), dim3(256), 0, m->s, m->d_h2, P + m->o_w3(),
-					   P + m->o_b3(), m->d_y, n, m->h, m->n_out, 0);
+	const float * none = nullptr;
+	hipLaunchKernelGGL(k_layer<false>, layer_grid(n, m->h), dim3(256), 0, m->s, m->d_x, P + m->o_w1(), P + m->o_b1(),
+					   none, m->d_h1, n, m->n_in, m->h, 1);
+	hipLaunchKernelGGL(k_layer<false>, layer_grid(n, m->h), dim3(256), 0, m->s, m->d_h1, P + m->o_w2(), P + m->o_b2(),
+					   none, m->d_h2, n, m->h, m->h, 1);
+	hipLaunchKernelGGL(k_layer<false>, layer_grid(n, m->n_out), dim3(256), 0, m->s, m->d_h2, P + m->o_w3(),
+					   P + m->o_b3(), none, m->d_y, n, m->h, m->n_out, 0);
+}
+
+// Row chunks of the weight gradients: up to 512 of at least 32 rows, as far
+// as their gradient vectors fit 64 MB.
+uint32_t grad_rows(const tm_mlp * m, uint32_t n) {
+	const uint64_t most = std::max<uint64_t>(1, std::min<uint64_t>(512, (16ull << 20) / m->n_params));
+	return (uint32_t)std::max<uint64_t>(32, (n + most - 1) / most);
+}
+
+int ensure_chunks(tm_mlp * m, uint32_t n) {
+	const uint32_t per = grad_rows(m, n);
+	const uint64_t need = (uint64_t)((n + per - 1) / per) * m->n_params;
+	if (need <= m->part_cap) return TM_OK;
+	dfree(m->d_part);
+	m->part_cap = 0;
+	TM_CHECK(dalloc(&m->d_part, need));
+	m->part_cap = need;
+	return TM_OK;
 }
 
 // loss and gradients of the n rows in d_x / d_t; loss left in d_loss
 void backward(tm_mlp * m, uint32_t n) {
 	const float * P = m->d_p;
-	float * G = m->d_g;
+	const float * none = nullptr;
+	const uint32_t per = grad_rows(m, n), chunks = (n + per - 1) / per;
+	const uint64_t np = m->n_params;
+	float * part = chunks == 1 ? m->d_g : m->d_part;
 	fill_u32(reinterpret_cast<uint32_t *>(m->d_loss), 0, 1, m->s);
 	const uint64_t no = (uint64_t)n * m->n_out;
 	hipLaunchKernelGGL(k_mse, dim3(grid(no)), dim3(256), 0, m->s, m->d_y, m->d_t, m->d_dy, no, m->d_loss);
-	hipLaunchKernelGGL(k_wgrad, dim3(grid((uint64_t)(m->h + 1) * m->n_out)), dim3(256), 0, m->s, m->d_h2, m->d_dy,
-					   G + m->o_w3(), G + m->o_b3(), n, m->h, m->n_out);
-	hipLaunchKernelGGL(k_back, dim3(grid((uint64_t)n * m->h)), dim3(256), 0, m->s, m->d_dy, P + m->o_w3(), m->d_h2,
-					   m->d_dh2, n, m->h, m->n_out);
-	hipLaunchKernelGGL(k_wgrad, dim3(grid((uint64_t)(m->h + 1) * m->h)), dim3(256), 0, m->s, m->d_h1, m->d_dh2,
-					   G + m->o_w2(), G + m->o_b2(), n, m->h, m->h);
-	hipLaunchKernelGGL(k_back, dim3(grid((uint64_t)n * m->h)), dim3(256), 0, m->s, m->d_dh2, P + m->o_w2(), m->d_h1,
-					   m->d_dh1, n, m->h, m->h);
-	hipLaunchKernelGGL(k_wgrad, dim3(grid((uint64_t)(m->n_in + 1) * m->h)), dim3(256), 0, m->s, m->d_x, m->d_dh1,
-					   G + m->o_w1(), G + m->o_b1(), n, m->n_in, m->h);
+	hipLaunchKernelGGL(k_wgrad, dim3((m->h + 63) / 64, (m->n_out + 63) / 64, chunks), dim3(256), 0, m->s, m->d_h2,
+					   m->d_dy, part, np, m->o_w3(), m->o_b3(), n, m->h, m->n_out, per);
+	hipLaunchKernelGGL(k_layer<true>, layer_grid(n, m->h), dim3(256), 0, m->s, m->d_dy, P + m->o_w3(), none, m->d_h2,
+					   m->d_dh2, n, m->n_out, m->h, 0);
+	hipLaunchKernelGGL(k_wgrad, dim3((m->h + 63) / 64, (m->h + 63) / 64, chunks), dim3(256), 0, m->s, m->d_h1,
+					   m->d_dh2, part, np, m->o_w2(), m->o_b2(), n, m->h, m->h, per);
+	hipLaunchKernelGGL(k_layer<true>, layer_grid(n, m->h), dim3(256), 0, m->s, m->d_dh2, P + m->o_w2(), none, m->d_h1,
+					   m->d_dh1, n, m->h, m->h, 0);
+	hipLaunchKernelGGL(k_wgrad, dim3((m->n_in + 63) / 64, (m->h + 63) / 64, chunks), dim3(256), 0, m->s, m->d_x,
+					   m->d_dh1, part, np, m->o_w1(), m->o_b1(), n, m->n_in, m->h, per);
+	if (chunks > 1)
+		hipLaunchKernelGGL(k_sum_chunks, dim3((uint32_t)((np + 63) / 64)), dim3(256), 0, m->s, m->d_part, np, chunks,
+						   m->d_g);
 }
 
 
@@ -513,6 +651,7 @@ int tm_mlp_loss_grad(tm_mlp * m, const float * x, const float * t, uint32_t n, f
 	if (!m || !x || !t || n == 0) return set_error(TM_ERR_INVALID, "bad argument");
 	TM_CHECK(require_device());
 	TM_CHECK(ensure_batch(m, n));
+	TM_CHECK(ensure_chunks(m, n));
 	TM_HIP(hipMemcpyAsync(m->d_x, x, (size_t)n * m->n_in * 4, hipMemcpyHostToDevice, m->s));
 	TM_HIP(hipMemcpyAsync(m->d_t, t, (size_t)n * m->n_out * 4, hipMemcpyHostToDevice, m->s));
 	forward(m, n);
@@ -532,6 +671,8 @@ int tm_mlp_train(tm_mlp * m, const float * x, const float * t, uint32_t n, uint3
 	TM_CHECK(require_device());
 	const uint32_t bs = std::min(batch, n);
 	TM_CHECK(ensure_batch(m, bs));
+	TM_CHECK(ensure_chunks(m, bs));
+	if (n % bs) TM_CHECK(ensure_chunks(m, n % bs));   // the last batch's chunks may be more
 	float * dX = nullptr, * dT = nullptr;
 	uint32_t * dIdx = nullptr;
 	TM_CHECK(dalloc(&dX, (size_t)n * m->n_in));
