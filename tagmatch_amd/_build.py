@@ -28,7 +28,7 @@ HIP_FLAGS = [
 ]
 CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-I", INCLUDE, "-I", os.path.join(INCLUDE, "tagmatch")]
 
-HIP_SOURCES = ["hip_util.hip", "fib.hip", "match.hip", "match_matrix.hip", "partition.hip", "cost_model.hip"]
+HIP_SOURCES = ["hip_util.hip", "fib.hip", "match.hip", "match_matrix.hip", "match_front.hip", "partition.hip", "cost_model.hip"]
 CXX_SOURCES = ["workload.cc", "engine.cc", "server.cc", "io.cc", "expand.cc"]
 
 

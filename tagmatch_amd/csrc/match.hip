@@ -7,12 +7,11 @@
 //
 //   k_step_init
 //        zeroes what the step counts in;
-//   k_rich_rows   (KEYS_UNIQUE, KEY_BITMAP)
-//        rows start with the keys of the rich filters each query contains;
-//        the queries whose rows are not complete are listed;
-//   k_lookup_hist
+//   k_front   (match_front.hip)
 //        queries per partition (reference front_end.cc:465-477 do_match, on
-//        the device);
+//        the device); key rows start with the keys of the rich filters each
+//        query contains, and the queries whose rows are not complete are
+//        listed;
 //   k_match_x   (match_matrix.hip)
 //        the listed queries against every block of 64 filters: candidates
 //        from the blocks' AND masks, then the subset tests (reference
@@ -31,6 +30,7 @@
 #include "cost_model.h"
 #include "fib.h"
 #include "match_dev.h"
+#include "match_front.h"
 #include "match_matrix.h"
 
 #include <algorithm>
@@ -575,7 +575,7 @@ k_match_q(mq_args a) {
 					// full (one coalesced load per tile here); in one segment
 					// the LDS row is the query's whole bitmap.
 					// Flags also mark the queries whose rows the rich-filter pass
-					// (k_rich_rows) already filled.
+					// (k_front) already filled.
 					if (use_flags && (qsel[t] & ~qfullm[t])) qfullm[t] |= load_flags(t);
 					qsel[t] &= ~qfullm[t];
 					if (a.nseg <= 1 && qsel[t])
@@ -733,15 +733,36 @@ __global__ void k_init_queues(uint64_t items, uint64_t * __restrict__ qbeg, unsi
 
 // ------------------------------------------------------------- finalize
 
-// KEYS_UNIQUE: one wave per query counts its bitmap bits.
+// KEYS_UNIQUE: the keys of each row, 16 lanes per row and COUNT_ROWS rows of
+// each lane in flight.  A row flagged full (qfull, when valid) is not read:
+// 22 us for 1M queries of 2048 keys, 97 % of them full, and 4 for 100k; a
+// wave per row, every row read, took 154 and 13.
+constexpr uint32_t COUNT_ROWS = 4;
+
 __global__ void __launch_bounds__(256)
-k_bm_count(const uint32_t * __restrict__ gbm, uint32_t kw, uint32_t nq, uint32_t * __restrict__ qcount) {
-	const uint32_t qi = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-	if (qi >= nq) return;
-	uint32_t c = 0;
-	for (uint32_t w = lane; w < kw; w += 64) c += __popc(gbm[(size_t)qi * kw + w]);
-	for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-	if (lane == 0) qcount[qi] = c;
+k_bm_count(const uint32_t * __restrict__ gbm, uint32_t kw, uint32_t nq, const uint32_t * __restrict__ qfull,
+		   uint32_t n_keys, uint32_t * __restrict__ qcount) {
+	const uint32_t l = threadIdx.x & 15, q0 = (blockIdx.x * 16 + (threadIdx.x >> 4)) * COUNT_ROWS;
+	bool read[COUNT_ROWS];
+	uint32_t c[COUNT_ROWS];
+#pragma unroll
+	for (uint32_t k = 0; k < COUNT_ROWS; ++k) {
+		read[k] = q0 + k < nq && !(qfull && qfull[q0 + k] != 0u);
+		c[k] = 0;
+	}
+	for (uint32_t w = l * 4; w < kw; w += 64) {
+		quad v[COUNT_ROWS];
+#pragma unroll
+		for (uint32_t k = 0; k < COUNT_ROWS; ++k)
+			v[k] = read[k] ? load_words(gbm + (size_t)(q0 + k) * kw, w, kw) : quad{0, 0, 0, 0};
+#pragma unroll
+		for (uint32_t k = 0; k < COUNT_ROWS; ++k) c[k] += __popc(v[k][0]) + __popc(v[k][1]) + __popc(v[k][2]) + __popc(v[k][3]);
+	}
+#pragma unroll
+	for (uint32_t k = 0; k < COUNT_ROWS; ++k) {
+		for (int o = 8; o > 0; o >>= 1) c[k] += __shfl_xor(c[k], o, 64);
+		if (l == 0 && q0 + k < nq) qcount[q0 + k] = read[k] ? c[k] : n_keys;
+	}
 }
 
 // KEY_BITMAP, packed delivery: flag each query whose row is not the whole
@@ -804,17 +825,49 @@ k_row_pack(const uint32_t * __restrict__ gbm, uint32_t kw, uint32_t nq, const ui
 // mostly dense) and the dictionary reads are coalesced.  The dictionary
 // reads of BM_GROUP such 64-id groups are issued before any of their stores,
 // so a wave waits for one round trip per BM_GROUP groups, not per group.
+// A row that holds every key (its list is as long as the dictionary) is not
+// read: the dictionary is copied, 16 bytes per lane to aligned addresses.
+// Bound by the stores: 8.2 GB in 1.65 ms, 5.0 TB/s (1.76 ms word by word;
+// 1.54 with constants in place of the dictionary, 1.85 with non-temporal
+// stores; a fill of one buffer reaches 6.9 TB/s).
 // A workgroup takes BM_WAVES consecutive queries: their outputs are one
 // contiguous stretch written from one CU (16 per group measured 0.6 ms
-// faster per 1M-query step than 4, and 1 slower than 4).
+// faster per 1M-query step than 4, and 1 slower than 4; with the copy 1.65
+// ms against 1.72 with 8 and 1.74 with 4).
 constexpr uint32_t BM_GROUP = 8;
 constexpr uint32_t BM_WAVES = 16;
 
 __global__ void __launch_bounds__(BM_WAVES * 64)
 k_bm_write(const uint32_t * __restrict__ gbm, uint32_t kw, uint32_t nq, const uint64_t * __restrict__ off,
-		   const uint32_t * __restrict__ dict, uint32_t * __restrict__ vals, uint64_t cap) {
+		   const uint32_t * __restrict__ dict, uint32_t n_keys, uint32_t * __restrict__ vals, uint64_t cap) {
 	const uint32_t qi = blockIdx.x * BM_WAVES + (threadIdx.x >> 6), lane = threadIdx.x & 63;
 	if (qi >= nq) return;
+	const uint64_t end = off[qi + 1];
+	if (end - off[qi] == n_keys) {
+		uint32_t * out = vals + off[qi];
+		if (end > cap) {
+			for (uint32_t i = lane; i < n_keys && off[qi] + i < cap; i += 64) out[i] = dict[i];
+			return;
+		}
+		const uint32_t head = min((uint32_t)(-(reinterpret_cast<uintptr_t>(out) >> 2) & 3u), n_keys);
+		const uint32_t quads = (n_keys - head) / 4, tail = head + quads * 4;
+		if (lane < head) out[lane] = dict[lane];
+		if (lane < n_keys - tail) out[tail + lane] = dict[tail + lane];
+		for (uint32_t i0 = 0; i0 < quads; i0 += 64 * BM_GROUP) {
+			quad v[BM_GROUP];
+#pragma unroll
+			for (uint32_t k = 0; k < BM_GROUP; ++k) {
+				const uint32_t i = i0 + k * 64 + lane;
+				if (i < quads) v[k] = *reinterpret_cast<const quad *>(dict + head + i * 4);
+			}
+#pragma unroll
+			for (uint32_t k = 0; k < BM_GROUP; ++k) {
+				const uint32_t i = i0 + k * 64 + lane;
+				if (i < quads) *reinterpret_cast<uint4 *>(out + head + i * 4) = make_uint4(v[k][0], v[k][1], v[k][2], v[k][3]);
+			}
+		}
+		return;
+	}
 	const uint32_t * row = gbm + (size_t)qi * kw;
 	uint64_t pos = off[qi];
 	for (uint32_t wb = 0; wb < kw; wb += 64) {   // 64 words (2048 ids) per pass
@@ -1002,166 +1055,6 @@ k_seg_bounds(const uint64_t * __restrict__ prefix, uint32_t nb, uint32_t nseg, u
 		if (prefix[mid] >= target) hi = mid; else lo = mid + 1;
 	}
 	segb[k] = lo;
-}
-
-// Rich-filter pass: the key bitmaps of the rich filters that a query
-// contains, ORed into its row, which this writes whole; flag 2 when the row
-// then holds every key (the match kernel's full-key-set exit drops the
-// query), else 0.  Exact: a filter contained in the query matches it,
-// whatever the partition lookup.  A wave takes qpw queries (at most 64):
-// first one lane per query against the rich filters that hold every key
-// (most queries contain one), whose rows the wave then writes full, row by
-// row; then the other queries one at a time with the whole wave, 64 rich
-// filters per test and eight bitmaps in flight.  Large steps use 64 queries
-// per wave; small ones fewer, so that their few incomplete queries are
-// spread over more waves.
-__global__ void __launch_bounds__(256)
-k_rich_rows(const uint32_t * __restrict__ q, uint32_t nq, uint32_t qpw, const uint32_t * __restrict__ rw,
-			const uint32_t * __restrict__ rbm, uint32_t nr, uint32_t nfull, uint32_t kw, uint32_t last_mask,
-			uint32_t * __restrict__ gbm, uint32_t * __restrict__ qfull, uint32_t * __restrict__ active,
-			uint32_t * __restrict__ qact, uint32_t * __restrict__ n_active) {
-	const uint32_t lane = threadIdx.x & 63;
-	const uint32_t base = (blockIdx.x * 4 + (threadIdx.x >> 6)) * qpw;
-	if (base >= nq) return;
-	const uint32_t qi = base + lane;
-	const bool valid = lane < qpw && qi < nq;
-	uint4 x = make_uint4(0, 0, 0, 0);
-	uint2 y = make_uint2(0, 0);
-	if (valid) {
-		x = *reinterpret_cast<const uint4 *>(q + (size_t)qi * 8);
-		y = *reinterpret_cast<const uint2 *>(q + (size_t)qi * 8 + 4);
-	}
-	// the first nfull rich filters hold every key: one contained is enough
-	bool full = false;
-	if (qpw == 1) {
-		// one query (lane 0's): lanes are rich filters, 64 at a time
-		const uint32_t qx = __shfl(x.x, 0, 64), qy = __shfl(x.y, 0, 64), qz = __shfl(x.z, 0, 64),
-					   qw = __shfl(x.w, 0, 64), q4 = __shfl(y.x, 0, 64), q5 = __shfl(y.y, 0, 64);
-		bool any_full = false;
-		for (uint32_t fb = 0; fb < nfull && !any_full; fb += 64) {
-			const uint32_t f = fb + lane;
-			bool hit = false;
-			if (f < nfull) {
-				const uint4 a = *reinterpret_cast<const uint4 *>(rw + (size_t)f * 8);
-				const uint2 b = *reinterpret_cast<const uint2 *>(rw + (size_t)f * 8 + 4);
-				hit = ((a.x & ~qx) | (a.y & ~qy) | (a.z & ~qz) | (a.w & ~qw) | (b.x & ~q4) | (b.y & ~q5)) == 0;
-			}
-			any_full = __ballot(hit) != 0;
-		}
-		full = valid && any_full;
-	} else {
-		// one lane per query; the filters' words are the same for every lane
-		for (uint32_t f = 0; f < nfull; ++f) {
-			const uint4 a = sld4(rw + (size_t)f * 8);
-			const uint2 b = sld2(rw + (size_t)f * 8 + 4);
-			full |= ((a.x & ~x.x) | (a.y & ~x.y) | (a.z & ~x.z) | (a.w & ~x.w) | (b.x & ~y.x) | (b.y & ~y.y)) == 0;
-			if ((f & 7) == 7 && __ballot(valid && !full) == 0) break;
-		}
-	}
-	uint64_t m = __ballot(valid && full);
-	while (m) {
-		const uint32_t j = (uint32_t)__builtin_ctzll(m);
-		m &= m - 1;
-		uint32_t * row = gbm + (size_t)(base + j) * kw;
-		for (uint32_t w = lane; w < kw; w += 64) row[w] = w + 1 == kw ? last_mask : 0xFFFFFFFFu;
-	}
-	bool done_full = full;
-	uint64_t rest = __ballot(valid && !full);
-	while (rest) {
-		const uint32_t j = (uint32_t)__builtin_ctzll(rest);
-		rest &= rest - 1;
-		const uint32_t qx = __shfl(x.x, (int)j, 64), qy = __shfl(x.y, (int)j, 64), qz = __shfl(x.z, (int)j, 64),
-					   qw = __shfl(x.w, (int)j, 64), q4 = __shfl(y.x, (int)j, 64), q5 = __shfl(y.y, (int)j, 64);
-		uint32_t * row = gbm + (size_t)(base + j) * kw;
-		uint32_t all = 0xFFFFFFFFu;
-		for (uint32_t wb = 0; wb < kw; wb += 64) {   // 64 words (2048 keys) per pass
-			const uint32_t w = wb + lane;
-			uint32_t acc = 0;
-			for (uint32_t fb = 0; fb < nr; fb += 64) {
-				const uint32_t f = fb + lane;
-				bool hit = false;
-				if (f < nr) {
-					const uint4 a = *reinterpret_cast<const uint4 *>(rw + (size_t)f * 8);
-					const uint2 b = *reinterpret_cast<const uint2 *>(rw + (size_t)f * 8 + 4);
-					hit = ((a.x & ~qx) | (a.y & ~qy) | (a.z & ~qz) | (a.w & ~qw) | (b.x & ~q4) | (b.y & ~q5)) == 0;
-				}
-				uint64_t hm = __ballot(hit);
-				while (hm) {   // eight bitmaps in flight per round (a repeat ORs twice)
-					uint32_t jj[8];
-#pragma unroll
-					for (int k = 0; k < 8; ++k) {
-						jj[k] = hm ? (uint32_t)__builtin_ctzll(hm) : jj[0];
-						hm &= hm - 1;
-					}
-					if (w < kw) {
-						uint32_t v[8];
-#pragma unroll
-						for (int k = 0; k < 8; ++k) v[k] = rbm[(size_t)(fb + jj[k]) * kw + w];
-#pragma unroll
-						for (int k = 0; k < 8; ++k) acc |= v[k];
-					}
-				}
-			}
-			if (w < kw) {
-				row[w] = acc;
-				all &= w + 1 == kw ? (acc | ~last_mask) : acc;
-			}
-		}
-		const bool f = __ballot(all != 0xFFFFFFFFu) == 0;
-		if (lane == j) done_full = f;
-	}
-	if (valid) qfull[qi] = done_full ? 2u : 0u;
-	if (active) {
-		const uint64_t am = __ballot(valid && !done_full);
-		if (am) {
-			uint32_t at = 0;
-			if (lane == 0) at = atomicAdd(n_active, (uint32_t)__popcll(am));
-			at = __shfl(at, 0, 64) + mbcnt64(am);
-			if (valid && !done_full) {
-				active[at] = qi;
-				uint4 * d = reinterpret_cast<uint4 *>(qact + (size_t)at * 8);
-				d[0] = x;
-				d[1] = make_uint4(y.x, y.y, 0u, 0u);
-			}
-		}
-	}
-}
-
-// Queries per partition (the lookup's counts).  Lanes are partitions, 64 at
-// a time; the wave's share of the queries is read with scalar loads, and
-// each lane counts the queries that select its partition in a register.
-// Counts meet in LDS (P counters), then one global atomic per partition per
-// workgroup.
-__global__ void __launch_bounds__(256)
-k_lookup_hist(const uint32_t * __restrict__ q, uint32_t nq, const uint32_t * __restrict__ part_info, uint32_t P,
-			  uint32_t * __restrict__ pcount) {
-	extern __shared__ uint32_t s_cnt[];
-	for (uint32_t p = threadIdx.x; p < P; p += 256) s_cnt[p] = 0;
-	__syncthreads();
-	const uint32_t lane = threadIdx.x & 63;
-	const uint32_t gw = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-	const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
-	const uint32_t per = (nq + nwaves - 1) / nwaves;
-	const uint32_t qa = min(gw * per, nq), qb = min(qa + per, nq);
-	for (uint32_t p0 = 0; p0 < P; p0 += 64) {
-		const uint32_t p = p0 + lane;
-		uint32_t m[6] = {0, 0, 0, 0, 0, 0};
-		if (p < P)
-			for (int j = 0; j < 6; ++j) m[j] = part_info[(size_t)p * 8 + j];
-		uint32_t cnt = 0;
-#pragma unroll 4
-		for (uint32_t i = qa; i < qb; ++i) {
-			const uint4 x = sld4(q + (size_t)i * 8);
-			const uint2 y = sld2(q + (size_t)i * 8 + 4);
-			const uint32_t t = (m[0] & ~x.x) | (m[1] & ~x.y) | (m[2] & ~x.z) | (m[3] & ~x.w) | (m[4] & ~y.x) |
-							   (m[5] & ~y.y);
-			cnt += t == 0;
-		}
-		if (p < P && cnt) atomicAdd(&s_cnt[p], cnt);
-	}
-	__syncthreads();
-	for (uint32_t p = threadIdx.x; p < P; p += 256)
-		if (s_cnt[p]) atomicAdd(&pcount[p], s_cnt[p]);
 }
 
 // ------------------------------------------------------------- kernel table
@@ -1489,15 +1382,15 @@ void enqueue_stats(tm_ring * r, uint32_t nq);
 void enqueue_finalize(tm_ring * r, uint32_t nq) {
 	hipStream_t s = r->s;
 	const int mode = r->cfg.mode;
-	uint32_t gq = (nq + 3) / 4;
-	if (gq == 0) gq = 1;
 	if (mode == TM_MODE_KEY_BITMAP) {
 		// the rows are the results: no expansion
 	} else if (mode == TM_MODE_KEYS_UNIQUE) {
-		hipLaunchKernelGGL(k_bm_count, dim3(gq), dim3(256), 0, s, r->d_gbm, r->kw, nq, r->d_qcount);
+		hipLaunchKernelGGL(k_bm_count, dim3(std::max(1u, (nq + 16 * COUNT_ROWS - 1) / (16 * COUNT_ROWS))), dim3(256), 0, s,
+						   r->d_gbm, r->kw, nq, r->qfull_valid ? r->d_qfull : (const uint32_t *)nullptr, r->fib->n_keys,
+						   r->d_qcount);
 		scan_u32_to_u64(r->d_qcount, r->d_off, nq, r->d_scan, s);
 		hipLaunchKernelGGL(k_bm_write, dim3(std::max(1u, (nq + BM_WAVES - 1) / BM_WAVES)), dim3(BM_WAVES * 64), 0, s,
-						   r->d_gbm, r->kw, nq, r->d_off, r->fib->key_dict, r->d_vals, r->val_cap);
+						   r->d_gbm, r->kw, nq, r->d_off, r->fib->key_dict, r->fib->n_keys, r->d_vals, r->val_cap);
 	} else {
 		const bool keys = mode == TM_MODE_KEYS_ALL;
 		dev_fib_view v = r->fib->view();
@@ -1597,6 +1490,33 @@ int enqueue_values(tm_ring * r, mx_args a, uint32_t rows, uint32_t grid, bool ev
 	return TM_OK;
 }
 
+// The pass before the match: partitions counted into pcount (NULL: not), and
+// with `rich` the rows started from the rich filters' keys.
+void enqueue_rows(tm_ring * r, uint32_t nq, bool rich, uint32_t * pcount, bool list) {
+	const tm_fib * f = r->fib;
+	front_args a;
+	std::memset(&a, 0, sizeof(a));
+	a.q = r->d_q;
+	a.nq = nq;
+	a.part_info = f->part_info;
+	a.P = r->P;
+	a.pcount = pcount;
+	if (rich) {
+		a.rich_words = f->d_rich_words;
+		a.rich_bm = f->d_rich_bm;
+		a.n_rich = f->n_rich;
+		a.n_full = f->n_rich_full;
+	}
+	a.kw = r->kw;
+	a.last_mask = (f->n_keys & 31) ? (1u << (f->n_keys & 31)) - 1u : 0xFFFFFFFFu;
+	a.gbm = r->d_gbm;
+	a.qfull = r->d_qfull;
+	a.active = list ? r->d_active : nullptr;
+	a.qact = r->d_qact;
+	a.n_active = r->d_nact;
+	front_launch(a, r->s);
+}
+
 // The persistent step on the matrix cores.
 int enqueue_matrix(tm_ring * r, uint32_t nq, bool events) {
 	hipStream_t s = r->s;
@@ -1605,29 +1525,10 @@ int enqueue_matrix(tm_ring * r, uint32_t nq, bool events) {
 	const bool exit_on = keys && r->lds_bm && r->kw > 0 && r->cfg.full_exit != 2;
 	const bool rich_pass = keys && r->kw > 0 && r->fib->n_rich > 0 && nq > 0;
 	const bool compact = rich_pass && exit_on;
-	const uint32_t last_mask = (r->fib->n_keys & 31) ? (1u << (r->fib->n_keys & 31)) - 1u : 0xFFFFFFFFu;
 	hipLaunchKernelGGL(k_step_init, dim3(1), dim3(256), 0, s, r->d_pcount, P, r->d_cnt, r->d_qnext,
 					   keys ? NQUEUE : 2 * NQUEUE, r->d_nact);
-	if (rich_pass) {
-		uint32_t qpw = 64;
-		while (qpw > 1 && (uint64_t)nq < (uint64_t)qpw * 4096) qpw >>= 1;
-		const uint32_t waves = (nq + qpw - 1) / qpw;
-		hipLaunchKernelGGL(k_rich_rows, dim3((waves + 3) / 4), dim3(256), 0, s, r->d_q, nq, qpw, r->fib->d_rich_words,
-						   r->fib->d_rich_bm, r->fib->n_rich, r->fib->n_rich_full, r->kw, last_mask, r->d_gbm,
-						   r->d_qfull, compact ? r->d_active : nullptr, r->d_qact, r->d_nact);
-	} else if (keys) {
-		fill_u32(r->d_gbm, 0, (uint64_t)nq * r->kw, s);
-	}
-	if (nq) {
-		if (P <= 16384) {
-			const uint32_t gh = (uint32_t)std::min<uint64_t>((nq + 255) / 256, 2048);
-			hipLaunchKernelGGL(k_lookup_hist, dim3(gh), dim3(256), (size_t)P * 4, s, r->d_q, nq, r->fib->part_info, P,
-							   r->d_pcount);
-		} else {
-			hipLaunchKernelGGL(k_lookup_count, dim3((nq + 255) / 256), dim3(256), 0, s, r->d_q, nq, r->fib->part_info,
-							   P, r->d_pcount);
-		}
-	}
+	if (keys && !rich_pass) fill_u32(r->d_gbm, 0, (uint64_t)nq * r->kw, s);
+	enqueue_rows(r, nq, rich_pass, r->d_pcount, compact);
 	if (!keys) {
 		mx_args a = matrix_args(r, MX_COUNT);
 		a.nq = nq;
@@ -1669,13 +1570,13 @@ int enqueue_matrix(tm_ring * r, uint32_t nq, bool events) {
 int enqueue_persistent(tm_ring * r, uint32_t nq, bool events) {
 	hipStream_t s = r->s;
 	const uint32_t P = r->P;
+	const bool exit_on = keyrows(r->cfg) && r->lds_bm && r->kw > 0 && r->cfg.full_exit != 2;
+	const bool rich_pass = exit_on && r->fib->n_rich > 0 && nq > 0;
+	if (!r->use_iorder && !r->cfg.log_units && (!exit_on || rich_pass)) return enqueue_matrix(r, nq, events);
 	fill_u32(r->d_pcount, 0, P, s);
 	fill_u64(reinterpret_cast<uint64_t *>(r->d_cnt), 0, 8, s);
 	const uint64_t nqg = (uint64_t)r->tiles * 64;
 	const uint64_t tiles = (nq + nqg - 1) / nqg;
-	const bool exit_on = keyrows(r->cfg) && r->lds_bm && r->kw > 0 && r->cfg.full_exit != 2;
-	const bool rich_pass = exit_on && r->fib->n_rich > 0 && nq > 0;
-	if (!r->use_iorder && !r->cfg.log_units && (!exit_on || rich_pass)) return enqueue_matrix(r, nq, events);
 	r->n_wgstat = 0;
 	const int nw = step_waves(r, tiles);
 	// Small submissions: cut each tile's work into block segments so that
@@ -1718,14 +1619,7 @@ int enqueue_persistent(tm_ring * r, uint32_t nq, bool events) {
 	if (rich_pass) {
 		// rows start with the keys of the rich filters each query contains
 		// (written whole, with the flags); full rows need no test at all
-		// queries per wave: 64 for large steps, fewer (down to 1) below
-		// 4096 waves' worth
-		uint32_t qpw = 64;
-		while (qpw > 1 && (uint64_t)nq < (uint64_t)qpw * 4096) qpw >>= 1;
-		const uint32_t waves = (nq + qpw - 1) / qpw;
-		hipLaunchKernelGGL(k_rich_rows, dim3((waves + 3) / 4), dim3(256), 0, s, r->d_q, nq, qpw, r->fib->d_rich_words,
-						   r->fib->d_rich_bm, r->fib->n_rich, r->fib->n_rich_full, r->kw, last_mask, r->d_gbm,
-						   r->d_qfull, (uint32_t *)nullptr, (uint32_t *)nullptr, (uint32_t *)nullptr);
+		enqueue_rows(r, nq, true, nullptr, false);
 	} else if (nseg > 1 && keyrows(r->cfg)) {
 		fill_u32(r->d_gbm, 0, (uint64_t)nq * r->kw, s);
 		fill_u32(r->d_qfull, 0, nq, s);

@@ -43,4 +43,25 @@ __device__ inline uint2 sld2(const uint32_t * p) {
 }
 __device__ inline uint32_t sld1(const uint32_t * p) { return *(cu32_t *)(p); }
 
+// Four words, not aligned: rows begin at any word.
+typedef uint32_t quad __attribute__((ext_vector_type(4), aligned(4)));
+
+// Words w .. w + 3 of a row of kw words.
+__device__ inline void store_words(uint32_t * row, uint32_t w, uint32_t kw, const quad & v) {
+	if (w + 4 <= kw) {
+		*reinterpret_cast<quad *>(row + w) = v;
+		return;
+	}
+#pragma unroll
+	for (uint32_t k = 0; k < 4; ++k)
+		if (w + k < kw) row[w + k] = v[k];
+}
+__device__ inline quad load_words(const uint32_t * row, uint32_t w, uint32_t kw) {
+	if (w + 4 <= kw) return *reinterpret_cast<const quad *>(row + w);
+	quad v = {0, 0, 0, 0};
+#pragma unroll
+	for (uint32_t k = 0; k < 4; ++k)
+		if (w + k < kw) v[k] = row[w + k];
+	return v;
+}
 } // namespace tmx

@@ -1,15 +1,7 @@
 // The subset match on the matrix cores.
-//
-// f is a subset of q exactly when f and ~q share no bit, that is when the
-// dot product of their bits is zero.  The bits of a 32-bit word spread over
-// 32 4-bit floats (E2M1) with four ANDs and a shift, in any order as long as
-// both operands use the same one, and a product of such values is zero or
-// positive; so one v_mfma_f32_32x32x64_f8f6f4 tests 64 bits of 32 filters
-// against 32 queries, three of them test the pairs whole, and an
-// accumulator is zero exactly where the filter is a subset.  Sums are
-// multiples of 0.25 up to 4 * 192: exact in FP32.
 #include "match_matrix.h"
 #include "match_dev.h"
+#include "match_mfma.h"
 
 #include <algorithm>
 
@@ -17,65 +9,10 @@ using namespace tmx;
 
 namespace {
 
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-
 constexpr uint32_t LIST = 256;   // candidate queries of a block taken at a time
 constexpr uint32_t LOG = 128;    // hits a wave stages
 constexpr uint32_t AHEAD = 3;    // blocks whose words are loaded together (one tile of queries)
 constexpr uint32_t PARTIAL = 0x8000;   // marks a listed block with fewer than 64 filters
-
-// 32 bits as 32 E2M1 values: bit b as 0.5, 1, 2, 2 for b mod 4 = 0, 1, 2, 3
-// (0x8 would be -0).
-__device__ inline v8i spread(uint32_t w) {
-	v8i r = {0, 0, 0, 0, 0, 0, 0, 0};
-	r[0] = (int)(w & 0x11111111u);
-	r[1] = (int)(w & 0x22222222u);
-	r[2] = (int)(w & 0x44444444u);
-	r[3] = (int)((w >> 1) & 0x44444444u);
-	return r;
-}
-
-__device__ inline v16f mfma(const v8i & a, const v8i & b, const v16f & c) {
-	return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 4, 4, 0, 0, 0, 0);
-}
-
-// Bit r set where register r of lo (r < 16) or r - 16 of hi is zero.  The
-// accumulators are multiples of 0.25 below 256, so their low halves are
-// zero: two high halves make one word, and a packed minimum with 1 leaves a
-// bit of each (1.5 instructions per register; compares and carries take 2
-// and wait states).
-__device__ inline uint32_t zero_mask(const v16f & lo, const v16f & hi) {
-	uint32_t m = 0;
-#pragma unroll
-	for (int i = 15; i >= 0; --i) {
-		const uint32_t two = __builtin_amdgcn_perm(__float_as_uint(hi[i]), __float_as_uint(lo[i]), 0x07060302u);
-		uint32_t one;
-		asm("v_pk_min_u16 %0, %1, %2" : "=v"(one) : "v"(two), "v"(0x00010001u));
-		m = (m << 1) | one;
-	}
-	return ~m;
-}
-
-// Wave-level ordering of LDS traffic between lanes.
-__device__ inline void wave_fence() {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ inline uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
-
-// Inclusive prefix sum over the wave's lanes.
-__device__ inline uint32_t wave_prefix(uint32_t x) {
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);   // row_shr:1
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);   // row_bcast:15
-	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);   // row_bcast:31
-	return x;
-}
 
 // ORs key ids into a row: a word is read first, and written only where the
 // bit is missing (rows hold most keys already; a stale read costs a
@@ -413,14 +350,6 @@ k_match_x(mx_args a) {
 					for (int k = 0; k < 3; ++k) fa[k][mt] = spread(fw[k][mt] | dead);
 				}
 			};
-			// valid_lanes in zero_mask's order, for this lane's half
-			auto half_mask = [&](uint64_t lm) -> uint32_t {
-				if (lm == ~0ULL) return ~0u;
-				uint64_t x = (lm >> (4 * h)) & 0x0F0F0F0F0F0F0F0FULL;
-				x = (x | (x >> 4)) & 0x00FF00FF00FF00FFULL;
-				x = (x | (x >> 8)) & 0x0000FFFF0000FFFFULL;
-				return (uint32_t)x | (uint32_t)(x >> 16);
-			};
 			// hm: the filters (zero_mask's order) of block b that query qi of
 			// this lane contains
 			auto take_hits = [&](uint32_t hm, uint32_t qi, uint32_t b) {
@@ -478,7 +407,7 @@ k_match_x(mx_args a) {
 							lo = mfma(fa[k][0], qv[k], lo);
 							hi = mfma(fa[k][1], qv[k], hi);
 						}
-						take_hits(n < nqs ? zero_mask(lo, hi) & half_mask(lm) : 0u, n, b);
+						take_hits(n < nqs ? zero_mask(lo, hi) & half_mask(lm, h) : 0u, n, b);
 					}
 				}
 			} else {
@@ -495,7 +424,7 @@ k_match_x(mx_args a) {
 					const uint64_t lm = valid_lanes(vis, b);
 					v8i fa[3][2];
 					operands(fw, lm, fa);
-					const uint32_t keep = half_mask(lm);
+					const uint32_t keep = half_mask(lm, h);
 					if (v + WAVES < nvis) {
 						next = uniform(s_vis[v + WAVES]);
 						load_words(p0 + (next & ~PARTIAL), fw);
