@@ -40,10 +40,17 @@ __host__ __device__ constexpr uint32_t mx_mask_words(int mode) {
 __host__ __device__ constexpr uint32_t mx_visits(int mode) { return mode == MX_KEYS_LDS ? 128u : MX_VISITS; }
 
 // Work items of a launch over nq queries and nblk blocks: item = segment *
-// nsuper + super, segments of seg blocks, supers of sq queries.  Few queries:
-// one item per workgroup.  Otherwise four per workgroup or more, so that
-// uneven items even out, as long as a segment has 64 blocks.  seg_min: least
-// blocks per segment (a bound on the segments), 0: none.
+// nsuper + super, supers of sq queries, segments of about seg blocks: every
+// nseg-th tile of 32, so that the blocks with many matches, which lie
+// together, are spread over all segments (against runs of blocks: 100k
+// queries on 1M filters 0.74 and 0.63 ms, the uneven units 3.95 and 3.52).
+// Work for at most five items of 64 blocks per workgroup: one item each (10M
+// filters: 1000 queries 31 us against 52, 10k 75 against 85; 1M filters, 16
+// queries 13 against 17 for two rounds).  Otherwise 128 blocks: between 64
+// and 256 it is the fastest or within 4 % of it (1M filters, 300k queries,
+// for 64, 128, 256: 1.58, 1.52, 1.65 ms; 10M, 1M queries: 1.00, 0.98, 1.00;
+// 65k without the full-row exit: 11.7, 11.4, 11.4).  seg_min: least blocks
+// per segment (a bound on the segments), 0: none.
 struct mx_shape {
 	uint32_t sq, nsuper, seg, nseg;
 };
@@ -55,27 +62,20 @@ __host__ __device__ inline mx_shape mx_shape_of(int mode, uint32_t nq, uint32_t 
 	// instead of 1.30 ms)
 	while (sq > 256 && (uint64_t)((nq + sq - 1) / sq) * ((nblk + 63) / 64) < 4ull * resident) sq = (sq / 2 + 63) & ~63u;
 	const uint32_t nsuper = (nq + sq - 1) / sq;
-	const uint32_t fit = mx_mask_words(mode) / (2 * (sq / 64) + 1);
-	const uint32_t most = (fit < mx_visits(mode) ? fit : mx_visits(mode)) & ~31u;   // 64 or more
-	uint32_t seg = most;
-	if ((uint64_t)nsuper * ((nblk + 63) / 64) <= 4ull * resident) {
+	uint32_t seg = 128;
+	if ((uint64_t)nsuper * ((nblk + 63) / 64) <= 5ull * resident) {
 		const uint64_t per = ((uint64_t)nblk * nsuper + resident - 1) / resident;
-		const uint64_t up = (per + 31) & ~31ull;
-		seg = up < 32 ? 32u : up < MX_VISITS ? (uint32_t)up : MX_VISITS;
-	} else {
-		while (seg > 64 && (uint64_t)nsuper * ((nblk + seg - 1) / seg) < 4ull * resident) {
-			seg = (seg / 2) & ~31u;
-			if (seg < 64) seg = 64;
-		}
+		seg = per < 32 ? 32u : (uint32_t)(per + 31) & ~31u;
 	}
 	if (seg < seg_min) seg = seg_min;
 	if (seg_fixed) seg = seg_fixed;
 	if (seg > MX_MAX_SEG) seg = MX_MAX_SEG;
+	const uint32_t tiles = (nblk + 31) / 32, per = (seg + 31) / 32;
 	mx_shape h;
 	h.sq = sq;
 	h.nsuper = nsuper;
 	h.seg = seg;
-	h.nseg = (nblk + seg - 1) / seg;
+	h.nseg = (tiles + per - 1) / per;
 	return h;
 }
 

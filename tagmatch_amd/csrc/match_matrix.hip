@@ -81,7 +81,8 @@ k_match_x(mx_args a) {
 			item = blockIdx.x;
 			if (turn || item >= items) break;
 		}
-		uint32_t q0, nqs, b0, b1, seg;
+		// blocks of the item: tiles of 32, `apart` blocks from one to the next
+		uint32_t q0, nqs, b0, apart, nloc, b_end, seg;
 		if (a.units) {
 			uint32_t lo = 0, hi = a.n_units;
 			while (hi - lo > 1) {
@@ -95,16 +96,20 @@ k_match_x(mx_args a) {
 			const uint32_t sup = local - seg * u0.w;
 			q0 = u0.y + sup * SUPER;
 			nqs = min(SUPER, u0.y + u0.z - q0);
-			b0 = u1.z + seg * u1.y;
-			b1 = min(b0 + u1.y, u1.w);
+			b0 = u1.z + seg * 32;
+			apart = u1.x * 32;
+			b_end = u1.w;
 		} else {
 			seg = item / sh.nsuper;
 			const uint32_t sup = item - seg * sh.nsuper;
 			q0 = sup * sh.sq;
 			nqs = min(sh.sq, nq_all - q0);
-			b0 = seg * sh.seg;
-			b1 = min(b0 + sh.seg, a.nblk);
+			b0 = seg * 32;
+			apart = sh.nseg * 32;
+			b_end = a.nblk;
 		}
+		nloc = b0 < b_end ? ((b_end - b0 + apart - 1) / apart) * 32 : 0u;
+		auto block_of = [&](uint32_t i) -> uint32_t { return b0 + (i >> 5) * apart + (i & 31u); };
 		// the item's queries, inverted; all ones (a subset of nothing but the
 		// empty filter) up to a whole number of tiles
 		if (MODE == MX_KEYS_LDS)
@@ -142,7 +147,7 @@ k_match_x(mx_args a) {
 				const bool mine = base + lane < nlog;
 				const uint32_t e = mine ? log[base + lane] : 0u;
 				const uint32_t qi = e & 0xFFFu, ql = q0 + qi;
-				const uint32_t slot = (b0 + (e >> 18)) * 64 + ((e >> 12) & 63u);
+				const uint32_t slot = block_of(e >> 18) * 64 + ((e >> 12) & 63u);
 				if (MODE == MX_WRITE) {
 					if (mine) {
 						const uint64_t at = a.off[ql] + atomicAdd(&s_cnt[qi], 1u);
@@ -262,9 +267,9 @@ k_match_x(mx_args a) {
 		if (n + 1 >= np)
 			for (uint32_t bit = 0; bit < 32; ++bit)
 				if (n * 64 + h * 4 + bit + (bit & 28u) >= nqs) tail &= ~(1u << bit);
-		const uint32_t pass = min(VISITS, MASK / stride);
-		for (uint32_t p0 = b0; p0 < b1; p0 += pass) {
-			const uint32_t nb = min(pass, b1 - p0);
+		const uint32_t pass = min(VISITS, MASK / stride) & ~31u;
+		for (uint32_t p0 = 0; p0 < nloc; p0 += pass) {
+			const uint32_t nb = min(pass, nloc - p0);
 			if (tid == 0) s_nvis = 0;
 			__syncthreads();
 			// Candidates: block masks (columns, 32 at a time) against every
@@ -283,8 +288,9 @@ k_match_x(mx_args a) {
 				{
 					uint32_t w[3] = {~0u, ~0u, ~0u};
 					const uint32_t b = bt * 32 + n;
-					if (b < nb) {
-						const uint32_t * bi = a.f.blk_info + (size_t)(p0 + b) * 8;
+					const uint32_t blk = block_of(p0 + b);
+					if (b < nb && blk < b_end) {
+						const uint32_t * bi = a.f.blk_info + (size_t)blk * 8;
 #pragma unroll
 						for (int k = 0; k < 3; ++k) w[k] = bi[2 * k + h];
 						nv = bi[6];
@@ -350,9 +356,9 @@ k_match_x(mx_args a) {
 					for (int k = 0; k < 3; ++k) fa[k][mt] = spread(fw[k][mt] | dead);
 				}
 			};
-			// hm: the filters (zero_mask's order) of block b that query qi of
-			// this lane contains
-			auto take_hits = [&](uint32_t hm, uint32_t qi, uint32_t b) {
+			// hm: the filters (zero_mask's order) of the item's block `at` that
+			// query qi of this lane contains
+			auto take_hits = [&](uint32_t hm, uint32_t qi, uint32_t at) {
 				const uint64_t ev = __ballot(hm != 0);
 				if (ev == 0) return;
 				w_hev += (uint32_t)__popc((uint32_t)ev | (uint32_t)(ev >> 32));
@@ -363,7 +369,7 @@ k_match_x(mx_args a) {
 				}
 				// rows known to hold every key gain nothing
 				if (MODE == MX_KEYS && a.qfull && ((s_full[qi >> 5] >> (qi & 31)) & 1u)) hm = 0;
-				const uint32_t tag = qi | ((b - b0) << 18) | (h << 14);
+				const uint32_t tag = qi | (at << 18) | (h << 14);
 				uint64_t hb = __ballot(hm != 0);
 				while (hb) {
 					const uint32_t c = (uint32_t)__popcll(hb);
@@ -390,13 +396,13 @@ k_match_x(mx_args a) {
 					for (uint32_t g = 0; g < AHEAD; ++g) {
 						// past the end: the first block again, not used
 						vis[g] = uniform(s_vis[v0 + g * WAVES < nvis ? v0 + g * WAVES : v0]);
-						load_words(p0 + (vis[g] & ~PARTIAL), fw[g]);
+						load_words(block_of(p0 + (vis[g] & ~PARTIAL)), fw[g]);
 					}
 #pragma unroll
 					for (uint32_t g = 0; g < AHEAD; ++g) {
 						if (v0 + g * WAVES >= nvis) break;
-						const uint32_t b = p0 + (vis[g] & ~PARTIAL);
-						const uint64_t lm = valid_lanes(vis[g], b);
+						const uint32_t at = p0 + (vis[g] & ~PARTIAL);
+						const uint64_t lm = valid_lanes(vis[g], block_of(at));
 						v8i fa[3][2];
 						operands(fw[g], lm, fa);
 						w_test += nqs;
@@ -407,7 +413,7 @@ k_match_x(mx_args a) {
 							lo = mfma(fa[k][0], qv[k], lo);
 							hi = mfma(fa[k][1], qv[k], hi);
 						}
-						take_hits(n < nqs ? zero_mask(lo, hi) & half_mask(lm, h) : 0u, n, b);
+						take_hits(n < nqs ? zero_mask(lo, hi) & half_mask(lm, h) : 0u, n, at);
 					}
 				}
 			} else {
@@ -416,18 +422,18 @@ k_match_x(mx_args a) {
 				uint32_t fw[3][2], next = 0;
 				if (wave < nvis) {
 					next = uniform(s_vis[wave]);
-					load_words(p0 + (next & ~PARTIAL), fw);
+					load_words(block_of(p0 + (next & ~PARTIAL)), fw);
 				}
 				for (uint32_t v = wave; v < nvis; v += WAVES) {
-					const uint32_t vis = next, bn = vis & ~PARTIAL, b = p0 + bn;
+					const uint32_t vis = next, bn = vis & ~PARTIAL, at = p0 + bn;
 					uint32_t m = n < np ? s_mask[bn * stride + h * np + n] : 0u;
-					const uint64_t lm = valid_lanes(vis, b);
+					const uint64_t lm = valid_lanes(vis, block_of(at));
 					v8i fa[3][2];
 					operands(fw, lm, fa);
 					const uint32_t keep = half_mask(lm, h);
 					if (v + WAVES < nvis) {
 						next = uniform(s_vis[v + WAVES]);
-						load_words(p0 + (next & ~PARTIAL), fw);
+						load_words(block_of(p0 + (next & ~PARTIAL)), fw);
 					}
 					// candidates as a list: each lane writes those of its mask
 					// behind the lanes before it, LIST at a time
@@ -461,7 +467,7 @@ k_match_x(mx_args a) {
 								hi = mfma(fa[k][1], qv, hi);
 							}
 							const uint32_t hm = zero_mask(lo, hi);
-							take_hits(valid ? hm & keep : 0u, qi, b);
+							take_hits(valid ? hm & keep : 0u, qi, at);
 						}
 						wave_fence();
 					}
