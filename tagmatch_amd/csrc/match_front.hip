@@ -95,7 +95,7 @@ k_front(front_args a) {
 				uint32_t w[3];
 				query_words(sub * 64 + mt * 32 + n, mt * 32 + n < nv, w);
 #pragma unroll
-				for (int k = 0; k < 3; ++k) qv[mt][k] = spread(w[k]);
+				for (int k = 0; k < 3; ++k) qv[mt][k] = spread_up(w[k]);
 			}
 			uint32_t m[3], m1[3];
 			auto load_masks = [&](uint32_t t, uint32_t (&w)[3]) {
@@ -106,7 +106,7 @@ k_front(front_args a) {
 			for (uint32_t t = f0; t < tiles; t += f_step) {
 				load_masks(t + f_step, m1);   // past the end: the last again
 				const uint32_t p = t * 32 + n;
-				v16f lo = {}, hi = {};
+				v16f lo = start_lo(), hi = start_hi();
 #pragma unroll
 				for (int k = 0; k < 3; ++k) {
 					const v8i pv = spread(m[k]);
@@ -114,7 +114,7 @@ k_front(front_args a) {
 					hi = mfma(qv[1][k], pv, hi);
 					m[k] = m1[k];
 				}
-				const uint32_t c = (uint32_t)__popc(zero_mask(lo, hi) & keep);
+				const uint32_t c = (uint32_t)__popc(subset_mask(lo, hi) & keep);
 				if (p < np && c) atomicAdd(&s_cnt[p], c);
 			}
 		}
@@ -191,10 +191,10 @@ k_front(front_args a) {
 			};
 			load_filters(ft0, f);
 #pragma unroll
-			for (int k = 0; k < 3; ++k) qv[k] = spread(w[k]);
+			for (int k = 0; k < 3; ++k) qv[k] = spread_up(w[k]);
 			for (uint32_t ft = ft0; ft < fts; ft += step) {
 				load_filters(ft + step, f1);
-				v16f lo = {}, hi = {};
+				v16f lo = start_lo(), hi = start_hi();
 #pragma unroll
 				for (int k = 0; k < 3; ++k) {
 					lo = mfma(spread(f[k]), qv[k], lo);
@@ -203,7 +203,7 @@ k_front(front_args a) {
 #pragma unroll
 				for (int k = 0; k < 6; ++k) f[k] = f1[k];
 				const uint32_t nf = min(64u, a.n_rich - ft * 64);
-				s_mask[c * MASKS + 2 * ft + h] = zero_mask(lo, hi) & half_mask(nf < 64 ? (1ULL << nf) - 1ULL : ~0ULL, h);
+				s_mask[c * MASKS + 2 * ft + h] = subset_mask(lo, hi) & half_mask(nf < 64 ? (1ULL << nf) - 1ULL : ~0ULL, h);
 			}
 		}
 		__syncthreads();

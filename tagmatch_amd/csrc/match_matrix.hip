@@ -296,19 +296,19 @@ k_match_x(mx_args a) {
 						nv = bi[6];
 					}
 #pragma unroll
-					for (int k = 0; k < 3; ++k) bm[k] = spread(w[k]);
+					for (int k = 0; k < 3; ++k) bm[k] = spread_up(w[k]);
 				}
 				uint32_t any = 0;
 				uint32_t * mw = s_mask + (bt * 32 + n) * stride + h * np;
 				for (; t < t1; ++t) {
 					const uint32_t * sq = s_q + h * SUPER + t * 64 + n;
-					v16f lo = {}, hi = {};
+					v16f lo = start_lo(), hi = start_hi();
 #pragma unroll
 					for (int k = 0; k < 3; ++k) {
 						lo = mfma(spread(sq[2 * k * SUPER]), bm[k], lo);
 						hi = mfma(spread(sq[2 * k * SUPER + 32]), bm[k], hi);
 					}
-					const uint32_t m = nv ? zero_mask(lo, hi) : 0u;
+					const uint32_t m = nv ? subset_mask(lo, hi) : 0u;
 					if (bt * 32 + n < nb) mw[t] = m;
 					any |= m;
 				}
@@ -353,10 +353,10 @@ k_match_x(mx_args a) {
 				for (int mt = 0; mt < 2; ++mt) {
 					const uint32_t dead = (lm >> (mt * 32 + n)) & 1 ? 0u : ~0u;
 #pragma unroll
-					for (int k = 0; k < 3; ++k) fa[k][mt] = spread(fw[k][mt] | dead);
+					for (int k = 0; k < 3; ++k) fa[k][mt] = spread_up(fw[k][mt] | dead);
 				}
 			};
-			// hm: the filters (zero_mask's order) of the item's block `at` that
+			// hm: the filters (subset_mask's order) of the item's block `at` that
 			// query qi of this lane contains
 			auto take_hits = [&](uint32_t hm, uint32_t qi, uint32_t at) {
 				const uint64_t ev = __ballot(hm != 0);
@@ -407,13 +407,13 @@ k_match_x(mx_args a) {
 						operands(fw[g], lm, fa);
 						w_test += nqs;
 						w_visit += 1;
-						v16f lo = {}, hi = {};
+						v16f lo = start_lo(), hi = start_hi();
 #pragma unroll
 						for (int k = 0; k < 3; ++k) {
 							lo = mfma(fa[k][0], qv[k], lo);
 							hi = mfma(fa[k][1], qv[k], hi);
 						}
-						take_hits(n < nqs ? zero_mask(lo, hi) & half_mask(lm, h) : 0u, n, at);
+						take_hits(n < nqs ? subset_mask(lo, hi) & half_mask(lm, h) : 0u, n, at);
 					}
 				}
 			} else {
@@ -459,14 +459,14 @@ k_match_x(mx_args a) {
 						for (uint32_t base = 0; base < cnt; base += 32) {
 							const bool valid = base + n < cnt;
 							const uint32_t qi = list[valid ? base + n : base];
-							v16f lo = {}, hi = {};
+							v16f lo = start_lo(), hi = start_hi();
 #pragma unroll
 							for (int k = 0; k < 3; ++k) {
 								const v8i qv = spread(s_q[(2 * k + h) * SUPER + qi]);
 								lo = mfma(fa[k][0], qv, lo);
 								hi = mfma(fa[k][1], qv, hi);
 							}
-							const uint32_t hm = zero_mask(lo, hi);
+							const uint32_t hm = subset_mask(lo, hi);
 							take_hits(valid ? hm & keep : 0u, qi, at);
 						}
 						wave_fence();

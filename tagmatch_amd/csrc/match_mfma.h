@@ -3,12 +3,12 @@
 //
 // f is a subset of q exactly when f and ~q share no bit, that is when the
 // dot product of their bits is zero.  The bits of a 32-bit word spread over
-// 32 4-bit floats (E2M1) with four ANDs and a shift, in any order as long as
-// both operands use the same one, and a product of such values is zero or
-// positive; so one v_mfma_f32_32x32x64_f8f6f4 tests 64 bits of 32 filters
-// against 32 queries, three of them test the pairs whole, and an
-// accumulator is zero exactly where the filter is a subset.  Sums are
-// multiples of 0.25 up to 4 * 192: exact in FP32.
+// 32 4-bit floats (E2M1) with a few ANDs and shifts, in any order as long as
+// both operands use the same one; so one v_mfma_f32_32x32x64_f8f6f4 tests 64
+// bits of 32 filters against 32 queries, and three of them test the pairs
+// whole.  A shared bit adds 1 or more, the accumulators start at -0.5 or -1:
+// the sign bit is set exactly where the filter is a subset.  Sums are
+// multiples of 0.5 up to 4 * 192: exact in FP32.
 //
 // Lane l = 32 h + n holds words 2 k + h (k = 0, 1, 2) of row or column n of
 // an operand, and of a result column n and the rows 8 (i / 4) + 4 h + i % 4.
@@ -31,26 +31,32 @@ __device__ inline v8i spread(uint32_t w) {
 	r[3] = (int)((w >> 1) & 0x44444444u);
 	return r;
 }
+// The other operand's: 2, 1, 2, 2, so that no product is below 1.
+__device__ inline v8i spread_up(uint32_t w) {
+	v8i r = spread(w);
+	r[0] = (int)((w << 2) & 0x44444444u);
+	return r;
+}
+
+// What a pair's accumulators start from: two values, since a constant of one
+// use stays in the instruction, and one of more takes 16 moves each time.
+__device__ inline v16f start_lo() { return (v16f)(-0.5f); }
+__device__ inline v16f start_hi() { return (v16f)(-1.0f); }
 
 __device__ inline v16f mfma(const v8i & a, const v8i & b, const v16f & c) {
 	return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 4, 4, 0, 0, 0, 0);
 }
 
-// Bit r set where register r of lo (r < 16) or r - 16 of hi is zero.  The
-// accumulators are multiples of 0.25 below 256, so their low halves are
-// zero: two high halves make one word, and a packed minimum with 1 leaves a
-// bit of each (1.5 instructions per register; compares and carries take 2
-// and wait states).
-__device__ inline uint32_t zero_mask(const v16f & lo, const v16f & hi) {
+// Bit r set where register r of lo (r < 16) or r - 16 of hi is negative: one
+// instruction a register (zero tests of packed halves took 1.5, compares and
+// carries 2 and wait states).
+__device__ inline uint32_t subset_mask(const v16f & lo, const v16f & hi) {
 	uint32_t m = 0;
 #pragma unroll
-	for (int i = 15; i >= 0; --i) {
-		const uint32_t two = __builtin_amdgcn_perm(__float_as_uint(hi[i]), __float_as_uint(lo[i]), 0x07060302u);
-		uint32_t one;
-		asm("v_pk_min_u16 %0, %1, %2" : "=v"(one) : "v"(two), "v"(0x00010001u));
-		m = (m << 1) | one;
-	}
-	return ~m;
+	for (int i = 15; i >= 0; --i) m = __builtin_amdgcn_alignbit(m, __float_as_uint(hi[i]), 31);
+#pragma unroll
+	for (int i = 15; i >= 0; --i) m = __builtin_amdgcn_alignbit(m, __float_as_uint(lo[i]), 31);
+	return m;
 }
 
 // Wave-level ordering of LDS traffic between lanes.
@@ -73,7 +79,7 @@ __device__ inline uint32_t wave_prefix(uint32_t x) {
 	return x;
 }
 
-// A mask of 64 rows (lo's, then hi's) in zero_mask's order, for half h.
+// A mask of 64 rows (lo's, then hi's) in subset_mask's order, for half h.
 __device__ inline uint32_t half_mask(uint64_t lm, uint32_t h) {
 	if (lm == ~0ULL) return ~0u;
 	uint64_t x = (lm >> (4 * h)) & 0x0F0F0F0F0F0F0F0FULL;
