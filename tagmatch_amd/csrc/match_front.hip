@@ -68,6 +68,7 @@ k_front(front_args a) {
 	__shared__ uint32_t s_n, s_left, s_base;
 	const uint32_t tid = threadIdx.x, lane = tid & 63, n = lane & 31, h = lane >> 5;
 	const uint32_t wave = uniform(tid >> 6);
+	const uint32_t rows[2] = {row_of(0, n), row_of(1, n)};   // of 64 queries or filters, in this lane
 	const uint32_t base = blockIdx.x * a.chunk, nqc = min(a.chunk, a.nq - base);
 	const uint32_t nsub = (nqc + 63) / 64;
 	// fewer than one 64 per wave: the waves share each one's filters
@@ -88,12 +89,12 @@ k_front(front_args a) {
 		__syncthreads();
 		for (uint32_t sub = sub0; sub < nsub; sub += sub_step) {
 			const uint32_t nv = min(64u, nqc - sub * 64);
-			const uint32_t keep = half_mask(nv < 64 ? (1ULL << nv) - 1ULL : ~0ULL, h);
+			const uint32_t keep = (uint32_t)((nv < 64 ? (1ULL << nv) - 1ULL : ~0ULL) >> (32 * h));
 			v8i qv[2][3];
 #pragma unroll
 			for (uint32_t mt = 0; mt < 2; ++mt) {
 				uint32_t w[3];
-				query_words(sub * 64 + mt * 32 + n, mt * 32 + n < nv, w);
+				query_words(sub * 64 + rows[mt], rows[mt] < nv, w);
 #pragma unroll
 				for (int k = 0; k < 3; ++k) qv[mt][k] = spread_up(w[k]);
 			}
@@ -187,7 +188,7 @@ k_front(front_args a) {
 			auto load_filters = [&](uint32_t ft, uint32_t (&f)[6]) {   // past the end: the last again
 				const uint32_t * r = a.rich_words + h;
 #pragma unroll
-				for (int k = 0; k < 6; ++k) f[k] = r[(size_t)min(ft * 64 + k / 3 * 32 + n, a.n_rich - 1) * 8 + k % 3 * 2];
+				for (int k = 0; k < 6; ++k) f[k] = r[(size_t)min(ft * 64 + rows[k / 3], a.n_rich - 1) * 8 + k % 3 * 2];
 			};
 			load_filters(ft0, f);
 #pragma unroll
@@ -203,7 +204,7 @@ k_front(front_args a) {
 #pragma unroll
 				for (int k = 0; k < 6; ++k) f[k] = f1[k];
 				const uint32_t nf = min(64u, a.n_rich - ft * 64);
-				s_mask[c * MASKS + 2 * ft + h] = subset_mask(lo, hi) & half_mask(nf < 64 ? (1ULL << nf) - 1ULL : ~0ULL, h);
+				s_mask[c * MASKS + 2 * ft + h] = subset_mask(lo, hi) & (uint32_t)((nf < 64 ? (1ULL << nf) - 1ULL : ~0ULL) >> (32 * h));
 			}
 		}
 		__syncthreads();
@@ -225,11 +226,11 @@ k_front(front_args a) {
 					uint32_t at = row_prefix((uint32_t)__popc(m));
 					const uint32_t total = (uint32_t)__shfl((int)at, (int)(lane | 15), 64);
 					at -= (uint32_t)__popc(m);
-					const uint32_t f = (c0 + l) / 2 * 64 + (l & 1) * 4;
+					const uint32_t f = (c0 + l) * 32;
 					while (m) {
 						const uint32_t bit = (uint32_t)__builtin_ctz(m);
 						m &= m - 1;
-						ids[at++] = (uint16_t)(f + bit + (bit & 28u));
+						ids[at++] = (uint16_t)(f + bit);
 					}
 					wave_fence();
 					if (w < a.kw)

@@ -48,6 +48,7 @@ k_match_x(mx_args a) {
 	__shared__ uint64_t s_stat[WAVES][4];
 	const uint32_t tid = threadIdx.x, lane = tid & 63, n = lane & 31, h = lane >> 5;
 	const uint32_t wave = uniform(tid >> 6);
+	const uint32_t rows[2] = {row_of(0, n), row_of(1, n)};   // of 64 filters or queries, in this lane
 	const uint32_t kw = a.f.kw;
 	const uint32_t nq_all = a.nq_dev ? sld1(a.nq_dev) : a.nq;
 	const uint32_t epoch = a.step_vals ? sld1(a.step_vals) : a.epoch;
@@ -261,12 +262,9 @@ k_match_x(mx_args a) {
 
 		const uint32_t np = (nqs + 63) / 64;   // pairs of 32-query tiles
 		const uint32_t stride = 2 * np + 1;
-		// the queries of this lane's pair of tiles that the item has, in a
-		// mask's order
+		// the queries of this lane's half of 64 that the item has
 		uint32_t tail = ~0u;
-		if (n + 1 >= np)
-			for (uint32_t bit = 0; bit < 32; ++bit)
-				if (n * 64 + h * 4 + bit + (bit & 28u) >= nqs) tail &= ~(1u << bit);
+		if (n * 64 + h * 32 + 32 > nqs) tail = n * 64 + h * 32 < nqs ? (1u << (nqs & 31u)) - 1u : 0u;
 		const uint32_t pass = min(VISITS, MASK / stride) & ~31u;
 		for (uint32_t p0 = 0; p0 < nloc; p0 += pass) {
 			const uint32_t nb = min(pass, nloc - p0);
@@ -301,12 +299,12 @@ k_match_x(mx_args a) {
 				uint32_t any = 0;
 				uint32_t * mw = s_mask + (bt * 32 + n) * stride + h * np;
 				for (; t < t1; ++t) {
-					const uint32_t * sq = s_q + h * SUPER + t * 64 + n;
+					const uint32_t * sq = s_q + h * SUPER + t * 64;
 					v16f lo = start_lo(), hi = start_hi();
 #pragma unroll
 					for (int k = 0; k < 3; ++k) {
-						lo = mfma(spread(sq[2 * k * SUPER]), bm[k], lo);
-						hi = mfma(spread(sq[2 * k * SUPER + 32]), bm[k], hi);
+						lo = mfma(spread(sq[2 * k * SUPER + rows[0]]), bm[k], lo);
+						hi = mfma(spread(sq[2 * k * SUPER + rows[1]]), bm[k], hi);
 					}
 					const uint32_t m = nv ? subset_mask(lo, hi) : 0u;
 					if (bt * 32 + n < nb) mw[t] = m;
@@ -317,8 +315,9 @@ k_match_x(mx_args a) {
 				uint64_t av = __ballot(any != 0);
 				const uint32_t a32 = (uint32_t)av | (uint32_t)(av >> 32);
 				if (a32) {
-					bool list_it = h == 0 && ((a32 >> n) & 1);
-					if (list_it) list_it = (atomicOr(&s_seen[bt], 1u << n) >> n & 1u) == 0;
+					uint32_t seen = 0;
+					if (lane == 0) seen = atomicOr(&s_seen[bt], a32);
+					const bool list_it = h == 0 && ((a32 & ~uniform(seen)) >> n & 1u);
 					const uint64_t lb = __ballot(list_it);
 					uint32_t at = 0;
 					if (lane == 0 && lb) at = atomicAdd(&s_nvis, (uint32_t)__popcll(lb));
@@ -340,23 +339,23 @@ k_match_x(mx_args a) {
 				return lm;
 			};
 			auto load_words = [&](uint32_t b, uint32_t (&fw)[3][2]) {
-				const uint32_t * bw = a.f.blk_words + (size_t)b * BLOCK_WORDS + h * 64 + n;
+				const uint32_t * bw = a.f.blk_words + (size_t)b * BLOCK_WORDS + h * 64;
 #pragma unroll
 				for (int k = 0; k < 3; ++k)
 #pragma unroll
-					for (int mt = 0; mt < 2; ++mt) fw[k][mt] = bw[k * 128 + mt * 32];
+					for (int mt = 0; mt < 2; ++mt) fw[k][mt] = bw[k * 128 + rows[mt]];
 			};
 			// filter operands; lanes without a filter: all ones, a subset of
 			// no query but the full one
 			auto operands = [&](const uint32_t (&fw)[3][2], uint64_t lm, v8i (&fa)[3][2]) {
 #pragma unroll
 				for (int mt = 0; mt < 2; ++mt) {
-					const uint32_t dead = (lm >> (mt * 32 + n)) & 1 ? 0u : ~0u;
+					const uint32_t dead = (lm >> rows[mt]) & 1 ? 0u : ~0u;
 #pragma unroll
 					for (int k = 0; k < 3; ++k) fa[k][mt] = spread_up(fw[k][mt] | dead);
 				}
 			};
-			// hm: the filters (subset_mask's order) of the item's block `at` that
+			// hm: the filters of the item's block `at` that
 			// query qi of this lane contains
 			auto take_hits = [&](uint32_t hm, uint32_t qi, uint32_t at) {
 				const uint64_t ev = __ballot(hm != 0);
@@ -369,14 +368,14 @@ k_match_x(mx_args a) {
 				}
 				// rows known to hold every key gain nothing
 				if (MODE == MX_KEYS && a.qfull && ((s_full[qi >> 5] >> (qi & 31)) & 1u)) hm = 0;
-				const uint32_t tag = qi | (at << 18) | (h << 14);
+				const uint32_t tag = qi | (at << 18) | (h << 17);
 				uint64_t hb = __ballot(hm != 0);
 				while (hb) {
 					const uint32_t c = (uint32_t)__popcll(hb);
 					if (nlog + c > LOG) drain();
 					if (hm) {
 						const uint32_t bit = (uint32_t)__builtin_ctz(hm);
-						log[nlog + mbcnt64(hb)] = tag + ((bit + (bit & 28u)) << 12);
+						log[nlog + mbcnt64(hb)] = tag + (bit << 12);
 						hm &= hm - 1;
 					}
 					nlog += c;
@@ -413,7 +412,7 @@ k_match_x(mx_args a) {
 							lo = mfma(fa[k][0], qv[k], lo);
 							hi = mfma(fa[k][1], qv[k], hi);
 						}
-						take_hits(n < nqs ? subset_mask(lo, hi) & half_mask(lm, h) : 0u, n, at);
+						take_hits(n < nqs ? subset_mask(lo, hi) & (uint32_t)(lm >> (32 * h)) : 0u, n, at);
 					}
 				}
 			} else {
@@ -430,14 +429,14 @@ k_match_x(mx_args a) {
 					const uint64_t lm = valid_lanes(vis, block_of(at));
 					v8i fa[3][2];
 					operands(fw, lm, fa);
-					const uint32_t keep = half_mask(lm, h);
+					const uint32_t keep = (uint32_t)(lm >> (32 * h));
 					if (v + WAVES < nvis) {
 						next = uniform(s_vis[v + WAVES]);
 						load_words(block_of(p0 + (next & ~PARTIAL)), fw);
 					}
 					// candidates as a list: each lane writes those of its mask
 					// behind the lanes before it, LIST at a time
-					const uint32_t qb = n * 64 + h * 4;
+					const uint32_t qb = n * 64 + h * 32;
 					m &= tail;
 					uint32_t pos = wave_prefix((uint32_t)__popc(m));
 					uint32_t left = (uint32_t)__builtin_amdgcn_readlane((int)pos, 63);
@@ -449,7 +448,7 @@ k_match_x(mx_args a) {
 							if (m != 0 && pos < LIST) {
 								const uint32_t bit = (uint32_t)__builtin_ctz(m);
 								m &= m - 1;
-								list[pos++] = (uint16_t)(qb + bit + (bit & 28u));
+								list[pos++] = (uint16_t)(qb + bit);
 							}
 						}
 						const uint32_t cnt = min(left, LIST);

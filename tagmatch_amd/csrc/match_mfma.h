@@ -12,6 +12,8 @@
 //
 // Lane l = 32 h + n holds words 2 k + h (k = 0, 1, 2) of row or column n of
 // an operand, and of a result column n and the rows 8 (i / 4) + 4 h + i % 4.
+// Of 64 rows in two tiles, row_of says which each lane holds, so that bit b
+// of a lane's subset_mask is row 32 h + b.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -47,16 +49,27 @@ __device__ inline v16f mfma(const v8i & a, const v8i & b, const v16f & c) {
 	return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 4, 4, 0, 0, 0, 0);
 }
 
-// Bit r set where register r of lo (r < 16) or r - 16 of hi is negative: one
-// instruction a register (zero tests of packed halves took 1.5, compares and
-// carries 2 and wait states).
+// The signs of both accumulators, one bit each.  A conversion to 6-bit floats
+// takes all 32 at once and leaves their signs 6 bits apart: those of words 0
+// to 2 at different odd bits, those of words 3 to 5 at the same ones.  88
+// cycles of the vector unit; a funnel shift per register took 128, zero
+// tests of packed halves 192.
+typedef uint32_t v6u __attribute__((ext_vector_type(6)));
 __device__ inline uint32_t subset_mask(const v16f & lo, const v16f & hi) {
-	uint32_t m = 0;
-#pragma unroll
-	for (int i = 15; i >= 0; --i) m = __builtin_amdgcn_alignbit(m, __float_as_uint(hi[i]), 31);
-#pragma unroll
-	for (int i = 15; i >= 0; --i) m = __builtin_amdgcn_alignbit(m, __float_as_uint(lo[i]), 31);
-	return m;
+	constexpr uint32_t A = 0x20820820u, B = 0x08208208u, ODD = 0xAAAAAAAAu;
+	const v6u r = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(lo, hi, 1.0f);
+	const uint32_t x = (A & r[0]) | (~A & ((B & r[1]) | (~B & r[2])));
+	const uint32_t y = (A & r[3]) | (~A & ((B & r[4]) | (~B & r[5])));
+	return (ODD & x) | (~ODD & (y >> 1));
+}
+// Its bit of register i of lo (mt = 0) or hi (1): the conversion alternates
+// between them.
+__host__ __device__ constexpr uint32_t mask_bit(uint32_t mt, uint32_t i) {
+	return (6 * ((2 * i + mt) % 16) + 5) % 32 - (2 * i + mt) / 16;
+}
+// The row, of 64, that lane n holds of tile mt.
+__device__ inline uint32_t row_of(uint32_t mt, uint32_t n) {
+	return 32 * (n / 4 % 2) + mask_bit(mt, n / 8 * 4 + n % 4);
 }
 
 // Wave-level ordering of LDS traffic between lanes.
@@ -77,15 +90,6 @@ __device__ inline uint32_t wave_prefix(uint32_t x) {
 	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);   // row_bcast:15
 	x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);   // row_bcast:31
 	return x;
-}
-
-// A mask of 64 rows (lo's, then hi's) in subset_mask's order, for half h.
-__device__ inline uint32_t half_mask(uint64_t lm, uint32_t h) {
-	if (lm == ~0ULL) return ~0u;
-	uint64_t x = (lm >> (4 * h)) & 0x0F0F0F0F0F0F0F0FULL;
-	x = (x | (x >> 4)) & 0x00FF00FF00FF00FFULL;
-	x = (x | (x >> 8)) & 0x0000FFFF0000FFFFULL;
-	return (uint32_t)x | (uint32_t)(x >> 16);
 }
 
 } // namespace tmx
