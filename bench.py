@@ -932,7 +932,7 @@ def main():
     for b in hbufs + pbufs:
         b.close()
 
-    # ---- roofline of the dominant kernel (k_match_q) and of the step
+    # ---- roofline of the dominant kernel (k_match_x) and of the step
     sizes = np.diff(part_off).astype(np.float64)
     batches = np.ceil(counts / args.batch)
     bytes_bruteforce = float(np.sum(batches * 24.0 * sizes) + 24.0 * counts.sum())
@@ -948,7 +948,7 @@ def main():
     kernel_s = kernel_ms / 1e3
     achieved = (traffic / kernel_s / 1e9) if traffic else alg_bytes / kernel_s / 1e9
     roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": "k_match_q", "kernel_ms": kernel_ms,
+            "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": "k_match_x", "kernel_ms": kernel_ms,
             "alg_bytes": alg_bytes, "alg_frac": alg_bytes / kernel_s / 1e9 / HBM_PEAK_GBS,
             "measured_valu_frac": (prof["valu_insts"] * 64 / kernel_s / 1e12 / VALU_PEAK_TOPS)
             if prof.get("valu_insts") else None,

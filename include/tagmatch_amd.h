@@ -414,13 +414,13 @@ int tm_ring_lookup_counts(tm_ring * ring, uint32_t * counts, uint32_t n_parts);
 /* No-allocation match.  No counterpart in the reference: it is for callers
  * that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  It runs the persistent
- * KEY_BITMAP step of a ring -- lookup, rich-filter pass, compacted match --
+ * KEY_BITMAP step of a ring -- lookup, rich-filter pass, match --
  * over nq queries already in device memory (dev_queries: nq x 8 words, the
  * 6 filter words and 2 pad words, the layout of tm_ring_query_buffer) and
  * writes their key bitmap rows to device memory (dev_rows: nq x
  * ceil(K/32) words), on `stream` (a hipStream_t; NULL: the default stream),
  * and returns when they are written.  It allocates nothing: its working
- * buffers live in a fixed static device array of 0.88 MiB per GPU,
+ * buffers live in a fixed static device array of 2.9 MiB per GPU,
  * which bounds nq by TM_STATIC_MAX_QUERIES and the FIB's partitions by
  * TM_STATIC_MAX_PARTS (larger sizes: TM_ERR_INVALID).  Calls on one GPU share
  * that array: calls that overlap on one GPU (from several threads) race.

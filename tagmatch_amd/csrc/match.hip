@@ -54,7 +54,8 @@ constexpr uint32_t WSEG_BASE = 64;          // block weight: fixed part, in unit
 constexpr uint32_t WSEG_MAX_TILES = 256;    // persistent: tiles up to which segments are cut by weight
 constexpr uint32_t PRICE_SAMPLE_TILES = 1024;  // cost model: tiles priced when only totals are needed
 constexpr uint32_t NO_QUERY = 0xFFFFFFFFu;
-constexpr uint64_t ROWS_LDS_MAX_WORK = 80000000;   // queries x blocks of steps whose rows are built in local memory
+constexpr uint32_t ROWS_LDS_MAX_BLOCKS = 2048;     // rows are built in local memory: blocks of the table, or
+constexpr uint64_t ROWS_LDS_MAX_WORK = 80000000;   // queries x blocks, at most
 constexpr uint64_t HCNT_MAX = 1ull << 26;     // hit-list steps: counts of (segment, query), at most
 constexpr uint32_t COPY_MAX = 4096;            // queries that a step's first kernel takes from host memory, at most
 constexpr uint32_t OFF_MAX = 4096;             // result lists written to host memory with the step: queries, values
@@ -1503,8 +1504,8 @@ mx_shape hits_shape(const tm_ring * r, uint32_t nq, uint32_t resident) {
 // prefix sums place them, and a second pass writes them.  The match runs
 // twice, but without a hit list in between, whose entries (8 bytes written
 // and read twice, two contended global atomics each) cost more: 1024
-// queries at 10M filters, 7.4M hits, took 1.1 ms to match and 3.4 ms to
-// group from a list.
+// queries at 10M filters, 7.4M hits, take 0.66 ms; from a list 1.1 ms to
+// match and 3.4 ms to group.
 int enqueue_values(tm_ring * r, mx_args a, uint32_t rows, uint32_t grid, bool events) {
 	hipStream_t s = r->s;
 	const bool ids = r->cfg.mode == TM_MODE_HITS;
@@ -1576,13 +1577,15 @@ int enqueue_matrix(tm_ring * r, uint32_t nq, bool events) {
 		return enqueue_values(r, a, h.nseg, a.resident, events);
 	}
 	// Rows in local memory where the match sets most of their bits: without
-	// a rich-filter pass, or in small steps where no rich filter holds every
-	// key.  In larger ones more queries per item win.  Both sides measured
-	// (filters, queries: local, HBM): 104k, 4.9k: 0.40, 0.49 ms; 101k, 44k:
-	// 1.08, 1.32; 402k, 13k: 0.51, 0.48; 158k, 612k: 14.9, 13.3; 1M, 100k:
-	// 1.73, 1.25.
+	// a rich-filter pass, or where no rich filter holds every key and the
+	// table or the step is small.  In larger ones more queries per item win.
+	// Both sides measured (blocks, queries: local, HBM): 735, 250k: 1.34,
+	// 1.65 ms; 1997, 44k: 0.66, 0.76; 1997, 700k: 9.0, 8.7; 2910, 10k: 0.31,
+	// 0.26; 2910, 700k: 12.6, 10.2; 6.9k, 13k: 0.39, 0.38; 6.9k, 40k: 1.08,
+	// 0.93; 17k, 5k: 0.091, 0.092; 17k, 100k: 1.13, 0.62.
 	const bool sparse = !rich_pass || (compact && r->fib->n_rich_full == 0 &&
-									   (uint64_t)nq * r->fib->n_blocks <= ROWS_LDS_MAX_WORK);
+									   (r->fib->n_blocks <= ROWS_LDS_MAX_BLOCKS ||
+										(uint64_t)nq * r->fib->n_blocks <= ROWS_LDS_MAX_WORK));
 	const int mode = sparse && r->kw <= MX_LDS_KW && r->kw > 0 ? MX_KEYS_LDS : MX_KEYS;
 	mx_args a = matrix_args(r, mode);
 	a.nq = nq;

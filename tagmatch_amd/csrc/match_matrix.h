@@ -29,8 +29,8 @@ constexpr int MX_WAVES = 8;             // waves per workgroup
 // more queries per item mean more candidates for each block whose filters
 // are loaded and spread.  Rows in local memory (48 KB for 192 queries at
 // 2048 keys) leave room for fewer: match times of the uneven units (541k
-// queries) 4.1 ms with 192, 4.7 with 128, 4.2 with 448 and one workgroup of
-// 16 waves per CU.
+// queries) 3.06 ms with 192, 3.73 with 128; with 448 and one workgroup of 16
+// waves per CU 4 % more than with 192.
 __host__ __device__ constexpr uint32_t mx_super(int mode) {
 	return mode == MX_KEYS ? 2048u : mode == MX_KEYS_LDS ? 192u : 1536u;
 }
@@ -43,7 +43,7 @@ __host__ __device__ constexpr uint32_t mx_visits(int mode) { return mode == MX_K
 // nsuper + super, supers of sq queries, segments of about seg blocks: every
 // nseg-th tile of 32, so that the blocks with many matches, which lie
 // together, are spread over all segments (against runs of blocks: 100k
-// queries on 1M filters 0.74 and 0.63 ms, the uneven units 3.95 and 3.52).
+// queries on 1M filters 0.63 and 0.74 ms, the uneven units 3.52 and 3.95).
 // Work for at most five items of 64 blocks per workgroup: one item each (10M
 // filters: 1000 queries 31 us against 52, 10k 75 against 85; 1M filters, 16
 // queries 13 against 17 for two rounds).  Otherwise 128 blocks: between 64

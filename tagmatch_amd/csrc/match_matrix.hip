@@ -29,6 +29,27 @@ __device__ inline uint32_t inline_keys(uint64_t kv) {
 	return n;
 }
 
+// The match.  A workgroup takes an item: up to SUPER queries, their inverted
+// words in local memory, and a segment's blocks of 64 filters.
+//
+//   Candidates: the blocks' AND masks (columns) against the queries (rows): a
+//   bit per pair, 6 instructions of the matrix unit for 64 x 32 pairs, and
+//   the blocks that have any listed.
+//   Tests: a wave takes a listed block, spreads its filters (rows) once, and
+//   tests them against its candidates (columns), 32 at a time: 6 matrix
+//   instructions and about 60 others for 2048 pairs.
+//   Hits go to a log in local memory, which the wave empties 64 at a time.
+//
+// Bound by the vector unit, which spreads the operands, turns accumulators
+// into masks and logs hits: where every match is enumerated (1M queries, 10M
+// filters, 146 ms, 48 G matches/s) it is busy 74 % of the time and the matrix
+// unit 37 %; with the full-row exit (1.02 ms) it is busy 52 %, and the waves
+// wait for blocks and keys 57 % of theirs.  One query at a time against 64
+// filters on the vector unit took 556 and 1.98 ms: each test read 24 bytes
+// of local memory per lane, 12 of its cycles, and 7 instructions.
+//
+// Two workgroups of eight waves per CU: 128 registers; with 96 (five waves a
+// SIMD) the operands spill (1.58 ms became 2.12).
 template <int MODE>
 __global__ void __launch_bounds__(MX_WAVES * 64, 4)
 k_match_x(mx_args a) {
