@@ -46,7 +46,9 @@ __host__ __device__ constexpr uint32_t mx_visits(int mode) { return mode == MX_K
 // queries on 1M filters 0.63 and 0.74 ms, the uneven units 3.52 and 3.95).
 // Work for at most five items of 64 blocks per workgroup: one item each (10M
 // filters: 1000 queries 31 us against 52, 10k 75 against 85; 1M filters, 16
-// queries 13 against 17 for two rounds).  Otherwise 128 blocks: between 64
+// queries 13 against 17 for two rounds).  One super: as many items of up to
+// 512 blocks (43.6M filters: 1000 queries 39 us, 83 with 128 blocks, 16k 99
+// and 135).  Otherwise 128 blocks: between 64
 // and 256 it is the fastest or within 4 % of it (1M filters, 300k queries,
 // for 64, 128, 256: 1.58, 1.52, 1.65 ms; 10M, 1M queries: 1.00, 0.98, 1.00;
 // 65k without the full-row exit: 11.7, 11.4, 11.4).  seg_min: least blocks
@@ -63,9 +65,10 @@ __host__ __device__ inline mx_shape mx_shape_of(int mode, uint32_t nq, uint32_t 
 	while (sq > 256 && (uint64_t)((nq + sq - 1) / sq) * ((nblk + 63) / 64) < 4ull * resident) sq = (sq / 2 + 63) & ~63u;
 	const uint32_t nsuper = (nq + sq - 1) / sq;
 	uint32_t seg = 128;
-	if ((uint64_t)nsuper * ((nblk + 63) / 64) <= 5ull * resident) {
-		const uint64_t per = ((uint64_t)nblk * nsuper + resident - 1) / resident;
-		seg = per < 32 ? 32u : (uint32_t)(per + 31) & ~31u;
+	if (nsuper == 1 || (uint64_t)nsuper * ((nblk + 63) / 64) <= 5ull * resident) {
+		const uint64_t per = ((uint64_t)nblk * nsuper + resident - 1) / resident;   // blocks of a workgroup
+		const uint64_t rounds = (per + 511) / 512;
+		seg = per == 0 ? 32u : (uint32_t)((per + rounds - 1) / rounds + 31) & ~31u;
 	}
 	if (seg < seg_min) seg = seg_min;
 	if (seg_fixed) seg = seg_fixed;
