@@ -69,7 +69,7 @@ k_match_x(mx_args a) {
 	__shared__ uint64_t s_stat[WAVES][4];
 	const uint32_t tid = threadIdx.x, lane = tid & 63, n = lane & 31, h = lane >> 5;
 	const uint32_t wave = uniform(tid >> 6);
-	const uint32_t rows[2] = {row_of(0, n), row_of(1, n)};   // of 64 filters or queries, in this lane
+	const uint32_t frow[2] = {near_row(0, n), near_row(1, n)};   // a block's filters in this lane
 	const uint32_t kw = a.f.kw;
 	const uint32_t nq_all = a.nq_dev ? sld1(a.nq_dev) : a.nq;
 	const uint32_t epoch = a.step_vals ? sld1(a.step_vals) : a.epoch;
@@ -162,14 +162,14 @@ k_match_x(mx_args a) {
 		uint32_t * log = s_log[wave];
 		uint16_t * list = s_list[wave];
 		uint32_t nlog = 0;
-		// The staged hits (query, lane and block of each, 64 at a time): their
+		// The staged hits (query, mask bit and block of each, 64 at a time): their
 		// keys into the queries' rows, or their values counted or written.
 		auto drain = [&]() {
 			for (uint32_t base = 0; base < nlog; base += 64) {
 				const bool mine = base + lane < nlog;
 				const uint32_t e = mine ? log[base + lane] : 0u;
 				const uint32_t qi = e & 0xFFFu, ql = q0 + qi;
-				const uint32_t slot = block_of(e >> 18) * 64 + ((e >> 12) & 63u);
+				const uint32_t slot = block_of(e >> 18) * 64 + near_bit((e >> 12) & 31u, (e >> 17) & 1u);
 				if (MODE == MX_WRITE) {
 					if (mine) {
 						const uint64_t at = a.off[ql] + atomicAdd(&s_cnt[qi], 1u);
@@ -324,8 +324,8 @@ k_match_x(mx_args a) {
 					v16f lo = start_lo(), hi = start_hi();
 #pragma unroll
 					for (int k = 0; k < 3; ++k) {
-						lo = mfma(spread(sq[2 * k * SUPER + rows[0]]), bm[k], lo);
-						hi = mfma(spread(sq[2 * k * SUPER + rows[1]]), bm[k], hi);
+						lo = mfma(spread(sq[2 * k * SUPER + row_of(0, n)]), bm[k], lo);
+						hi = mfma(spread(sq[2 * k * SUPER + row_of(1, n)]), bm[k], hi);
 					}
 					const uint32_t m = nv ? subset_mask(lo, hi) : 0u;
 					if (bt * 32 + n < nb) mw[t] = m;
@@ -364,14 +364,14 @@ k_match_x(mx_args a) {
 #pragma unroll
 				for (int k = 0; k < 3; ++k)
 #pragma unroll
-					for (int mt = 0; mt < 2; ++mt) fw[k][mt] = bw[k * 128 + rows[mt]];
+					for (int mt = 0; mt < 2; ++mt) fw[k][mt] = bw[k * 128 + frow[mt]];
 			};
 			// filter operands; lanes without a filter: all ones, a subset of
 			// no query but the full one
 			auto operands = [&](const uint32_t (&fw)[3][2], uint64_t lm, v8i (&fa)[3][2]) {
 #pragma unroll
 				for (int mt = 0; mt < 2; ++mt) {
-					const uint32_t dead = (lm >> rows[mt]) & 1 ? 0u : ~0u;
+					const uint32_t dead = (lm >> frow[mt]) & 1 ? 0u : ~0u;
 #pragma unroll
 					for (int k = 0; k < 3; ++k) fa[k][mt] = spread_up(fw[k][mt] | dead);
 				}
@@ -433,7 +433,7 @@ k_match_x(mx_args a) {
 							lo = mfma(fa[k][0], qv[k], lo);
 							hi = mfma(fa[k][1], qv[k], hi);
 						}
-						take_hits(n < nqs ? subset_mask(lo, hi) & (uint32_t)(lm >> (32 * h)) : 0u, n, at);
+						take_hits(n < nqs ? subset_mask(lo, hi) & near_mask(lm, h) : 0u, n, at);
 					}
 				}
 			} else {
@@ -450,7 +450,7 @@ k_match_x(mx_args a) {
 					const uint64_t lm = valid_lanes(vis, block_of(at));
 					v8i fa[3][2];
 					operands(fw, lm, fa);
-					const uint32_t keep = (uint32_t)(lm >> (32 * h));
+					const uint32_t keep = near_mask(lm, h);
 					if (v + WAVES < nvis) {
 						next = uniform(s_vis[v + WAVES]);
 						load_words(block_of(p0 + (next & ~PARTIAL)), fw);
