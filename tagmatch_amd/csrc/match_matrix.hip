@@ -438,23 +438,12 @@ k_match_x(mx_args a) {
 				}
 			} else {
 				// A block's filters (rows) against its candidates (columns),
-				// 32 at a time; the next block's words are loaded meanwhile.
-				uint32_t fw[3][2], next = 0;
-				if (wave < nvis) {
-					next = uniform(s_vis[wave]);
-					load_words(block_of(p0 + (next & ~PARTIAL)), fw);
-				}
+				// 32 at a time.
 				for (uint32_t v = wave; v < nvis; v += WAVES) {
-					const uint32_t vis = next, bn = vis & ~PARTIAL, at = p0 + bn;
+					const uint32_t vis = uniform(s_vis[v]), bn = vis & ~PARTIAL, at = p0 + bn;
+					uint32_t fw[3][2];
+					load_words(block_of(at), fw);   // (on their way while the list is written)
 					uint32_t m = n < np ? s_mask[bn * stride + h * np + n] : 0u;
-					const uint64_t lm = valid_lanes(vis, block_of(at));
-					v8i fa[3][2];
-					operands(fw, lm, fa);
-					const uint32_t keep = near_mask(lm, h);
-					if (v + WAVES < nvis) {
-						next = uniform(s_vis[v + WAVES]);
-						load_words(block_of(p0 + (next & ~PARTIAL)), fw);
-					}
 					// candidates as a list: each lane writes those of its mask
 					// behind the lanes before it, LIST at a time
 					const uint32_t qb = n * 64 + h * 32;
@@ -464,7 +453,7 @@ k_match_x(mx_args a) {
 					pos -= (uint32_t)__popc(m);
 					w_test += left;
 					w_visit += left != 0;
-					while (left) {
+					auto write_list = [&]() {
 						while (__ballot(m != 0 && pos < LIST)) {
 							if (m != 0 && pos < LIST) {
 								const uint32_t bit = (uint32_t)__builtin_ctz(m);
@@ -472,24 +461,44 @@ k_match_x(mx_args a) {
 								list[pos++] = (uint16_t)(qb + bit);
 							}
 						}
+					};
+					write_list();
+					const uint64_t lm = valid_lanes(vis, block_of(at));
+					v8i fa[3][2];
+					operands(fw, lm, fa);
+					const uint32_t keep = near_mask(lm, h);
+					while (left) {
 						const uint32_t cnt = min(left, LIST);
 						left -= cnt;
 						pos -= LIST;   // only of lanes with more to list
 						wave_fence();
+						// the words of the next 32 are read meanwhile
+						auto read_words = [&](uint32_t qi, uint32_t (&w)[3]) {
+#pragma unroll
+							for (int k = 0; k < 3; ++k) w[k] = s_q[(2 * k + h) * SUPER + qi];
+						};
+						uint32_t qi = list[n < cnt ? n : 0u], w[3];
+						read_words(qi, w);
 						for (uint32_t base = 0; base < cnt; base += 32) {
 							const bool valid = base + n < cnt;
-							const uint32_t qi = list[valid ? base + n : base];
+							const uint32_t qi1 = list[base + 32 + n < cnt ? base + 32 + n : base];
+							uint32_t w1[3];
+							read_words(qi1, w1);
 							v16f lo = start_lo(), hi = start_hi();
 #pragma unroll
 							for (int k = 0; k < 3; ++k) {
-								const v8i qv = spread(s_q[(2 * k + h) * SUPER + qi]);
+								const v8i qv = spread(w[k]);
 								lo = mfma(fa[k][0], qv, lo);
 								hi = mfma(fa[k][1], qv, hi);
 							}
 							const uint32_t hm = subset_mask(lo, hi);
 							take_hits(valid ? hm & keep : 0u, qi, at);
+							qi = qi1;
+#pragma unroll
+							for (int k = 0; k < 3; ++k) w[k] = w1[k];
 						}
 						wave_fence();
+						if (left) write_list();
 					}
 				}
 			}
