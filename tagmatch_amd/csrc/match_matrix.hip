@@ -37,19 +37,22 @@ __device__ inline uint32_t inline_keys(uint64_t kv) {
 //   the blocks that have any listed.
 //   Tests: a wave takes a listed block, spreads its filters (rows) once, and
 //   tests them against its candidates (columns), 32 at a time: 6 matrix
-//   instructions and about 60 others for 2048 pairs.
+//   instructions, a conversion and about 40 others for 2048 pairs.
 //   Hits go to a log in local memory, which the wave empties 64 at a time.
 //
 // Bound by the vector unit, which spreads the operands, turns accumulators
 // into masks and logs hits: where every match is enumerated (1M queries, 10M
-// filters, 146 ms, 48 G matches/s) it is busy 74 % of the time and the matrix
-// unit 37 %; with the full-row exit (1.02 ms) it is busy 52 %, and the waves
-// wait for blocks and keys 57 % of theirs.  One query at a time against 64
+// filters, 139 ms, 50 G matches/s) it is busy 79 % of the time and the matrix
+// unit 40 %; with the full-row exit (0.95 ms) it is busy 57 %, and the waves
+// wait for blocks and keys 55 % of theirs.  One query at a time against 64
 // filters on the vector unit took 556 and 1.98 ms: each test read 24 bytes
 // of local memory per lane, 12 of its cycles, and 7 instructions.
 //
 // Two workgroups of eight waves per CU: 128 registers; with 96 (five waves a
-// SIMD) the operands spill (1.58 ms became 2.12).
+// SIMD) the operands spill (a third slower).  A block's words are loaded
+// before its candidates are listed, and the next 32 queries' words during the
+// tests of the last (9.39 and 9.19 ms for 65k queries against all matches;
+// loaded a whole block ahead, they went to scratch memory: 9.68).
 template <int MODE>
 __global__ void __launch_bounds__(MX_WAVES * 64, 4)
 k_match_x(mx_args a) {
