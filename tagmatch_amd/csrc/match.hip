@@ -1372,9 +1372,33 @@ void ensure_weights(tm_ring * r, hipStream_t s) {
 int grow_u32(uint32_t ** p, uint64_t & cap, uint64_t need) {
 	if (need <= cap && *p) return TM_OK;
 	dfree(*p);
+	cap = 0;
 	uint64_t n = std::max<uint64_t>(need, 1);
 	TM_CHECK(dalloc(p, n));
 	cap = n;
+	return TM_OK;
+}
+
+void drop_graph(tm_ring * r) {
+	for (auto & g : r->graphs) (void)hipGraphExecDestroy(g.exec);
+	r->graphs.clear();
+}
+
+// The same for a buffer whose address captured steps hold: they go before it
+// does, whoever grows it.
+int grow_captured(tm_ring * r, uint32_t ** p, uint64_t & cap, uint64_t need) {
+	if (need <= cap && *p) return TM_OK;
+	drop_graph(r);
+	return grow_u32(p, cap, need);
+}
+
+// A hit list of `cap` entries in place of the ring's.
+int grow_hits(tm_ring * r, uint64_t cap) {
+	drop_graph(r);
+	dfree(r->d_hits);
+	r->hit_cap = 0;
+	TM_CHECK(dalloc(&r->d_hits, cap));
+	r->hit_cap = cap;
 	return TM_OK;
 }
 
@@ -2032,7 +2056,7 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 	a.n_units = n;
 	const uint32_t grid = (uint32_t)std::min<uint64_t>(resident, std::max<uint64_t>(items, 1));
 	if (!keys) {
-		TM_CHECK(grow_u32(&r->d_hcnt, r->hcnt_cap, (uint64_t)max_nseg * nq));
+		TM_CHECK(grow_captured(r, &r->d_hcnt, r->hcnt_cap, (uint64_t)max_nseg * nq));
 		fill_u32(r->d_hcnt, 0, (uint64_t)max_nseg * nq, s);   // units have different numbers of segments
 		TM_CHECK(enqueue_values(r, a, max_nseg, grid, true));
 		TM_HIP(hipStreamSynchronize(s));   // tab and pre are pageable host memory
@@ -2169,11 +2193,6 @@ int enqueue_step(tm_ring * r, bool allow_graph) {
 	return TM_OK;
 }
 
-void drop_graph(tm_ring * r) {
-	for (auto & g : r->graphs) (void)hipGraphExecDestroy(g.exec);
-	r->graphs.clear();
-}
-
 // Price the submission's (query tile, partition) units with the cost model:
 // order tiles longest-first (dealt round-robin over the NQUEUE queues so
 // every queue starts with heavy tiles) and grow result buffers to the
@@ -2215,7 +2234,7 @@ int price_submission(tm_ring * r, uint32_t nq) {
 		r->trows_cap = rows;
 	}
 	if (n_tiles > r->tiles_cap) {
-		const bool graph_uses = r->d_iorder != nullptr;
+		if (r->d_iorder) drop_graph(r);
 		dfree(r->d_tcost);
 		dfree(r->d_thits);
 		dfree(r->d_tkeys);
@@ -2226,7 +2245,6 @@ int price_submission(tm_ring * r, uint32_t nq) {
 		TM_CHECK(dalloc(&r->d_tkeys, n_tiles));
 		TM_CHECK(dalloc(&r->d_iorder, n_tiles));
 		r->tiles_cap = n_tiles;
-		if (graph_uses) drop_graph(r);
 	}
 	launch_unit_features_tiles(r->fib->view(), r->d_q, nq_priced, nqt, n_tiles, r->d_tfeat, s);
 	TM_CHECK(mlp_infer(r->model, r->d_tfeat, (uint32_t)rows, r->d_tpred, s));
@@ -2290,18 +2308,9 @@ int price_submission(tm_ring * r, uint32_t nq) {
 		} else {
 			slots = (uint64_t)(total * margin) + 4096;
 			results = r->cfg.mode == TM_MODE_KEYS_ALL ? (uint64_t)(total_keys * margin) + 4096 : slots;
-			if (slots > r->hit_cap) {
-				dfree(r->d_hits);
-				r->hit_cap = 0;
-				TM_CHECK(dalloc(&r->d_hits, slots));
-				r->hit_cap = slots;
-				drop_graph(r);
-			}
+			if (slots > r->hit_cap) TM_CHECK(grow_hits(r, slots));
 		}
-		if (results > r->val_cap) {
-			TM_CHECK(grow_u32(&r->d_vals, r->val_cap, results));
-			drop_graph(r);
-		}
+		if (results > r->val_cap) TM_CHECK(grow_captured(r, &r->d_vals, r->val_cap, results));
 	}
 	r->st.model_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 	return TM_OK;
@@ -2359,11 +2368,7 @@ int submit_common(tm_ring * r, uint32_t nq) {
 	if (!r->units_mode && !keyrows(r->cfg) && r->cfg.schedule == TM_SCHED_PERSISTENT && !r->cfg.log_units) {
 		const mx_args a = matrix_args(r, MX_COUNT);
 		const mx_shape h = hits_shape(r, r->run_nq, a.resident);
-		const uint64_t need = (uint64_t)h.nseg * r->run_nq;
-		if (need > r->hcnt_cap) {
-			drop_graph(r);
-			TM_CHECK(grow_u32(&r->d_hcnt, r->hcnt_cap, need));
-		}
+		TM_CHECK(grow_captured(r, &r->d_hcnt, r->hcnt_cap, (uint64_t)h.nseg * r->run_nq));
 	}
 	int rc = enqueue_step(r, true);
 	if (rc != TM_OK) return rc;
@@ -2568,20 +2573,16 @@ int tm_wait(tm_ring * r, tm_status * st) {
 				again = true;
 			}
 			if (!keyrows(r->cfg) && slots > r->hit_cap) {
-				dfree(r->d_hits);
-				uint64_t cap = slots + slots / 4 + 1024;
-				TM_CHECK(dalloc(&r->d_hits, cap));
-				r->hit_cap = cap;
+				TM_CHECK(grow_hits(r, slots + slots / 4 + 1024));
 				// a matrix step keeps no hit list: its values are whole
 				if (r->n_wgstat) {
 					r->hits_grown = true;
-					drop_graph(r);   // holds the old buffer
 				} else {
 					again = true;
 				}
 			}
 			if (results > r->val_cap) {
-				TM_CHECK(grow_u32(&r->d_vals, r->val_cap, results + results / 4 + 1024));
+				TM_CHECK(grow_captured(r, &r->d_vals, r->val_cap, results + results / 4 + 1024));
 				again = true;
 			}
 			if (!again) break;
