@@ -1140,6 +1140,8 @@ struct tm_ring {
 	float rho_l2 = -1.f;            // log2 mean bit density of the last host queries
 	uint2 * d_hits = nullptr;
 	uint64_t hit_cap = 0;
+	uint64_t hit_limit = 0;        // the most hits reported within capacity, where that is more: steps
+	                               // of the matrix kernel keep no hit list
 	uint32_t * d_qcount = nullptr;
 	uint64_t * d_off = nullptr;
 	unsigned long long * d_qcur = nullptr;
@@ -1158,7 +1160,7 @@ struct tm_ring {
 	uint32_t copy_nq = 0;          // queries the next step takes from h_q
 	uint32_t * d_hcnt = nullptr;   // hit-list steps: values per segment and query
 	uint64_t hcnt_cap = 0;
-	bool hits_grown = false;       // the last step had more hits than the ring's hit capacity
+	bool hits_over = false;        // the last step had more hits than that, and kept no hit list
 	uint32_t * d_log = nullptr;
 	uint64_t log_cap = 0;
 	uint32_t * d_stage = nullptr;     // plain: key bitmap rows of one unit's batch
@@ -1202,6 +1204,7 @@ struct tm_ring {
 		const uint32_t * slot_epoch = nullptr;
 		bool weighted = false;       // reads the block weights, refreshed outside the graph
 		bool qfull_valid = false;    // writes d_qfull
+		uint32_t n_wgstat = 0;       // its statistics' records
 	};
 	bool capturing = false;          // enqueue_persistent runs inside a stream capture
 	bool qfull_valid = false;        // the last step wrote d_qfull: a set flag means a full row
@@ -2174,11 +2177,13 @@ int enqueue_step(tm_ring * r, bool allow_graph) {
 			e.slot_epoch = r->fib->slot_epoch;
 			e.weighted = r->step_weighted;
 			e.qfull_valid = r->qfull_valid;
+			e.n_wgstat = r->n_wgstat;
 			r->graphs.push_back(e);
 			ge = &r->graphs.back();
 		}
 		if (ge->weighted) ensure_weights(r, r->s);
 		r->qfull_valid = ge->qfull_valid;
+		r->n_wgstat = ge->n_wgstat;
 		TM_HIP(hipGraphLaunch(ge->exec, r->s));
 		r->match_events = false;
 	} else if (persistent) {
@@ -2308,7 +2313,10 @@ int price_submission(tm_ring * r, uint32_t nq) {
 		} else {
 			slots = (uint64_t)(total * margin) + 4096;
 			results = r->cfg.mode == TM_MODE_KEYS_ALL ? (uint64_t)(total_keys * margin) + 4096 : slots;
-			if (slots > r->hit_cap) TM_CHECK(grow_hits(r, slots));
+			if (!r->use_iorder && !r->cfg.log_units && r->cfg.mode == TM_MODE_HITS)
+				r->hit_limit = std::max(r->hit_limit, slots);
+			else if (slots > r->hit_cap)
+				TM_CHECK(grow_hits(r, slots));
 		}
 		if (results > r->val_cap) TM_CHECK(grow_captured(r, &r->d_vals, r->val_cap, results));
 	}
@@ -2350,7 +2358,7 @@ int submit_common(tm_ring * r, uint32_t nq) {
 	r->st = tm_status();
 	r->last_nq = nq;
 	r->retries = 0;
-	r->hits_grown = false;
+	r->hits_over = false;
 	r->epoch = r->fib->epoch;   // the inserts this submission sees
 	TM_CHECK(sync_fib(r));
 	TM_CHECK(ensure_capacity(r));
@@ -2572,14 +2580,17 @@ int tm_wait(tm_ring * r, tm_status * st) {
 				TM_CHECK(grow_u32(&r->d_list, r->list_cap, pairs + pairs / 4 + 1024));
 				again = true;
 			}
-			if (!keyrows(r->cfg) && slots > r->hit_cap) {
-				TM_CHECK(grow_hits(r, slots + slots / 4 + 1024));
-				// a matrix step keeps no hit list: its values are whole
-				if (r->n_wgstat) {
-					r->hits_grown = true;
-				} else {
-					again = true;
-				}
+			const uint64_t room = slots + slots / 4 + 1024;
+			if (!keyrows(r->cfg) && r->n_wgstat == 0 && slots > r->hit_cap) {
+				TM_CHECK(grow_hits(r, room));
+				again = true;
+			} else if (!keyrows(r->cfg) && r->n_wgstat && slots > std::max(r->hit_cap, r->hit_limit)) {
+				// no hit list: the values are whole.  KEYS_ALL records its long
+				// key lists in the list's memory, and writes those that have no
+				// room there all the same, so a failure here is none of the step's
+				r->hits_over = true;
+				r->hit_limit = room;
+				if (r->cfg.mode == TM_MODE_KEYS_ALL) (void)grow_hits(r, room);
 			}
 			if (results > r->val_cap) {
 				TM_CHECK(grow_captured(r, &r->d_vals, r->val_cap, results + results / 4 + 1024));
@@ -2618,8 +2629,8 @@ int tm_wait(tm_ring * r, tm_status * st) {
 		r->st.n_hits = r->h_stat[2];
 		r->st.n_results = r->h_stat[3];
 		if (r->cfg.schedule == TM_SCHED_PERSISTENT) r->st.n_items = (uint32_t)r->h_stat[4];
-		r->st.hit_capacity = r->hit_cap;
-		r->st.overflow = r->retries > 0 || r->hits_grown;
+		r->st.hit_capacity = std::max(r->hit_cap, r->hit_limit);
+		r->st.overflow = r->retries > 0 || r->hits_over;
 		r->st.error = TM_OK;
 		r->st.device_ms = dms;
 		r->st.match_ms = mms;

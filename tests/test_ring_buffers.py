@@ -1,6 +1,8 @@
 """Submissions of different kinds and sizes in turn on one ring: buffers that
 one kind grows are those that another's captured steps use.  Exact: sets of
 whole numbers."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -28,6 +30,13 @@ def queries(n, first):
 def ordered(o, v):
     qid = np.repeat(np.arange(len(o) - 1, dtype=np.uint64), np.diff(o.astype(np.int64)))
     return np.sort((qid << np.uint64(32)) | v)
+
+
+def free_memory():
+    """Bytes of device memory left (the HIP runtime that the library uses)."""
+    free, total = C.c_size_t(), C.c_size_t()
+    assert tm.load().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
 
 
 def check(ring, exp, what):
@@ -76,3 +85,57 @@ def test_replays_between_units(gpu, table, mode, om):
             ring.submit(q0)
             ring.wait()
             check(ring, small, f"mode {mode}: 60 queries after {n} in units, turn {turn}")
+
+
+@pytest.mark.parametrize("mode,om", LISTS)
+def test_replayed_hit_list_outgrown_after_units(gpu, table, mode, om):
+    """A captured step with a hit list (work items logged) has more hits than
+    the list holds, with units in between, which keep none: it is run again."""
+    tab, fib = table
+    few, fit, many = np.zeros((64, 6), np.uint32), np.zeros((64, 6), np.uint32), queries(64, 3)
+    few[:4] = queries(4, 7)
+    fit[:2] = 0xFFFFFFFF
+    many[:5] = 0xFFFFFFFF
+    exp_few, exp_many = orc.match(*tab, few, mode=om), orc.match(*tab, many, mode=om)
+    ring = tm.Ring(fib, 64, mode=mode, use_graph=1, log_units=1, hit_capacity=41000)
+    part, off = np.array([1], np.uint32), np.array([0, 4], np.uint32)
+
+    def units():
+        ring.submit_units(few[:4], part, off)
+        assert ring.wait().overflow == 0
+        check(ring, unit_lists(tab, few[:4], part, off, om), f"mode {mode}: units")
+
+    units()                 # their counts do not grow again
+    ring.submit(fit)        # 40000 hits: the ring's values have room for those of a full hit list
+    ring.wait()
+    check(ring, orc.match(*tab, fit, mode=om), f"mode {mode}: as many hits as the list holds")
+    for _ in range(2):
+        ring.submit(few)
+        assert ring.wait().overflow == 0
+        check(ring, exp_few, f"mode {mode}: few hits")
+    units()
+    ring.submit(many)
+    st = ring.wait()
+    assert st.overflow == 1 and st.hit_capacity >= st.n_hits >= 100000
+    check(ring, exp_many, f"mode {mode}: many hits")
+
+
+def test_hits_take_no_list_memory(gpu, table):
+    """HITS values are written in place: 40M of them take their own memory
+    (4 bytes and a quarter more), none for a hit list (8 bytes)."""
+    tab, fib = table
+    n = 2000
+    q = np.full((n, 6), 0xFFFFFFFF, np.uint32)
+    ring = tm.Ring(fib, n, mode=tm.MODE_HITS, hit_capacity=1000)
+    before = free_memory()
+    ring.submit(q)
+    st = ring.wait()
+    used = before - free_memory()
+    print(f"{st.n_hits} hits, {used / 1e6:.0f} MB", flush=True)
+    assert st.n_hits == st.n_results == n * 20000
+    assert st.overflow == 1 and st.hit_capacity >= st.n_hits
+    assert used < 5 * st.n_hits + (64 << 20)
+    ring.submit_resident(n)
+    assert ring.wait().overflow == 0
+    o, v = ring.results()
+    assert np.array_equal(np.sort(v[:20000]), np.arange(20000)) and int(o[1]) == 20000
