@@ -2028,6 +2028,9 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 	// ms, 384: 3.07, 128: 3.39)
 	uint32_t seg = r->cfg.chunk_blocks ? r->cfg.chunk_blocks
 									   : (uint32_t)std::min<uint64_t>(384, std::max<uint64_t>(64, (work + 4 * resident - 1) / (4 * resident)));
+	// list modes count by segment and query: at most as many segments as
+	// HCNT_MAX counts allow (or items of MX_MAX_SEG blocks)
+	const uint64_t most = keys ? 0xFFFFFFFFu : std::max<uint64_t>(1, HCNT_MAX / std::max<uint32_t>(nq, 1));
 	std::vector<uint32_t> tab((size_t)std::max<uint32_t>(n, 1) * 8, 0), pre(n + 1, 0);
 	uint32_t max_nseg = 1;
 	uint64_t items = 0;
@@ -2037,7 +2040,9 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 		const uint32_t blo = f->h_part_info[(size_t)p * 8 + 6], nb = f->h_part_info[(size_t)p * 8 + 7];
 		const uint32_t ntiles = (qn + nqg - 1) / nqg;
 		const uint32_t useg = tuned && r->seg_bucket[size_bucket(nb)] ? r->seg_bucket[size_bucket(nb)] : seg;
-		const uint32_t sb = std::max<uint32_t>(1, std::min<uint32_t>(std::min(useg, MX_MAX_SEG), std::max<uint32_t>(nb, 1)));
+		// whole tiles of 32 blocks: what is smaller leaves items without any
+		const uint32_t least = (uint32_t)((nb + most - 1) / most);
+		const uint32_t sb = (std::min(std::max({useg, least, 1u}), std::min(MX_MAX_SEG, std::max(nb, 1u))) + 31) & ~31u;
 		const uint32_t nseg = nb ? (nb + sb - 1) / sb : 1;
 		uint32_t * t = &tab[(size_t)i * 8];
 		t[0] = p; t[1] = q0; t[2] = qn; t[3] = std::max<uint32_t>(ntiles, 1);

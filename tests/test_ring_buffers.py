@@ -139,3 +139,45 @@ def test_hits_take_no_list_memory(gpu, table):
     assert ring.wait().overflow == 0
     o, v = ring.results()
     assert np.array_equal(np.sort(v[:20000]), np.arange(20000)) and int(o[1]) == 20000
+
+
+def test_units_cut_into_whole_tiles(gpu, table):
+    """Segments of fewer blocks than a tile (32) make no items without any."""
+    tab, fib = table
+    part, off = np.array([0, 1, 2], np.uint32), np.array([0, 3, 73, 100], np.uint32)
+    q = queries(100, 5)
+    for seg in (1, 4, 31, 33, 0):
+        ring = tm.Ring(fib, 100, mode=tm.MODE_KEYS_UNIQUE, chunk_blocks=seg)
+        ring.submit_units(q, part, off)
+        st = ring.wait()
+        tiles = 1 + 5 + 6          # of 1, 140 and 172 blocks
+        print(f"segment {seg}: {st.n_items} items", flush=True)
+        assert st.n_items <= tiles, seg
+        check(ring, unit_lists(tab, q, part, off, 0), f"segment {seg}")
+
+
+@pytest.mark.parametrize("mode,om", LISTS)
+def test_unit_counts_are_bounded(gpu, mode, om):
+    """Units in the list modes: counts by segment and query take 256 MB at
+    most, however many queries and however small the segments."""
+    g = tm.Generator(seed=0xB0F)
+    w, ko, k = tm.canonicalize(*g.filters(240000))
+    n, nq = 200000, 800000     # 98 segments of 32 blocks x 800k queries: 314 MB
+    w, ko = np.ascontiguousarray(w[:n]), ko[:n + 1]
+    k = k[:int(ko[-1])]
+    assert w[0].any()          # no empty filter: the empty query matches nothing
+    fib, _ = tm.fib_from_runs(w, ko, k, np.array([0, n], np.uint32))
+    q = np.zeros((nq, 6), np.uint32)
+    at = np.arange(40) * 20011
+    q[at] = g.queries(40, 240000)[0]
+    ring = tm.Ring(fib, nq, mode=mode, chunk_blocks=32, hit_capacity=1000)
+    before = free_memory()
+    ring.submit_units(q, np.zeros(1, np.uint32), np.array([0, nq], np.uint32))
+    st = ring.wait()
+    used = before - free_memory()
+    print(f"mode {mode}: {st.n_hits} hits, {used / 1e6:.0f} MB", flush=True)
+    eo, ev = orc.match(w, ko, k, q[at], mode=om)
+    o, v = ring.results()
+    assert np.array_equal(np.diff(o.astype(np.int64))[at], np.diff(eo.astype(np.int64)))
+    assert int(o[-1]) == len(ev) and np.array_equal(np.sort(v), np.sort(ev))
+    assert used <= (256 << 20) + (32 << 20)
