@@ -1524,7 +1524,7 @@ mx_args matrix_args(tm_ring * r, int mode) {
 mx_shape hits_shape(const tm_ring * r, uint32_t nq, uint32_t resident) {
 	const uint64_t rows = std::max<uint64_t>(1, HCNT_MAX / std::max<uint32_t>(nq, 1));
 	const uint32_t seg_min = (uint32_t)((r->fib->n_blocks + rows - 1) / rows);
-	return mx_shape_of(MX_COUNT, nq, r->fib->n_blocks, resident, r->cfg.chunk_blocks ? std::max(r->cfg.chunk_blocks, seg_min) : 0, seg_min);
+	return mx_shape_of(MX_COUNT, r->kw, nq, r->fib->n_blocks, resident, r->cfg.chunk_blocks ? std::max(r->cfg.chunk_blocks, seg_min) : 0, seg_min);
 }
 
 // HITS and KEYS_ALL: one pass counts each query's values by segment, their
@@ -1586,6 +1586,42 @@ void enqueue_rows(tm_ring * r, uint32_t nq, bool rich, uint32_t * pcount, bool l
 	front_launch(a, r->s);
 }
 
+// Key rows that start empty, by their width: products of queries and blocks
+// up to which they are built in local memory, and from which to which (and
+// for how many queries at most) the vector kernel takes the step; other steps
+// build them in HBM, one atomic per bit, which is slow where few lines get
+// many (a line takes one after another).  Wider rows leave local memory for
+// fewer queries an item.  Match times, no list longer than 4 keys (filters,
+// queries: local, HBM, vector kernel), in us:
+//   4096 keys: 1M, 1000: 170, 384, 412; 5000: 564, 852, 733; 20000: 1983,
+//     2868, 2347; 100000: 9519, 9160, 10274; 4M, 5000: 1720, 1992, 1551
+//   8192: 1M, 1000: 250, 397, 416; 10000: 2033, 1674, 1359; 20000: 4016,
+//     3128, 4018; 4M, 2500: 1808, 1416, 1051; 10M, 5000: 8158, 3216, 3719
+//   16384: 1M, 1000: 307, 386, 424; 5000: 1349, 962, 1233; 4M, 1000: 1016,
+//     683, 593
+//   32768: 1M, 1000: 562, 354, -
+struct rows_rule {
+	uint32_t kw;
+	uint64_t lds, vec_from, vec_to;
+	uint32_t vec_nq;
+};
+constexpr rows_rule EMPTY_ROWS[] = {
+	{64, ~0ull, 0, 0, 0},
+	{128, 200000000, 200000000, 600000000, 24000},
+	{256, 24000000, 70000000, 600000000, 12000},
+	{512, 24000000, 50000000, 600000000, 1500},
+};
+enum empty_rows { ROWS_LDS, ROWS_HBM, ROWS_VECTOR };
+empty_rows empty_rows_of(const tm_ring * r, uint32_t nq) {
+	const uint64_t work = (uint64_t)nq * r->fib->n_blocks;
+	for (const rows_rule & w : EMPTY_ROWS) {
+		if (r->kw > w.kw) continue;
+		if (work <= w.lds || (w.kw <= 128 && r->fib->n_blocks <= ROWS_LDS_MAX_BLOCKS)) return ROWS_LDS;
+		return r->lds_bm && work >= w.vec_from && work <= w.vec_to && nq <= w.vec_nq ? ROWS_VECTOR : ROWS_HBM;
+	}
+	return ROWS_HBM;
+}
+
 // The persistent step on the matrix cores.
 int enqueue_matrix(tm_ring * r, uint32_t nq, bool events) {
 	hipStream_t s = r->s;
@@ -1604,16 +1640,22 @@ int enqueue_matrix(tm_ring * r, uint32_t nq, bool events) {
 		return enqueue_values(r, a, h.nseg, a.resident, events);
 	}
 	// Rows in local memory where the match sets most of their bits: without
-	// a rich-filter pass, or where no rich filter holds every key and the
-	// table or the step is small.  In larger ones more queries per item win.
+	// a rich-filter pass (empty_rows_of), or where no rich filter holds every
+	// key and the table or the step is small.  In larger ones more queries per
+	// item win.
 	// Both sides measured (blocks, queries: local, HBM): 735, 250k: 1.34,
 	// 1.65 ms; 1997, 44k: 0.66, 0.76; 1997, 700k: 9.0, 8.7; 2910, 10k: 0.31,
 	// 0.26; 2910, 700k: 12.6, 10.2; 6.9k, 13k: 0.39, 0.38; 6.9k, 40k: 1.08,
-	// 0.93; 17k, 5k: 0.091, 0.092; 17k, 100k: 1.13, 0.62.
-	const bool sparse = !rich_pass || (compact && r->fib->n_rich_full == 0 &&
-									   (r->fib->n_blocks <= ROWS_LDS_MAX_BLOCKS ||
-										(uint64_t)nq * r->fib->n_blocks <= ROWS_LDS_MAX_WORK));
-	const int mode = sparse && r->kw <= MX_LDS_KW && r->kw > 0 ? MX_KEYS_LDS : MX_KEYS;
+	// 0.93; 17k, 5k: 0.091, 0.092; 17k, 100k: 1.13, 0.62.  Rows of up to twice
+	// the width, and in steps five times as large where few rich filters leave
+	// them nearly empty: 4096 keys, 3 rich filters, 15k, 5k: 0.56, 0.83 (0.75
+	// with the vector kernel), 20k: 1.98, 2.83 (2.77); 57k, 5k: 1.71, 2.00
+	// (1.88), 20k: 6.6, 4.8; 781 rich filters, 15k, 20k: 2.31, 1.94.
+	const bool sparse = !rich_pass ? empty_rows_of(r, nq) == ROWS_LDS
+								   : compact && r->fib->n_rich_full == 0 && r->kw <= 2 * MX_LDS_KW &&
+										 (r->fib->n_blocks <= ROWS_LDS_MAX_BLOCKS ||
+										  (uint64_t)nq * r->fib->n_blocks <= (r->kw > MX_LDS_KW && r->fib->n_rich <= 64 ? 5 : 1) * ROWS_LDS_MAX_WORK);
+	const int mode = sparse && r->kw > 0 ? MX_KEYS_LDS : MX_KEYS;
 	mx_args a = matrix_args(r, mode);
 	a.nq = nq;
 	if (compact) {
@@ -1641,7 +1683,8 @@ int enqueue_persistent(tm_ring * r, uint32_t nq, bool events) {
 	const uint32_t P = r->P;
 	const bool exit_on = keyrows(r->cfg) && r->lds_bm && r->kw > 0 && r->cfg.full_exit != 2;
 	const bool rich_pass = exit_on && r->fib->n_rich > 0 && nq > 0;
-	if (!r->use_iorder && !r->cfg.log_units && (!exit_on || rich_pass)) return enqueue_matrix(r, nq, events);
+	const bool vector = keyrows(r->cfg) && r->kw > 0 && r->fib->n_rich == 0 && empty_rows_of(r, nq) == ROWS_VECTOR;
+	if (!r->use_iorder && !r->cfg.log_units && (!exit_on || rich_pass) && !vector) return enqueue_matrix(r, nq, events);
 	start_step(r, nq, 0);
 	const uint64_t nqg = (uint64_t)r->tiles * 64;
 	const uint64_t tiles = (nq + nqg - 1) / nqg;
@@ -2014,9 +2057,16 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 	}
 	// persistent: segment size from the whole submission's work
 	const bool keys = keyrows(r->cfg);
-	const int mode = !keys ? MX_COUNT : r->kw > MX_LDS_KW || r->kw == 0 ? MX_KEYS : MX_KEYS_LDS;
+	// Rows in local memory, but for wide ones that gain few bits: a unit has a
+	// query's matches in one partition, so most words of a row stay empty, and
+	// long lists cost an atomic per key in HBM.  Local and HBM, us: 1M filters
+	// in large partitions, 65k queries, 4096 keys 552, 9597 (the vector kernel
+	// 1497), 32768 keys 1810, 47538 (8681); lists of 4 keys at most, 32768 keys
+	// 1351, 1526 (3023); in small partitions, 2.6M queries 4172, 1169 (3108),
+	// 16384 keys 2092, 1091 (8788), 4096 keys 795, 934 (1411).
+	const int mode = !keys ? MX_COUNT : r->kw == 0 || (r->kw > 8 * MX_LDS_KW && f->ovf_valid <= 1) ? MX_KEYS : MX_KEYS_LDS;
 	mx_args a = matrix_args(r, mode);
-	const uint32_t nqg = mx_super(mode);
+	const uint32_t nqg = mx_super_of(mode, r->kw);
 	const uint64_t resident = a.resident;
 	uint64_t work = 0;   // tile x blocks
 	for (uint32_t i = 0; i < n; ++i) {

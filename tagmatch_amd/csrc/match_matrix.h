@@ -13,7 +13,8 @@ namespace tmx {
 //   MX_WRITE, MX_WRITE_KEYS   the values, behind those of earlier segments.
 enum mx_mode { MX_KEYS, MX_KEYS_LDS, MX_COUNT, MX_COUNT_KEYS, MX_WRITE, MX_WRITE_KEYS, MX_MODES };
 
-constexpr uint32_t MX_LDS_KW = 64;      // MX_KEYS_LDS: words of a row, at most
+constexpr uint32_t MX_LDS_KW = 64;      // MX_KEYS_LDS: words of a row with the most queries per item
+constexpr uint32_t MX_ROW_WORDS = 192 * MX_LDS_KW;   // MX_KEYS_LDS: words of an item's rows, at most
 constexpr uint32_t MX_QUEUES = 8;       // work queues, one per XCD
 constexpr uint32_t MX_QPAD = 32;        // queue cursors 256 B apart
 constexpr uint32_t MX_MAX_SEG = 16384;  // blocks per work item, at most
@@ -34,6 +35,13 @@ constexpr int MX_WAVES = 8;             // waves per workgroup
 __host__ __device__ constexpr uint32_t mx_super(int mode) {
 	return mode == MX_KEYS ? 2048u : mode == MX_KEYS_LDS ? 192u : 1536u;
 }
+// The same for rows of kw words: wider ones leave room for fewer (128 KB of
+// rows and one workgroup per CU took longer at every width up to 1024 words
+// but 256: 4096 keys 552 and 691 us, 16384 keys 1067 and 1593).
+__host__ __device__ inline uint32_t mx_super_of(int mode, uint32_t kw) {
+	const uint32_t most = mx_super(mode);
+	return mode != MX_KEYS_LDS || kw * most <= MX_ROW_WORDS ? most : MX_ROW_WORDS / kw;
+}
 __host__ __device__ constexpr uint32_t mx_mask_words(int mode) {
 	return mode == MX_KEYS ? 64u * 65u : mode == MX_KEYS_LDS ? 128u * 7u : 64u * 49u;
 }
@@ -51,15 +59,21 @@ __host__ __device__ constexpr uint32_t mx_visits(int mode) { return mode == MX_K
 // and 135).  Otherwise 128 blocks: between 64
 // and 256 it is the fastest or within 4 % of it (1M filters, 300k queries,
 // for 64, 128, 256: 1.58, 1.52, 1.65 ms; 10M, 1M queries: 1.00, 0.98, 1.00;
-// 65k without the full-row exit: 11.7, 11.4, 11.4).  seg_min: least blocks
+// 65k without the full-row exit: 11.7, 11.4, 11.4); up to 512 for wide rows
+// in local memory, cleared and merged for each item, at four items per
+// workgroup (4096 keys, no long list, 1M filters, 20k queries: 2.37 ms with
+// 128, 1.98 with 512; 4M, 5k: 2.06, 1.72).  seg_min: least blocks
 // per segment (a bound on the segments), 0: none.
 struct mx_shape {
 	uint32_t sq, nsuper, seg, nseg;
 };
-__host__ __device__ inline mx_shape mx_shape_of(int mode, uint32_t nq, uint32_t nblk, uint32_t resident,
+__host__ __device__ inline mx_shape mx_shape_of(int mode, uint32_t kw, uint32_t nq, uint32_t nblk, uint32_t resident,
 												uint32_t seg_fixed, uint32_t seg_min) {
-	uint32_t sq = mx_super(mode);
-	if (nq < sq) sq = nq > 64 ? (nq + 63) & ~63u : 64u;
+	uint32_t sq = mx_super_of(mode, kw);
+	if (nq < sq) {
+		const uint32_t some = nq > 64 ? (nq + 63) & ~63u : 64u;
+		if (some < sq) sq = some;
+	}
 	// few blocks: fewer queries per item (20k queries, 8.8k blocks: 0.70
 	// instead of 1.30 ms)
 	while (sq > 256 && (uint64_t)((nq + sq - 1) / sq) * ((nblk + 63) / 64) < 4ull * resident) sq = (sq / 2 + 63) & ~63u;
@@ -69,6 +83,9 @@ __host__ __device__ inline mx_shape mx_shape_of(int mode, uint32_t nq, uint32_t 
 		const uint64_t per = ((uint64_t)nblk * nsuper + resident - 1) / resident;   // blocks of a workgroup
 		const uint64_t rounds = (per + 511) / 512;
 		seg = per == 0 ? 32u : (uint32_t)((per + rounds - 1) / rounds + 31) & ~31u;
+	} else if (mode == MX_KEYS_LDS && kw > MX_LDS_KW) {
+		const uint64_t per = (uint64_t)nblk * nsuper / (4ull * resident);
+		seg = per < 128 ? 128u : per > 512 ? 512u : (uint32_t)per & ~31u;
 	}
 	if (seg < seg_min) seg = seg_min;
 	if (seg_fixed) seg = seg_fixed;

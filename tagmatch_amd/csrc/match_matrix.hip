@@ -59,7 +59,7 @@ k_match_x(mx_args a) {
 	constexpr int WAVES = MX_WAVES, NT = WAVES * 64;
 	constexpr uint32_t SUPER = mx_super(MODE), MASK = mx_mask_words(MODE), VISITS = mx_visits(MODE);
 	constexpr bool ROWS = MODE == MX_KEYS || MODE == MX_KEYS_LDS;
-	__shared__ uint32_t s_rows[MODE == MX_KEYS_LDS ? SUPER * MX_LDS_KW : 1];   // key rows, kw words each
+	__shared__ uint32_t s_rows[MODE == MX_KEYS_LDS ? MX_ROW_WORDS : 1];   // key rows, kw words each
 	__shared__ uint32_t s_cnt[ROWS ? 1 : SUPER];    // values of each query so far
 	__shared__ uint32_t s_q[6 * SUPER];             // inverted words, one plane per word
 	__shared__ uint32_t s_full[SUPER / 32];         // queries whose rows hold every key
@@ -77,7 +77,8 @@ k_match_x(mx_args a) {
 	const uint32_t nq_all = a.nq_dev ? sld1(a.nq_dev) : a.nq;
 	const uint32_t epoch = a.step_vals ? sld1(a.step_vals) : a.epoch;
 	const uint32_t ovf_n = a.step_vals ? sld1(a.step_vals + 1) : a.f.ovf_n;
-	const mx_shape sh = mx_shape_of(MODE, nq_all, a.nblk, a.resident, a.seg_fixed, a.seg_min);
+	const mx_shape sh = mx_shape_of(MODE, kw, nq_all, a.nblk, a.resident, a.seg_fixed, a.seg_min);
+	const uint32_t usq = mx_super_of(MODE, kw);   // queries of a unit's items
 	const uint32_t items = a.units ? sld1(a.uprefix + a.n_units) : sh.nsuper * sh.nseg;
 	if (blockIdx.x == 0 && tid == 0) *a.n_items = items;
 	const bool queued = items > gridDim.x;
@@ -108,6 +109,7 @@ k_match_x(mx_args a) {
 		}
 		// blocks of the item: tiles of 32, `apart` blocks from one to the next
 		uint32_t q0, nqs, b0, apart, nloc, b_end, seg;
+		bool sole = false;   // no other item adds to its queries' rows, which are empty
 		if (a.units) {
 			uint32_t lo = 0, hi = a.n_units;
 			while (hi - lo > 1) {
@@ -119,11 +121,12 @@ k_match_x(mx_args a) {
 			const uint32_t local = item - sld1(a.uprefix + lo);
 			seg = local / u0.w;
 			const uint32_t sup = local - seg * u0.w;
-			q0 = u0.y + sup * SUPER;
-			nqs = min(SUPER, u0.y + u0.z - q0);
+			q0 = u0.y + sup * usq;
+			nqs = min(usq, u0.y + u0.z - q0);
 			b0 = u1.z + seg * 32;
 			apart = u1.x * 32;
 			b_end = u1.w;
+			sole = u1.x == 1;
 		} else {
 			seg = item / sh.nsuper;
 			const uint32_t sup = item - seg * sh.nsuper;
@@ -520,7 +523,8 @@ k_match_x(mx_args a) {
 				uint32_t * dst = a.gbm + (size_t)(a.qmap ? sld1(a.qmap + q0 + j) : q0 + j) * kw;
 				for (uint32_t w = lane; w < kw; w += 64) {
 					const uint32_t v = s_rows[j * kw + w];
-					if (v && (v & ~dst[w])) atomicOr(&dst[w], v);
+					if (sole && v) dst[w] = v;
+					else if (v && (v & ~dst[w])) atomicOr(&dst[w], v);
 				}
 			}
 			__syncthreads();
