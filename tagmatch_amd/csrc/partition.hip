@@ -28,8 +28,9 @@
 //
 // A NONZERO segment needs up to 192 splits in a row, each on what the last
 // one left: one workgroup makes them all without the host (k_nonzero), on
-// lists of positions instead of the records.  Larger segments than NZ_MAX
-// filters are split level by level until they fit.
+// lists of positions instead of the records.  Segments of more filters than
+// NZ_MAX, or of more set bits than NZ_BITS, are split level by level until
+// they fit.
 #include "hip_util.h"
 
 #include <algorithm>
@@ -43,7 +44,13 @@ namespace {
 constexpr uint32_t TILE = 1024;
 // A workgroup takes about 0.5 us per 1024 filters left and split: a million
 // would keep one CU busy for milliseconds, where the levels use them all.
+// Each filter it moves also has its set bits counted out, 0.2 us per 1024:
+// segments of more set bits than NZ_BITS are split by the levels, too (whole
+// calls on 200k filters with half, an eighth, a fiftieth of their bits set:
+// 5.2, 4.7, 11.7 ms without this bound, 1.4, 3.9, 11.6 with 4M, 1.07, 1.9, 8.7
+// with 0.5M).
 constexpr uint32_t NZ_MAX = 256 * 1024;
+constexpr uint64_t NZ_BITS = 500000;
 constexpr uint32_t NZ_ROUNDS = 193;   // splits of a NONZERO segment (a pivot bit is gone after its split) + 1
 constexpr int NO_PIVOT = -1;
 
@@ -51,6 +58,7 @@ enum seg_mode : uint8_t { BALANCE = 0, NONZERO = 1, DONE = 2 };
 
 struct seg_t {
 	uint32_t begin, end;
+	uint64_t bits;          // set bits of its filters, at most
 	uint32_t used[6];       // pivot bits used on the path (BALANCE only)
 	uint8_t mode;
 	uint8_t mask_nonempty;  // some 1-side pivot on the path
@@ -416,6 +424,7 @@ extern "C" int tm_partition(const uint32_t * words, uint32_t n, uint32_t maxp, u
 	segs[0].begin = 0;
 	segs[0].end = n;
 	segs[0].mode = n > maxp ? BALANCE : NONZERO;
+	segs[0].bits = (uint64_t)n * 192;
 
 	// Host arrays of a level, in one upload each; a buffer is filled again
 	// only after the stream was waited for since its upload.
@@ -456,7 +465,9 @@ extern "C" int tm_partition(const uint32_t * words, uint32_t n, uint32_t maxp, u
 		// segments to split by this level's kernels
 		act.clear();
 		for (uint32_t k = 0; k < segs.size(); ++k)
-			if (segs[k].mode == BALANCE || (segs[k].mode == NONZERO && segs[k].end - segs[k].begin > NZ_MAX)) act.push_back(k);
+			if (segs[k].mode == BALANCE ||
+				(segs[k].mode == NONZERO && (segs[k].end - segs[k].begin > NZ_MAX || segs[k].bits > NZ_BITS)))
+				act.push_back(k);
 		if (act.empty()) break;
 		if (level > 100000) return set_error(TM_ERR_HIP, "partitioner did not converge");
 		TM_CHECK(histograms());
@@ -475,13 +486,20 @@ extern "C" int tm_partition(const uint32_t * words, uint32_t n, uint32_t maxp, u
 		std::vector<std::pair<uint32_t, uint32_t>> split_ranges;
 		uint32_t a = 0;
 		for (uint32_t k = 0; k < segs.size(); ++k) {
-			const seg_t g = segs[k];
+			seg_t g = segs[k];
 			if (a >= na || act[a] != k) {
 				next.push_back(g);
 				continue;
 			}
 			const uint32_t * f = &freq[(size_t)a * 192];
 			const uint32_t size = g.end - g.begin;
+			g.bits = 0;
+			for (int b = 0; b < 192; ++b) g.bits += f[b];
+			if (g.mode == NONZERO && size <= NZ_MAX && g.bits <= NZ_BITS) {   // now that its bits are known
+				next.push_back(g);
+				++a;
+				continue;
+			}
 			int pv = NO_PIVOT;
 			if (g.mode == NONZERO) {
 				uint32_t mf = f[0];
@@ -502,6 +520,8 @@ extern "C" int tm_partition(const uint32_t * words, uint32_t n, uint32_t maxp, u
 			seg_t z = g, o = g;
 			z.end = g.begin + (size - f[pv]);
 			o.begin = z.end;
+			z.bits = g.bits - f[pv];   // the pivot's are the other side's
+			for (seg_t * c : {&z, &o}) c->bits = std::min(c->bits, (uint64_t)(c->end - c->begin) * 192);
 			if (g.mode == NONZERO) {
 				o.mode = DONE;
 			} else {
