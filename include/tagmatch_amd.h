@@ -300,7 +300,7 @@ int tm_ring_autotune(tm_ring * ring, uint32_t nq, const tm_match_config * cands,
  * bucket(nb) = 0 below 16 blocks, 1 below 64, 2 below 256, 3 below 1024,
  * 4 below 4096, 5 from 4096; 0 = the automatic size (the submission's
  * tile-blocks spread over about four items per resident workgroup, at most
- * 384).  Sizes are rounded up to multiples of 32; in HITS and KEYS_ALL they
+ * 384).  Sizes are rounded to multiples of 32; in HITS and KEYS_ALL they
  * are raised until the submission's counts by segment and query take 256 MB
  * at most.  The reference runs one fixed launch shape per (partition, batch)
  * (gpu.cu:878-912). */

@@ -1521,10 +1521,10 @@ mx_args matrix_args(tm_ring * r, int mode) {
 }
 
 // Segments of a hit-list step: as many as its per-segment counts may take.
-mx_shape hits_shape(const tm_ring * r, uint32_t nq, uint32_t resident) {
+mx_shape hits_shape(const tm_ring * r, uint32_t nq, mx_args & a) {
 	const uint64_t rows = std::max<uint64_t>(1, HCNT_MAX / std::max<uint32_t>(nq, 1));
-	const uint32_t seg_min = (uint32_t)((r->fib->n_blocks + rows - 1) / rows);
-	return mx_shape_of(MX_COUNT, r->kw, nq, r->fib->n_blocks, resident, r->cfg.chunk_blocks ? std::max(r->cfg.chunk_blocks, seg_min) : 0, seg_min);
+	a.seg_min = (uint32_t)((r->fib->n_blocks + rows - 1) / rows);
+	return mx_shape_of(MX_COUNT, r->kw, nq, r->fib->n_blocks, a.resident, a.seg_fixed, a.seg_min);
 }
 
 // HITS and KEYS_ALL: one pass counts each query's values by segment, their
@@ -1635,9 +1635,8 @@ int enqueue_matrix(tm_ring * r, uint32_t nq, bool events) {
 	if (!keys) {
 		mx_args a = matrix_args(r, MX_COUNT);
 		a.nq = nq;
-		const mx_shape h = hits_shape(r, nq, a.resident);
-		a.seg_fixed = h.seg;
-		return enqueue_values(r, a, h.nseg, a.resident, events);
+		const uint32_t rows = hits_shape(r, nq, a).nseg;
+		return enqueue_values(r, a, rows, a.resident, events);
 	}
 	// Rows in local memory where the match sets most of their bits: without
 	// a rich-filter pass (empty_rows_of), or where no rich filter holds every
@@ -2090,9 +2089,9 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 		const uint32_t blo = f->h_part_info[(size_t)p * 8 + 6], nb = f->h_part_info[(size_t)p * 8 + 7];
 		const uint32_t ntiles = (qn + nqg - 1) / nqg;
 		const uint32_t useg = tuned && r->seg_bucket[size_bucket(nb)] ? r->seg_bucket[size_bucket(nb)] : seg;
-		// whole tiles of 32 blocks: what is smaller leaves items without any
-		const uint32_t least = (uint32_t)((nb + most - 1) / most);
-		const uint32_t sb = (std::min(std::max({useg, least, 1u}), std::min(MX_MAX_SEG, std::max(nb, 1u))) + 31) & ~31u;
+		// whole tiles of 32 blocks, the nearest: less leaves items without any
+		const uint32_t least = (uint32_t)((nb + most - 1) / most + 31) & ~31u;
+		const uint32_t sb = std::min(MX_MAX_SEG, std::max({(std::min(useg, MX_MAX_SEG) + 16) & ~31u, least, 32u}));
 		const uint32_t nseg = nb ? (nb + sb - 1) / sb : 1;
 		uint32_t * t = &tab[(size_t)i * 8];
 		t[0] = p; t[1] = q0; t[2] = qn; t[3] = std::max<uint32_t>(ntiles, 1);
@@ -2429,9 +2428,8 @@ int submit_common(tm_ring * r, uint32_t nq) {
 	}
 	if (!r->units_mode) TM_CHECK(price_submission(r, r->run_nq));
 	if (!r->units_mode && !keyrows(r->cfg) && r->cfg.schedule == TM_SCHED_PERSISTENT && !r->cfg.log_units) {
-		const mx_args a = matrix_args(r, MX_COUNT);
-		const mx_shape h = hits_shape(r, r->run_nq, a.resident);
-		TM_CHECK(grow_captured(r, &r->d_hcnt, r->hcnt_cap, (uint64_t)h.nseg * r->run_nq));
+		mx_args a = matrix_args(r, MX_COUNT);
+		TM_CHECK(grow_captured(r, &r->d_hcnt, r->hcnt_cap, (uint64_t)hits_shape(r, r->run_nq, a).nseg * r->run_nq));
 	}
 	int rc = enqueue_step(r, true);
 	if (rc != TM_OK) return rc;

@@ -181,3 +181,29 @@ def test_unit_counts_are_bounded(gpu, mode, om):
     assert np.array_equal(np.diff(o.astype(np.int64))[at], np.diff(eo.astype(np.int64)))
     assert int(o[-1]) == len(ev) and np.array_equal(np.sort(v), np.sort(ev))
     assert used <= (256 << 20) + (32 << 20)
+
+
+def test_few_configured_segments(gpu):
+    """Few segments, configured: items of fewer queries, so that the GPU is
+    not left idle (and the counts by segment and query agree with the shape
+    that the kernel takes)."""
+    g = tm.Generator(seed=0xB0F)
+    tab = tm.canonicalize(*g.filters(100000))
+    fib, *_ = tm.build_fib(*tab, 30000)
+    nq = 150000
+    q = np.zeros((nq, 6), np.uint32)
+    at = np.arange(60) * 2477
+    q[at] = g.queries(60, 100000)[0]
+    for mode, om in LISTS:
+        eo, ev = orc.match(*tab, q[at], mode=om)
+        for seg in (64, 1000, 4096):
+            ring = tm.Ring(fib, nq, mode=mode, chunk_blocks=seg)
+            ring.submit(q)
+            st = ring.wait()
+            o, v = ring.results()
+            print(f"mode {mode} segment {seg}: {st.n_items} items", flush=True)
+            assert np.array_equal(np.diff(o.astype(np.int64))[at], np.diff(eo.astype(np.int64)))
+            got = [np.sort(v[int(o[i]):int(o[i + 1])]) for i in at]
+            want = [np.sort(ev[int(eo[i]):int(eo[i + 1])]) for i in range(60)]
+            assert all(np.array_equal(x, y) for x, y in zip(got, want))
+            assert st.n_items >= 400
