@@ -236,13 +236,13 @@ typedef struct tm_match_config {
 	                            step size for PERSISTENT (16 up to 16 query
 	                            tiles, 8 up to 256, else 4; 8 in the matrix
 	                            kernel), 8 for PLAIN                         */
-	uint32_t groups_per_cu;  /* PERSISTENT: resident workgroups per CU; 0 = auto */
+	uint32_t groups_per_cu;  /* PERSISTENT: resident workgroups per CU, at most;
+	                            0 = as many as fit                           */
 	uint64_t hit_capacity;   /* HITS / KEYS_ALL: hit slots; 0 = default      */
 	uint32_t use_graph;      /* PERSISTENT: replay steady-state steps from a
 	                            captured hipGraph                            */
 	uint32_t log_units;      /* record per-work-item hit counts and cycles   */
-	uint32_t order_by_cost;  /* PERSISTENT: visit partitions in the order set
-	                            by tm_ring_set_order                          */
+	uint32_t order_by_cost;  /* accepted and ignored (TM_COST_ORDER orders tiles) */
 	uint32_t variant;        /* accepted and ignored (there is one inner loop)  */
 	uint32_t full_exit;      /* PERSISTENT KEYS_UNIQUE: stop testing a query
 	                            once its key set holds every key of the
@@ -491,7 +491,13 @@ int tm_ring_unit_log(tm_ring * ring, float * features, uint32_t * hits, uint32_t
 /* Use a trained TM_UNIT_FEATURES-64-64-3 model in the ring's PERSISTENT
  * submissions (NULL: none).  The model must outlive its use by the ring. */
 #define TM_COST_PRESIZE 1u  /* grow result buffers to the predicted size first */
-#define TM_COST_ORDER   2u  /* visit query tiles longest-predicted first        */
+#define TM_COST_ORDER   2u  /* visit query tiles longest-predicted first, where
+                             * a step's tiles fill the GPU twice and its table
+                             * is one segment (up to 1024 blocks, or
+                             * chunk_blocks).  Such a step runs on the vector
+                             * kernel, like steps that log work items: where
+                             * the matrix kernel would take it, ordering costs
+                             * more than it balances.                         */
 int tm_ring_set_cost_model(tm_ring * ring, tm_mlp * model, uint32_t flags);
 
 /* ------------------------------------------------------------------------ */

@@ -1509,6 +1509,8 @@ mx_args matrix_args(tm_ring * r, int mode) {
 	a.seg_fixed = r->cfg.chunk_blocks;
 	if (!r->mx_groups[mode]) r->mx_groups[mode] = (int)mx_resident(mode);
 	a.resident = (uint32_t)r->mx_groups[mode];
+	if (r->cfg.groups_per_cu)
+		a.resident = (uint32_t)std::min<uint64_t>(a.resident, (uint64_t)r->cfg.groups_per_cu * dev().num_cu);
 	a.wg_stats = r->d_wgstat;
 	a.qnext = r->d_qnext;
 	a.gbm = r->d_gbm;

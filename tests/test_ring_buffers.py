@@ -207,3 +207,23 @@ def test_few_configured_segments(gpu):
             want = [np.sort(ev[int(eo[i]):int(eo[i + 1])]) for i in range(60)]
             assert all(np.array_equal(x, y) for x, y in zip(got, want))
             assert st.n_items >= 400
+
+
+def test_groups_per_cu_holds(gpu):
+    """groups_per_cu bounds the workgroups that a step is cut for: a small
+    step, one item each, makes about half as many items with one per CU as
+    with two."""
+    g = tm.Generator(seed=0xB0F)
+    tab = tm.canonicalize(*g.filters(800000))
+    fib, *_ = tm.build_fib(*tab, 60000)
+    q = queries(500, 3)
+    items, res = [], []
+    for groups in (0, 2, 1):
+        ring = tm.Ring(fib, 500, mode=tm.MODE_HITS, groups_per_cu=groups)
+        ring.submit(q)
+        items.append(ring.wait().n_items)
+        res.append(ring.results())
+        assert np.array_equal(res[0][0], res[-1][0])
+        assert np.array_equal(ordered(*res[0]), ordered(*res[-1]))
+    print(f"items {items}", flush=True)
+    assert items[0] == items[1] and items[2] < 0.7 * items[1]
