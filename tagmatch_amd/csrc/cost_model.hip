@@ -58,18 +58,20 @@ struct tm_mlp {
 namespace {
 
 // Y[n][m] = X[n][K] B[K][m], a 64 x 64 tile per workgroup and 4 x 4 per
-// thread, operands in local memory 16 of K at a time; each output adds its
-// products in ascending order of K.
+// thread, operands in local memory 64 of K at a time, their loads all in flight
+// together (16 at a time, loaded during the 16 before: a call of one row, all
+// latency, 121 us; 112 so); each output adds its products in ascending order
+// of K.
 //   BACK false: B = W[K][m]; sums start at bias[c]; ReLU if relu
 //   BACK true:  B = W[m][K] transposed; outputs whose H is not positive are 0
 // Bound by its operands' bytes at the cost model's sizes: the 65536 x 64 x 64
-// backward product takes 21 us, one thread per output with W's rows read a
+// backward product takes 17 us, one thread per output with W's rows read a
 // line per lane 283 us.
 template <bool BACK>
 __global__ void __launch_bounds__(256)
 k_layer(const float * __restrict__ X, const float * __restrict__ W, const float * __restrict__ bias,
 		const float * __restrict__ H, float * __restrict__ Y, uint32_t n, uint32_t K, uint32_t m, int relu) {
-	__shared__ float s_x[16][68], s_w[16][68];
+	__shared__ float s_x[64][68], s_w[64][68];
 	const uint32_t tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
 	const uint32_t r0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
 	float acc[4][4];
@@ -80,33 +82,38 @@ k_layer(const float * __restrict__ X, const float * __restrict__ W, const float 
 #pragma unroll
 		for (int i = 0; i < 4; ++i) acc[i][j] = b;
 	}
-	float lx[4], lw[4];   // the next 16 of K, loaded while these are multiplied
-	auto load = [&](uint32_t k0) {
+	for (uint32_t k0 = 0; k0 < K; k0 += 64) {
+		float lx[4][4], lw[4][4];
 #pragma unroll
-		for (int e = 0; e < 4; ++e) {
-			const uint32_t x = tid + e * 256, k = x & 15, r = x >> 4;   // 16 of K per row
-			lx[e] = r0 + r < n && k0 + k < K ? X[(size_t)(r0 + r) * K + k0 + k] : 0.f;
-			if (BACK) {
-				lw[e] = c0 + r < m && k0 + k < K ? W[(size_t)(c0 + r) * K + k0 + k] : 0.f;
-			} else {
-				const uint32_t c = x & 63, kk = x >> 6;
-				lw[e] = c0 + c < m && k0 + kk < K ? W[(size_t)(k0 + kk) * m + c0 + c] : 0.f;
+		for (uint32_t g = 0; g < 4; ++g) {   // 16 of K each
+			if (k0 + g * 16 >= K) continue;
+#pragma unroll
+			for (uint32_t e = 0; e < 4; ++e) {
+				const uint32_t x = tid + e * 256, k = k0 + g * 16 + (x & 15), r = x >> 4;   // 16 of K per row
+				lx[g][e] = r0 + r < n && k < K ? X[(size_t)(r0 + r) * K + k] : 0.f;
+				if (BACK) {
+					lw[g][e] = c0 + r < m && k < K ? W[(size_t)(c0 + r) * K + k] : 0.f;
+				} else {
+					const uint32_t c = x & 63, kk = k0 + g * 16 + (x >> 6);
+					lw[g][e] = c0 + c < m && kk < K ? W[(size_t)kk * m + c0 + c] : 0.f;
+				}
 			}
 		}
-	};
-	load(0);
-	for (uint32_t k0 = 0; k0 < K; k0 += 16) {
+		if (k0) __syncthreads();
 #pragma unroll
-		for (int e = 0; e < 4; ++e) {
-			const uint32_t x = tid + e * 256;
-			s_x[x & 15][x >> 4] = lx[e];
-			if (BACK) s_w[x & 15][x >> 4] = lw[e];
-			else s_w[x >> 6][x & 63] = lw[e];
+		for (uint32_t g = 0; g < 4; ++g) {
+			if (k0 + g * 16 >= K) continue;
+#pragma unroll
+			for (uint32_t e = 0; e < 4; ++e) {
+				const uint32_t x = tid + e * 256;
+				s_x[g * 16 + (x & 15)][x >> 4] = lx[g][e];
+				if (BACK) s_w[g * 16 + (x & 15)][x >> 4] = lw[g][e];
+				else s_w[g * 16 + (x >> 6)][x & 63] = lw[g][e];
+			}
 		}
 		__syncthreads();
-		if (k0 + 16 < K) load(k0 + 16);
-#pragma unroll
-		for (uint32_t k = 0; k < 16; ++k) {
+		const uint32_t kn = min(64u, K - k0);
+		auto step = [&](uint32_t k) {
 			const float4 x = *reinterpret_cast<const float4 *>(&s_x[k][ty * 4]);
 			const float4 w = *reinterpret_cast<const float4 *>(&s_w[k][tx * 4]);
 			const float xs[4] = {x.x, x.y, x.z, x.w}, ws[4] = {w.x, w.y, w.z, w.w};
@@ -114,8 +121,13 @@ k_layer(const float * __restrict__ X, const float * __restrict__ W, const float 
 			for (int i = 0; i < 4; ++i)
 #pragma unroll
 				for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(xs[i], ws[j], acc[i][j]);
+		};
+		uint32_t k = 0;
+		for (; k + 16 <= kn; k += 16) {
+#pragma unroll
+			for (uint32_t i = 0; i < 16; ++i) step(k + i);
 		}
-		__syncthreads();
+		for (; k < kn; ++k) step(k);
 	}
 #pragma unroll
 	for (int i = 0; i < 4; ++i) {
@@ -193,8 +205,7 @@ k_wgrad(const float * __restrict__ A, const float * __restrict__ dY, float * __r
 		}
 		__syncthreads();
 		if (rb + 16 < r1) load(rb + 16);
-#pragma unroll
-		for (uint32_t r = 0; r < 16; ++r) {
+		auto row = [&](uint32_t r) {
 			const float4 x = *reinterpret_cast<const float4 *>(&s_a[r][ty * 4]);
 			const float4 d = *reinterpret_cast<const float4 *>(&s_d[r][tx * 4]);
 			const float xs[4] = {x.x, x.y, x.z, x.w}, ds[4] = {d.x, d.y, d.z, d.w};
@@ -204,8 +215,14 @@ k_wgrad(const float * __restrict__ A, const float * __restrict__ dY, float * __r
 #pragma unroll
 				for (int i = 0; i < 4; ++i) acc[i][j] = fmaf(xs[i], ds[j], acc[i][j]);
 			}
+		};
+		if (rb + 16 <= r1) {
+#pragma unroll
+			for (uint32_t r = 0; r < 16; ++r) row(r);
+		} else {
+			for (uint32_t r = 0; r < r1 - rb; ++r) row(r);
 		}
-		__syncthreads();
+		if (rb + 16 < r1) __syncthreads();
 	}
 #pragma unroll
 	for (int j = 0; j < 4; ++j) {
