@@ -422,7 +422,7 @@ int tm_ring_lookup_counts(tm_ring * ring, uint32_t * counts, uint32_t n_parts);
  * writes their key bitmap rows to device memory (dev_rows: nq x
  * ceil(K/32) words), on `stream` (a hipStream_t; NULL: the default stream),
  * and returns when they are written.  It allocates nothing: its working
- * buffers live in a fixed static device array of 2.9 MiB per GPU,
+ * buffers live in a fixed static device array of 2.8 MiB per GPU,
  * which bounds nq by TM_STATIC_MAX_QUERIES and the FIB's partitions by
  * TM_STATIC_MAX_PARTS (larger sizes: TM_ERR_INVALID).  Calls on one GPU share
  * that array: calls that overlap on one GPU (from several threads) race.

@@ -165,12 +165,11 @@ k_build_items(const uint32_t * __restrict__ pcount, const uint64_t * __restrict_
 	if (tid < NQUEUE) qnext[tid * QPAD] = carry * tid / NQUEUE;
 }
 
-// ------------------------------------------------------------- match
-
 // ------------------------------------------------------------- query-major match
 
-// Persistent schedule.  A work item is a group of NQ = 64*TILES consecutive
-// queries of the submission, owned by one workgroup for the whole match:
+// The vector kernel (k_match_q).  A work item is a group of NQ = 64*TILES
+// consecutive queries of the submission and a segment of the table's blocks,
+// taken by one workgroup:
 //
 //   for each partition p (schedule order):
 //     lookup, fused: qsel = queries of the group whose bits cover p's mask
@@ -182,10 +181,10 @@ k_build_items(const uint32_t * __restrict__ pcount, const uint64_t * __restrict_
 //       hits: OR the filters' dense key ids into the group's key bitmaps in
 //       LDS (KEYS_UNIQUE), or stage (query, slot) pairs per wave (HITS).
 //
-// Because a group's results never leave its workgroup until the end, the
-// bitmaps are written out once with plain stores: no global atomics on
-// results.  The reference instead merges partial results on the host under
-// a per-query mutex (back_end.cc:288-301, tagmatch_query.hh:80-93).
+// With one segment a group's bitmaps are written out once, with plain stores;
+// with several each is merged, with an atomic for words that gain bits.  The
+// reference instead merges partial results on the host under a per-query
+// mutex (back_end.cc:288-301, tagmatch_query.hh:80-93).
 
 struct mq_args {
 	dev_fib_view f;
@@ -1312,7 +1311,7 @@ int resolve_params(tm_ring * r) {
 						 "KEYS_UNIQUE and KEY_BITMAP support up to 65536 distinct keys (FIB has %u); use KEYS_ALL",
 						 r->fib->n_keys);
 	// default batch: the reference's 256 for the plain form (parameters.hh:22),
-	// 128-query tiles for the persistent kernel (measured best at 10M filters)
+	// 64 queries per work item of the vector kernel
 	uint32_t bs = c.batch_size ? c.batch_size : (c.schedule == TM_SCHED_PLAIN ? 256 : 64);
 	if (bs != 64 && bs != 128 && bs != 256)
 		return set_error(TM_ERR_INVALID, "batch_size must be 64, 128 or 256 (got %u)", bs);
@@ -2960,13 +2959,13 @@ int tm_match(tm_fib * fib, const uint32_t * words, uint32_t nq, const tm_match_c
 //
 // The persistent KEY_BITMAP step of a ring, for callers that cannot
 // allocate device memory: every buffer the step's kernels need beyond the
-// caller's queries and rows (lookup counts and their prefix sums, the work
-// queues, counters, full-key-set flags and the active-query list) is carved
-// out of `scratch`, a file-scope device array of fixed size.  Each GPU the
-// library runs on holds its own copy of it until the process ends.  Host
-// code must not use the array's name as a device address: its address on
-// each device comes from hipGetSymbolAddress, taken once per device on the
-// entry point's first call there.  Calls on one GPU share that GPU's array;
+// caller's queries and rows (lookup counts, the work queues, counters,
+// full-key-set flags, the list of queries left and their words, and the
+// workgroups' statistics) is carved out of `scratch`, a file-scope device
+// array of fixed size.  Each GPU the library runs on holds its own copy of it
+// until the process ends.  Host code must not use the array's name as a
+// device address: its address on each device comes from hipGetSymbolAddress,
+// taken once per device on the entry point's first call there.  Calls on one GPU share that GPU's array;
 // the call clears what must start at zero, and calls that overlap on one GPU
 // race (the call is synchronous, so calls from one thread never overlap).
 
@@ -2978,16 +2977,13 @@ constexpr size_t SC_P = (size_t)TM_STATIC_MAX_PARTS + 1;
 constexpr size_t SC_Q = (size_t)TM_STATIC_MAX_QUERIES;
 // byte offsets of the sub-arrays
 constexpr size_t SC_PCOUNT = 0;                                          // u32 [P + 1]
-constexpr size_t SC_PBASE = SC_PCOUNT + sc_round(SC_P * 4);             // u64 [P + 1]
-constexpr size_t SC_IPREFIX = SC_PBASE + sc_round(SC_P * 8);            // u64 [P + 1]
+constexpr size_t SC_IPREFIX = SC_PCOUNT + sc_round(SC_P * 4);           // u64 [P + 1]
 constexpr size_t SC_QBEG = SC_IPREFIX + sc_round(SC_P * 8);             // u64 [NQUEUE + 1]
 constexpr size_t SC_QNEXT = SC_QBEG + sc_round((NQUEUE + 1) * 8);       // u64 [NQUEUE * QPAD]
 constexpr size_t SC_CNT = SC_QNEXT + sc_round((size_t)NQUEUE * QPAD * 8);   // u64 [8]
 constexpr size_t SC_STAT = SC_CNT + sc_round(8 * 8);                    // u64 [8]
 constexpr size_t SC_NACT = SC_STAT + sc_round(8 * 8);                   // u32 [4]
-constexpr size_t SC_SCAN = SC_NACT + sc_round(4 * 4);                   // u64 [scan words of P]
-constexpr size_t SC_SCAN_WORDS = (SC_P + 255) / 256 + 2;                // >= scan_tmp_words(P)
-constexpr size_t SC_QFULL = SC_SCAN + sc_round(SC_SCAN_WORDS * 8);      // u32 [Q]
+constexpr size_t SC_QFULL = SC_NACT + sc_round(4 * 4);                  // u32 [Q]
 constexpr size_t SC_ACTIVE = SC_QFULL + sc_round(SC_Q * 4);             // u32 [Q]
 constexpr size_t SC_QACT = SC_ACTIVE + sc_round(SC_Q * 4);               // u32 [Q x 8]
 constexpr size_t SC_WGSTAT = SC_QACT + sc_round(SC_Q * 32);              // u64 [MX_MAX_GROUPS x 4]
@@ -3041,21 +3037,17 @@ int tm_match_rows_static(tm_fib * fib, const uint32_t * dev_queries, uint32_t nq
 	r.P = fib->n_parts;
 	r.kw = (fib->n_keys + 31) / 32;
 	TM_CHECK(resolve_params(&r));
-	if (scan_tmp_words(r.P) > SC_SCAN_WORDS)
-		return set_error(TM_ERR_STATE, "scan scratch too small");
 	r.no_weights = true;
 	r.s = static_cast<hipStream_t>(stream);
 	r.d_q = const_cast<uint32_t *>(dev_queries);
 	r.d_gbm = dev_rows;
 	r.d_pcount = reinterpret_cast<uint32_t *>(sc + SC_PCOUNT);
-	r.d_pbase = reinterpret_cast<uint64_t *>(sc + SC_PBASE);
 	r.d_iprefix = reinterpret_cast<uint64_t *>(sc + SC_IPREFIX);
 	r.d_qbeg = reinterpret_cast<uint64_t *>(sc + SC_QBEG);
 	r.d_qnext = reinterpret_cast<unsigned long long *>(sc + SC_QNEXT);
 	r.d_cnt = reinterpret_cast<unsigned long long *>(sc + SC_CNT);
 	r.d_stat = reinterpret_cast<uint64_t *>(sc + SC_STAT);
 	r.d_nact = reinterpret_cast<uint32_t *>(sc + SC_NACT);
-	r.d_scan = reinterpret_cast<uint64_t *>(sc + SC_SCAN);
 	r.d_qfull = reinterpret_cast<uint32_t *>(sc + SC_QFULL);
 	r.d_active = reinterpret_cast<uint32_t *>(sc + SC_ACTIVE);
 	r.d_qact = reinterpret_cast<uint32_t *>(sc + SC_QACT);
