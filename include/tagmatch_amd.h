@@ -231,7 +231,8 @@ typedef struct tm_match_config {
 	uint32_t chunk_blocks;   /* PLAIN: least blocks per segment of a unit
 	                            (0 = 64); PERSISTENT: blocks per segment of
 	                            the table (0 = automatic, by the step's
-	                            size)                                        */
+	                            size), fewer where the matrix kernel would
+	                            have no item for each workgroup              */
 	uint32_t waves_per_group;/* waves per workgroup (4, 8 or 16); 0 = by
 	                            step size for PERSISTENT (16 up to 16 query
 	                            tiles, 8 up to 256, else 4; 8 in the matrix
