@@ -2066,8 +2066,20 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 	// 16384 keys 2092, 1091 (8788), 4096 keys 795, 934 (1411).
 	const int mode = !keys ? MX_COUNT : r->kw == 0 || (r->kw > 8 * MX_LDS_KW && f->ovf_valid <= 1) ? MX_KEYS : MX_KEYS_LDS;
 	mx_args a = matrix_args(r, mode);
-	const uint32_t nqg = mx_super_of(mode, r->kw);
+	// few items of 64 blocks: fewer queries per item, then 32 blocks (HITS,
+	// 1000 queries on 157 blocks: 429 us with 1536 queries per item, 99 so,
+	// 298 with the vector kernel; KEYS_ALL, 16 blocks: 334, 111, 146)
+	uint32_t nqg = mx_super_of(mode, r->kw);
 	const uint64_t resident = a.resident;
+	auto few = [&]() {
+		uint64_t n_items = 0;
+		for (uint32_t i = 0; i < n && n_items < resident; ++i)
+			n_items += (uint64_t)((r->u_off[i + 1] - r->u_off[i] + nqg - 1) / nqg) *
+					   ((f->h_part_info[(size_t)r->u_part[i] * 8 + 7] + 63) / 64);
+		return n_items < resident;
+	};
+	while (nqg > 64 && few()) nqg = (nqg / 2 + 63) & ~63u;
+	const uint32_t least_seg = few() ? 32 : 64;
 	uint64_t work = 0;   // tile x blocks
 	for (uint32_t i = 0; i < n; ++i) {
 		const uint32_t p = r->u_part[i], qn = r->u_off[i + 1] - r->u_off[i];
@@ -2077,7 +2089,7 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 	// uneven otherwise (541k queries on 10M filters, 2000 blocks an item: 3.30
 	// ms, 384: 3.07, 128: 3.39)
 	uint32_t seg = r->cfg.chunk_blocks ? r->cfg.chunk_blocks
-									   : (uint32_t)std::min<uint64_t>(384, std::max<uint64_t>(64, (work + 4 * resident - 1) / (4 * resident)));
+									   : (uint32_t)std::min<uint64_t>(384, std::max<uint64_t>(least_seg, (work + 4 * resident - 1) / (4 * resident)));
 	// list modes count by segment and query: at most as many segments as
 	// HCNT_MAX counts allow (or items of MX_MAX_SEG blocks)
 	const uint64_t most = keys ? 0xFFFFFFFFu : std::max<uint64_t>(1, HCNT_MAX / std::max<uint32_t>(nq, 1));
@@ -2112,6 +2124,7 @@ int enqueue_units(tm_ring * r, uint32_t nq) {
 	a.units = r->d_xunits;
 	a.uprefix = r->d_xprefix;
 	a.n_units = n;
+	a.unit_sq = nqg;
 	const uint32_t grid = (uint32_t)std::min<uint64_t>(resident, std::max<uint64_t>(items, 1));
 	if (!keys) {
 		TM_CHECK(grow_captured(r, &r->d_hcnt, r->hcnt_cap, (uint64_t)max_nseg * nq));

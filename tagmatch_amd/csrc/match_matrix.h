@@ -116,6 +116,7 @@ struct mx_args {
 	                                       // block, end block
 	const uint32_t * __restrict__ uprefix; // n_units + 1: first work item of each unit
 	uint32_t n_units;
+	uint32_t unit_sq;                      // queries of a unit's items, at most mx_super_of()
 	unsigned long long * qnext;            // MX_QUEUES cursors, MX_QPAD apart, zero at the start
 	uint32_t * gbm;                        // key rows
 	const uint32_t * __restrict__ qfull;   // flags of rows that hold every key (NULL: none known)

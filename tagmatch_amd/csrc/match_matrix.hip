@@ -78,7 +78,6 @@ k_match_x(mx_args a) {
 	const uint32_t epoch = a.step_vals ? sld1(a.step_vals) : a.epoch;
 	const uint32_t ovf_n = a.step_vals ? sld1(a.step_vals + 1) : a.f.ovf_n;
 	const mx_shape sh = mx_shape_of(MODE, kw, nq_all, a.nblk, a.resident, a.seg_fixed, a.seg_min);
-	const uint32_t usq = mx_super_of(MODE, kw);   // queries of a unit's items
 	const uint32_t items = a.units ? sld1(a.uprefix + a.n_units) : sh.nsuper * sh.nseg;
 	if (blockIdx.x == 0 && tid == 0) *a.n_items = items;
 	const bool queued = items > gridDim.x;
@@ -121,8 +120,8 @@ k_match_x(mx_args a) {
 			const uint32_t local = item - sld1(a.uprefix + lo);
 			seg = local / u0.w;
 			const uint32_t sup = local - seg * u0.w;
-			q0 = u0.y + sup * usq;
-			nqs = min(usq, u0.y + u0.z - q0);
+			q0 = u0.y + sup * a.unit_sq;
+			nqs = min(a.unit_sq, u0.y + u0.z - q0);
 			b0 = u1.z + seg * 32;
 			apart = u1.x * 32;
 			b_end = u1.w;

@@ -150,7 +150,7 @@ def test_units_cut_into_whole_tiles(gpu, table):
         ring = tm.Ring(fib, 100, mode=tm.MODE_KEYS_UNIQUE, chunk_blocks=seg)
         ring.submit_units(q, part, off)
         st = ring.wait()
-        tiles = 1 + 5 + 6          # of 1, 140 and 172 blocks
+        tiles = 1 + 2 * 5 + 6      # of 1, 140 and 172 blocks, for 3, 70 (64 and 6) and 27 queries
         print(f"segment {seg}: {st.n_items} items", flush=True)
         assert st.n_items <= tiles, seg
         check(ring, unit_lists(tab, q, part, off, 0), f"segment {seg}")
@@ -227,3 +227,21 @@ def test_groups_per_cu_holds(gpu):
         assert np.array_equal(ordered(*res[0]), ordered(*res[-1]))
     print(f"items {items}", flush=True)
     assert items[0] == items[1] and items[2] < 0.7 * items[1]
+
+
+ALL_MODES = LISTS + [(tm.MODE_KEYS_UNIQUE, 0)]
+
+
+@pytest.mark.parametrize("mode,om", ALL_MODES)
+def test_units_of_few_blocks_are_spread(gpu, table, mode, om):
+    """1000 queries on one small partition: more than a few items."""
+    tab, fib = table
+    q = queries(1063, 9)
+    for part, n in ((0, 1000), (1, 1063), (0, 65), (0, 64)):
+        ring = tm.Ring(fib, n, mode=mode)
+        p, off = np.array([part], np.uint32), np.array([0, n], np.uint32)
+        ring.submit_units(q[:n], p, off)
+        st = ring.wait()
+        print(f"mode {mode} partition {part}: {n} queries, {st.n_items} items", flush=True)
+        check(ring, unit_lists(tab, q[:n], p, off, om), f"mode {mode} partition {part} queries {n}")
+        assert st.n_items >= n // 64
