@@ -245,3 +245,19 @@ def test_units_of_few_blocks_are_spread(gpu, table, mode, om):
         print(f"mode {mode} partition {part}: {n} queries, {st.n_items} items", flush=True)
         check(ring, unit_lists(tab, q[:n], p, off, om), f"mode {mode} partition {part} queries {n}")
         assert st.n_items >= n // 64
+
+
+@pytest.mark.parametrize("mode,om", ALL_MODES)
+def test_steps_on_few_blocks_are_spread(gpu, mode, om):
+    """1000 queries on a table of 1000 filters: more than a few items."""
+    g = tm.Generator(seed=0xB0F)
+    tab = tm.canonicalize(*g.filters(1000))
+    fib, _ = tm.fib_from_runs(*tab, np.array([0, len(tab[0])], np.uint32))   # 15 blocks
+    for n in (1000, 1025, 65, 64, 3):
+        q = queries(n, 31)
+        ring = tm.Ring(fib, n, mode=mode, full_exit=2)
+        ring.submit(q)
+        st = ring.wait()
+        print(f"mode {mode}: {n} queries, {st.n_items} items", flush=True)
+        check(ring, orc.match(*tab, q, mode=om), f"mode {mode} queries {n}")
+        assert st.n_items >= n // 64
