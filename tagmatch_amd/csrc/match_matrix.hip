@@ -77,7 +77,8 @@ k_match_x(mx_args a) {
 	const uint32_t nq_all = a.nq_dev ? sld1(a.nq_dev) : a.nq;
 	const uint32_t epoch = a.step_vals ? sld1(a.step_vals) : a.epoch;
 	const uint32_t ovf_n = a.step_vals ? sld1(a.step_vals + 1) : a.f.ovf_n;
-	const mx_shape sh = mx_shape_of(MODE, kw, nq_all, a.nblk, a.resident, a.seg_fixed, a.seg_min);
+	mx_shape sh = {0, 0, 0, 0};
+	if (!a.units) sh = mx_shape_of(MODE, kw, nq_all, a.nblk, a.resident, a.seg_fixed, a.seg_min);
 	const uint32_t items = a.units ? sld1(a.uprefix + a.n_units) : sh.nsuper * sh.nseg;
 	if (blockIdx.x == 0 && tid == 0) *a.n_items = items;
 	const bool queued = items > gridDim.x;
