@@ -795,9 +795,9 @@ def main():
     log(f"first step (with H2D and capacity growth): {time.time() - t:.2f}s, overflow={st.overflow}")
     tuned = None
     if args.autotune and sched == tm.SCHED_PERSISTENT and not args.tile:
-        # the autotuner (tm_ring_autotune) picks the tile size, waves per
-        # workgroup, segment size and graph replay on this workload, before
-        # the timed steps
+        # the autotuner (tm_ring_autotune) picks the segment size and graph
+        # replay on this workload, before the timed steps (tile size and waves
+        # per workgroup change steps of the vector kernel only)
         cands = [dict(batch_size=b, waves_per_group=w, chunk_blocks=c, use_graph=int(g or args.graph))
                  for b, w, c, g in AUTOTUNE_CANDIDATES]
         best, times = ring.autotune(nq, cands, reps=1)
@@ -1052,7 +1052,8 @@ def main():
         "host_expand": host_expand,
         "parity_checked": parity,
         "matches_per_s": no_exit["matches_per_s"],
-        "matches_note": "every (query, filter) match enumerated, in a step without the full-key-set exit",
+        "matches_note": "every (query, filter) match tested and counted, in a step without the full-key-set exit; "
+                        "the keys of a match are read unless the rich-filter pass has completed its query's row",
         "keys_per_s": st["n_results"] / (ms_per_step / 1e3),
         "hits_per_query": n_hits / nq,
         "no_full_exit": no_exit,

@@ -248,7 +248,10 @@ typedef struct tm_match_config {
 	uint32_t full_exit;      /* PERSISTENT KEYS_UNIQUE: stop testing a query
 	                            once its key set holds every key of the
 	                            table (results unchanged); 0 = default (on),
-	                            1 = on, 2 = off                              */
+	                            1 = on, 2 = off: every match is tested and
+	                            counted, and its keys are read unless the
+	                            rich-filter pass has completed its query's
+	                            row                                          */
 	uint32_t compact_tiles;  /* accepted and ignored: every KEYS_UNIQUE /
 	                            KEY_BITMAP step with a rich-filter pass
 	                            matches only the queries that pass leaves

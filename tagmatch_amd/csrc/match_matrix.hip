@@ -42,11 +42,14 @@ __device__ inline uint32_t inline_keys(uint64_t kv) {
 //
 // Bound by the vector unit, which spreads the operands, turns accumulators
 // into masks and logs hits: where every match is enumerated (1M queries, 10M
-// filters, 139 ms, 50 G matches/s) it is busy 79 % of the time and the matrix
+// filters, 140 ms, 50 G matches/s) it is busy 79 % of the time and the matrix
 // unit 40 %; with the full-row exit (0.95 ms) it is busy 57 %, and the waves
 // wait for blocks and keys 55 % of theirs.  One query at a time against 64
 // filters on the vector unit took 556 and 1.98 ms: each test read 24 bytes
-// of local memory per lane, 12 of its cycles, and 7 instructions.
+// of local memory per lane, 12 of its cycles, and 7 instructions.  Of the 556
+// ms' gain a part is key work left out: matches of rows that are complete
+// before the match (97 % of them there) are counted and their keys not read;
+// with them read the 140 ms are 335 (65k queries: 9.2 and 21.8).
 //
 // Two workgroups of eight waves per CU: 128 registers; with 96 (five waves a
 // SIMD) the operands spill (a third slower).  A block's words are loaded

@@ -170,7 +170,8 @@ struct nz_seg {
 // lie last split first), rounds the splits.  Bound by one CU's latency (a
 // gather and a barrier per 4096 filters, three barriers per split): 1.5 ms for
 // the 1M-filter table's segment of about 64k filters and 75 splits (2.6 ms
-// with 1024 filters at a time); split level by level over all the records,
+// with 1024 filters at a time), 1.08 for what is left of it after the five that
+// the levels make down to NZ_BITS; split level by level over all the records,
 // each with its round trips to the host, they took 17 ms.
 __global__ void __launch_bounds__(1024)
 k_nonzero(const uint32_t * __restrict__ rec, const nz_seg * __restrict__ segs, const uint32_t * __restrict__ freq,
