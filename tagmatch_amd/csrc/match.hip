@@ -1156,6 +1156,7 @@ struct tm_ring {
 	uint64_t * h_stat = nullptr;
 	uint64_t * h_off = nullptr;
 	uint32_t * h_vals = nullptr;
+	uint32_t host_nq = 0;          // queries whose offsets the last collected step left there
 	uint32_t copy_nq = 0;          // queries the next step takes from h_q
 	uint32_t * d_hcnt = nullptr;   // hit-list steps: values per segment and query
 	uint64_t hcnt_cap = 0;
@@ -2694,6 +2695,7 @@ int tm_wait(tm_ring * r, tm_status * st) {
 			r->pack_guess = n + n / 8 + 64;
 		}
 		end_pending(r);
+		r->host_nq = r->run_nq <= OFF_MAX ? r->run_nq : 0;
 		float dms = 0.f, mms = 0.f;
 		(void)hipEventElapsedTime(&dms, r->e0, r->e1);
 		if (r->match_events) (void)hipEventElapsedTime(&mms, r->em0, r->em1);
@@ -2727,7 +2729,7 @@ int tm_read_results(tm_ring * r, uint64_t * offsets, uint32_t * values, uint64_t
 		offsets[0] = 0;
 		return TM_OK;
 	}
-	const bool here = r->run_nq <= OFF_MAX;   // the step left them in host memory
+	const bool here = nq <= r->host_nq;   // the step left them in host memory
 	if (here)
 		std::memcpy(offsets, r->h_off, ((size_t)nq + 1) * sizeof(uint64_t));
 	else

@@ -261,3 +261,27 @@ def test_steps_on_few_blocks_are_spread(gpu, mode, om):
         print(f"mode {mode}: {n} queries, {st.n_items} items", flush=True)
         check(ring, orc.match(*tab, q, mode=om), f"mode {mode} queries {n}")
         assert st.n_items >= n // 64
+
+
+def test_results_after_a_refused_submission(gpu):
+    """A submission that the table's growth makes impossible (more keys than
+    rows can hold) leaves the last one's lists: those of its first queries."""
+    w, _, _ = tm.Generator(seed=0xB0F).filters(48000)
+    w = np.unique(w, axis=0)[:35100]
+    small = tm.canonicalize(w, np.arange(len(w) + 1, dtype=np.uint64), (np.arange(len(w)) % 3000).astype(np.uint32))
+    large = tm.canonicalize(w, np.arange(0, 2 * len(w) + 1, 2, dtype=np.uint64), np.arange(2 * len(w), dtype=np.uint32))
+    off, mask = np.array([0, len(w)], np.uint32), np.zeros((1, 6), np.uint32)
+    fib = tm.Fib(small[0], off, mask, small[1], small[2])
+    q = queries(5000, 77)
+    exp = orc.match(*small, q, mode=0)
+    ring = tm.Ring(fib, 5000, mode=tm.MODE_KEYS_UNIQUE)
+    ring.submit(q[-5:])      # lists in host memory, then more than it takes
+    ring.wait()
+    ring.submit(q)
+    ring.wait()
+    check(ring, exp, "before the upload")
+    fib.upload(large[0], off, mask, large[1], large[2])
+    with pytest.raises(tm.TagMatchError):
+        ring.submit(q[:20])
+    o, v = ring.results()
+    assert np.array_equal(o, exp[0][:21]) and np.array_equal(v, exp[1][:int(exp[0][20])])
